@@ -13,7 +13,7 @@ enum EpiMode : int {
   EPI_RESID = 2,      // resid += C + bias + ple_scale * ple[m, ple_off + n % ple_dim]
   EPI_QKV = 3,        // q | k | v split; k, v (+ value embedding) appended to the KV pool
   EPI_SCALE_ADD = 4,  // out = (C + addend) * scale                      (out_dtype)
-  EPI_RESID_LN = 5,   // EPI_RESID, then out = LayerNorm(resid row)      (out_dtype); N <= 256
+  EPI_RESID_LN = 5,   // EPI_RESID, then out = LayerNorm(resid row)      (out_dtype); N <= 256, bf16
 };
 
 struct GemmArgs {
@@ -41,6 +41,10 @@ struct GemmArgs {
   float scale;
   const float *ln_w, *ln_b;  // EPI_RESID_LN
   float eps;
+  // LayerNorm of A's rows as they are read (fp32, where split_gemm_norms says so): A holds the fp32
+  // residual stream, the product takes LayerNorm(A) with these parameters.
+  const float *a_ln_w, *a_ln_b;
+  float a_eps;
   // EPI_QKV: columns [0, q_cols) -> q (fp32, ld ldo); then kv_heads * head_dim columns of
   // K and as many of V, appended at (tok_row[m], head, tok_pos[m]).
   int32_t q_cols;
@@ -53,6 +57,10 @@ struct GemmArgs {
 };
 
 void launch_gemm(const GemmArgs &g, hipStream_t stream);
+
+// Whether an fp32 m x n product over k takes LayerNorm(A; w, b) of the rows it reads by itself
+// (GemmArgs::a_ln_w).
+bool split_gemm_norms(int32_t m, int32_t n, int32_t k, const float *w, const float *b);
 
 // y[i] = LayerNorm(x[index ? index[i] : i]) (fp32 statistics), stored as y_dtype.
 void launch_layernorm_rows(const float *x, const int32_t *index, const float *w, const float *b,

@@ -650,10 +650,22 @@ void trunk_forward(const cg_trunk *trunk, const cg_kv_layer *cache, const float 
   }
 
   if (x != w.x) CG_HIP(hipMemcpyAsync(w.x, x, size_t(N) * d * 4, hipMemcpyDeviceToDevice, s));
-  launch_layernorm_rows(w.x, nullptr, t.layers[0].ln_attn_w, t.layers[0].ln_attn_b, c.eps, w.xn,
-                        act_dtype, N, d, s);
-  // Whole-row residual tiles fuse the next LayerNorm into the residual epilogue.
-  const bool fused_ln = d <= 256;
+  // Whole-row bf16 residual tiles fuse the next LayerNorm into the residual epilogue; small fp32
+  // products take the LayerNorm of the rows they read (split_gemm_norms), so that neither their
+  // producer's tiles have to be whole rows nor the normalised rows travel.
+  const bool f32 = t.compute == CG_F32, fused_ln = !f32 && d <= 256;
+  auto normed = [&](GemmArgs &g, const float *ln_w, const float *ln_b, bool ready) {
+    if (f32 && split_gemm_norms(g.M, g.N, g.K, ln_w, ln_b)) {
+      g.A = w.x;
+      g.a_ln_w = ln_w;
+      g.a_ln_b = ln_b;
+      g.a_eps = c.eps;
+    } else {
+      if (!ready) launch_layernorm_rows(w.x, nullptr, ln_w, ln_b, c.eps, w.xn, act_dtype, N, d, s);
+      g.A = w.xn;
+    }
+    g.lda = d;
+  };
 
   auto residual = [&](const void *A, int K, const void *W, const float *bias, const float *ln_w,
                       const float *ln_b, const float *ple_rows, int layer) {
@@ -688,7 +700,6 @@ void trunk_forward(const cg_trunk *trunk, const cg_kv_layer *cache, const float 
     }
     g.epi = EPI_RESID;
     launch_gemm(g, s);
-    if (ln_w) launch_layernorm_rows(w.x, nullptr, ln_w, ln_b, c.eps, w.xn, act_dtype, N, d, s);
   };
 
   for (int l = 0; l < c.n_layers; ++l) {
@@ -700,8 +711,7 @@ void trunk_forward(const cg_trunk *trunk, const cg_kv_layer *cache, const float 
       g.N = (H + 2 * KVH) * D;
       g.K = d;
       g.compute = t.compute;
-      g.A = w.xn;
-      g.lda = d;
+      normed(g, P.ln_attn_w, P.ln_attn_b, fused_ln && l > 0);
       g.W = t.qkv_w[l];
       g.epi = EPI_QKV;
       g.out = w.q;
@@ -729,8 +739,7 @@ void trunk_forward(const cg_trunk *trunk, const cg_kv_layer *cache, const float 
       g.N = c.d_ff;
       g.K = d;
       g.compute = t.compute;
-      g.A = w.xn;
-      g.lda = d;
+      normed(g, P.ln_mlp_w, P.ln_mlp_b, fused_ln);
       g.W = t.up_w[l];
       g.bias = P.mlp_up_b;
       g.epi = EPI_GELU;
