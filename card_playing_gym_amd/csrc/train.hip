@@ -20,6 +20,7 @@
 #include <string>
 
 #include "common.h"
+#include "split_tile.h"
 
 namespace cg {
 namespace {
@@ -103,137 +104,23 @@ __device__ __forceinline__ void epilogue(const Epi &e, float v, float beta, floa
 }
 
 // ---- strided GEMM ---------------------------------------------------------------------
-// Tile 128 x 128, four waves (2 x 2, each 64 x 64 = 4 x 4 MFMA tiles), 16 k per LDS stage,
-// double-buffered.  A(m, k) = A[m * sam + k * sak], B(k, n) = B[k * sbk + n * sbn]; tiles are
-// staged through LDS with 16-byte loads along whichever index has stride 1, and sit there as
-// [row][16 k] (row pitch GT_LDK).  MFMA 16x16x4 f32: lane (li, lg) gives A(row li, k) and
-// B(k, col li) for the instruction's k index lg; the result sits in lane (li, lg) as rows
-// 4 lg + r, column li.  The four MFMAs s = 0..3 of a stage give lane group lg the stage's k
-// = 4 lg + s (the sum over k does not depend on which instruction adds which term), so a
-// lane's fragments for a whole stage are one 16-byte LDS read per 16-row block.  Split K
-// (grid.z > 1): slice z covers k in [z kc, (z + 1) kc) and writes its partial product to
-// part[z] ([m, n]); a second pass sums them.
-constexpr int GT_M = 128, GT_N = 128, GT_K = 16;
-constexpr int GT_LDK = GT_K + 4;  // LDS row pitch, floats: 16-lane groups of 16-byte reads hit 64 banks once
-
-// A ROWS x 16 (rows x k) operand tile (ROWS 64 or 128) with element (r, k) at p[r * sr + k *
-// sk], ROWS / 64 float4 per thread.  MODE 1: k contiguous (float4 = 4 k of a row; k extent a multiple of 4); MODE 2:
-// rows contiguous (float4 = 4 rows at one k; row extent a multiple of 4); MODE 0: any strides.
-// Loads go to clamped, always valid addresses with no branches (so the next stage's loads all
-// fly at once during this stage's MFMAs); rows >= rows_left or k >= k_left are zeroed when the
-// tile is written to LDS, after the MFMAs.
-template <int ROWS>
-struct TileRegs {
-  float4 v[ROWS / 64];
-};
-
-// Row of float4 slot idx in the k-contiguous layouts (MODE 1 and 0): four 4-k blocks of 16 rows
-// per 64 slots, the four rows of each 16-slot group 4 apart, so that their LDS rows (pitch 20
-// floats) start 0, 16, 32, 48 banks apart and a 16-lane write covers the 64 banks once.
-__device__ __forceinline__ int slot_row(int idx) { return (idx >> 6) * 16 + ((idx >> 2) & 3) * 4 + ((idx >> 4) & 3); }
-
-template <int MODE, int ROWS>
-__device__ __forceinline__ TileRegs<ROWS> load_tile(const float *__restrict__ p, int64_t sr, int64_t sk, int rows_left,
-                                                    int k_left, int tid) {
-  TileRegs<ROWS> t;
-#pragma unroll
-  for (int e = 0; e < ROWS / 64; ++e) {
-    const int idx = tid + e * 256;  // ROWS x 16 floats = ROWS * 4 float4
-    if constexpr (MODE == 2) {      // 32 groups of 4 rows x 16 k (k fastest across lanes)
-      const int k = idx & 15, r = (idx >> 4) * 4;
-      const int rc = max(0, min(r, rows_left - 4)), kc = min(k, k_left - 1);
-      t.v[e] = *reinterpret_cast<const float4 *>(p + int64_t(kc) * sk + rc);
-    } else if constexpr (MODE == 1) {  // 128 rows x 4 groups of 4 k
-      const int r = slot_row(idx), k = (idx & 3) * 4;
-      const int rc = min(r, rows_left - 1), kc = max(0, min(k, k_left - 4));
-      t.v[e] = *reinterpret_cast<const float4 *>(p + int64_t(rc) * sr + kc);
-    } else {  // same slots as MODE 1, element by element
-      const int r = slot_row(idx), k = (idx & 3) * 4;
-      const int64_t base = int64_t(min(r, rows_left - 1)) * sr;
-      t.v[e] = float4{p[base + int64_t(min(k, k_left - 1)) * sk], p[base + int64_t(min(k + 1, k_left - 1)) * sk],
-                      p[base + int64_t(min(k + 2, k_left - 1)) * sk], p[base + int64_t(min(k + 3, k_left - 1)) * sk]};
-    }
-  }
-  return t;
-}
-
-template <int MODE, int ROWS>
-__device__ __forceinline__ void store_tile(float *lds, const TileRegs<ROWS> &t, int tid, int rows_left, int k_left) {
-#pragma unroll
-  for (int e = 0; e < ROWS / 64; ++e) {
-    const int idx = tid + e * 256;
-    const float4 v = t.v[e];
-    if constexpr (MODE == 2) {
-      const int k = idx & 15, r = (idx >> 4) * 4;
-      const bool ok = k < k_left && r < rows_left;  // row extent a multiple of 4: all four rows or none
-      lds[(r + 0) * GT_LDK + k] = ok ? v.x : 0.f;
-      lds[(r + 1) * GT_LDK + k] = ok ? v.y : 0.f;
-      lds[(r + 2) * GT_LDK + k] = ok ? v.z : 0.f;
-      lds[(r + 3) * GT_LDK + k] = ok ? v.w : 0.f;
-    } else {
-      const int r = slot_row(idx), k = (idx & 3) * 4;
-      const bool row = r < rows_left;
-      float4 o;
-      if constexpr (MODE == 1) {
-        const bool ok = row && k < k_left;  // k extent a multiple of 4
-        o = ok ? v : float4{0.f, 0.f, 0.f, 0.f};
-      } else {
-        o = float4{row && k < k_left ? v.x : 0.f, row && k + 1 < k_left ? v.y : 0.f, row && k + 2 < k_left ? v.z : 0.f,
-                   row && k + 3 < k_left ? v.w : 0.f};
-      }
-      *reinterpret_cast<float4 *>(lds + r * GT_LDK + k) = o;
-    }
-  }
-}
-
-// bf16 operands: the same tile converted once as it is written to LDS, [row][16 k] bf16 at a
-// 40-byte row pitch (16-lane groups of 8-byte fragment reads hit distinct banks).
-constexpr int GT_LDKB = GT_K + 4;  // row pitch in bf16 elements
-
-template <int MODE, int ROWS>
-__device__ __forceinline__ void store_tile_bf16(unsigned short *lds, const TileRegs<ROWS> &t, int tid, int rows_left,
-                                                int k_left) {
-#pragma unroll
-  for (int e = 0; e < ROWS / 64; ++e) {
-    const int idx = tid + e * 256;
-    const float4 v = t.v[e];
-    if constexpr (MODE == 2) {
-      const int k = idx & 15, r = (idx >> 4) * 4;
-      const bool ok = k < k_left && r < rows_left;
-      const unsigned lo = pack_bf16(ok ? v.x : 0.f, ok ? v.y : 0.f), hi = pack_bf16(ok ? v.z : 0.f, ok ? v.w : 0.f);
-      lds[(r + 0) * GT_LDKB + k] = static_cast<unsigned short>(lo);
-      lds[(r + 1) * GT_LDKB + k] = static_cast<unsigned short>(lo >> 16);
-      lds[(r + 2) * GT_LDKB + k] = static_cast<unsigned short>(hi);
-      lds[(r + 3) * GT_LDKB + k] = static_cast<unsigned short>(hi >> 16);
-    } else {
-      const int r = slot_row(idx), k = (idx & 3) * 4;
-      const bool row = r < rows_left;
-      float4 o;
-      if constexpr (MODE == 1) {
-        o = (row && k < k_left) ? v : float4{0.f, 0.f, 0.f, 0.f};
-      } else {
-        o = float4{row && k < k_left ? v.x : 0.f, row && k + 1 < k_left ? v.y : 0.f, row && k + 2 < k_left ? v.z : 0.f,
-                   row && k + 3 < k_left ? v.w : 0.f};
-      }
-      *reinterpret_cast<u32x2 *>(lds + r * GT_LDKB + k) = u32x2{pack_bf16(o.x, o.y), pack_bf16(o.z, o.w)};
-    }
-  }
-}
+// A(m, k) = A[m * sam + k * sak], B(k, n) = B[k * sbk + n * sbn]; TM x 128 tiles through
+// tile_product (split_tile.h): fp32 products in three bf16 parts, bf16 (autocast) ones with
+// operands rounded as they are staged.  Split K (grid.z > 1): slice z covers k in
+// [z kc, (z + 1) kc) and writes its partial product to part[z] ([m, n]); a second pass sums
+// them.
+constexpr int GT_M = 128, GT_N = ST_N, GT_K = 32;
 
 template <int AM, int BM, int TM, bool BF>
-__global__ __launch_bounds__(256, 3) void gemm_strided_kernel(int32_t M, int32_t N, int32_t K, int32_t kc, float alpha,
+__global__ __launch_bounds__(256, 2) void gemm_strided_kernel(int32_t M, int32_t N, int32_t K, int32_t kc, float alpha,
                                                            const float *__restrict__ A, int64_t sam, int64_t sak,
                                                            const float *__restrict__ B, int64_t sbk, int64_t sbn,
                                                            float beta, float *__restrict__ C, int64_t ldc,
                                                            float *__restrict__ part, const Epi epi) {
   constexpr int FM = TM / 32;  // 16-row MFMA blocks per wave: a wave takes TM / 2 rows x 64 columns
-  // fp32 tiles [row][GT_LDK floats]; bf16 tiles [row][GT_LDKB halves] (half the storage)
-  constexpr int PITCH = BF ? GT_LDKB / 2 : GT_LDK;  // row pitch in 4-byte words
-  __shared__ __align__(16) float as[2][TM * PITCH];
-  __shared__ __align__(16) float bs[2][GT_N * PITCH];
-  auto as16 = [&](int b) { return reinterpret_cast<unsigned short *>(as[b]); };
-  auto bs16 = [&](int b) { return reinterpret_cast<unsigned short *>(bs[b]); };
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int PLANES = BF ? 1 : 3, NK = BF ? 2 : 1;
+  __shared__ __align__(16) char lds[tile_lds_bytes<TM, PLANES, NK>()];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int li = lane & 15, lg = lane >> 4;
   int mt = blockIdx.y, nt = blockIdx.x;
@@ -247,75 +134,12 @@ __global__ __launch_bounds__(256, 3) void gemm_strided_kernel(int32_t M, int32_t
   }
   const int m0 = mt * TM, n0 = nt * GT_N;
   const int kbeg = blockIdx.z * kc, kend = min(K, kbeg + kc);
-  const float *a0 = A + int64_t(m0) * sam, *b0 = B + int64_t(n0) * sbn;
   f32x4 acc[FM][4];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int buf = 0;
-  const int ma = M - m0, nb_ = N - n0;
-  if (kbeg < kend) {
-    const auto ta0 = load_tile<AM, TM>(a0 + int64_t(kbeg) * sak, sam, sak, ma, kend - kbeg, tid);
-    const auto tb0 = load_tile<BM, GT_N>(b0 + int64_t(kbeg) * sbk, sbn, sbk, nb_, kend - kbeg, tid);
-    if constexpr (BF) {
-      store_tile_bf16<AM, TM>(as16(0), ta0, tid, ma, kend - kbeg);
-      store_tile_bf16<BM, GT_N>(bs16(0), tb0, tid, nb_, kend - kbeg);
-    } else {
-      store_tile<AM, TM>(as[0], ta0, tid, ma, kend - kbeg);
-      store_tile<BM, GT_N>(bs[0], tb0, tid, nb_, kend - kbeg);
-    }
-  }
-  __syncthreads();
-  for (int k0 = kbeg; k0 < kend; k0 += GT_K) {
-    const bool more = k0 + GT_K < kend;
-    const int kl = kend - k0 - GT_K;  // k left after this stage
-    TileRegs<TM> na;
-    TileRegs<GT_N> nb;
-    if (more) {  // the next stage's loads fly during this stage's MFMAs
-      na = load_tile<AM, TM>(a0 + int64_t(k0 + GT_K) * sak, sam, sak, ma, kl, tid);
-      nb = load_tile<BM, GT_N>(b0 + int64_t(k0 + GT_K) * sbk, sbn, sbk, nb_, kl, tid);
-    }
-    const float *ta = as[buf], *tb = bs[buf];
-    if constexpr (BF) {  // bf16 operands: the stage's 16 k in one v_mfma_f32_16x16x16_bf16 per tile,
-                         // lane group lg holding k = 4 lg .. 4 lg + 3 as the fp32 path does
-      const unsigned short *ta16 = as16(buf), *tb16 = bs16(buf);
-      s16x4 bb[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        bb[j] = *reinterpret_cast<const s16x4 *>(tb16 + (wn * 64 + j * 16 + li) * GT_LDKB + 4 * lg);
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const s16x4 ab = *reinterpret_cast<const s16x4 *>(ta16 + (wm * (TM / 2) + i * 16 + li) * GT_LDKB + 4 * lg);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ab, bb[j], acc[i][j], 0, 0, 0);
-      }
-    } else {
-      f32x4 bf[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bf[j] = *reinterpret_cast<const f32x4 *>(tb + (wn * 64 + j * 16 + li) * GT_LDK + 4 * lg);
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const f32x4 af = *reinterpret_cast<const f32x4 *>(ta + (wm * (TM / 2) + i * 16 + li) * GT_LDK + 4 * lg);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[s], bf[j][s], acc[i][j], 0, 0, 0);
-      }
-    }
-    if (more) {
-      if constexpr (BF) {
-        store_tile_bf16<AM, TM>(as16(buf ^ 1), na, tid, ma, kl);
-        store_tile_bf16<BM, GT_N>(bs16(buf ^ 1), nb, tid, nb_, kl);
-      } else {
-        store_tile<AM, TM>(as[buf ^ 1], na, tid, ma, kl);
-        store_tile<BM, GT_N>(bs[buf ^ 1], nb, tid, nb_, kl);
-      }
-    }
-    __syncthreads();
-    buf ^= 1;
-  }
+  tile_product<AM, BM, TM, PLANES, NK>(A + int64_t(m0) * sam, sam, sak, M - m0, B + int64_t(n0) * sbn, sbk, sbn, N - n0,
+                                       kbeg, kend, lds, acc);
+  if constexpr (!BF)
+    tile_repair<FM>(acc, A + int64_t(kbeg) * sak, sam, sak, B + int64_t(kbeg) * sbk, sbk, sbn, m0 + wm * (TM / 2),
+                    n0 + wn * 64, M, N, kend - kbeg);
   if (part) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
