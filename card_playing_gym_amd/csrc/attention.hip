@@ -68,6 +68,33 @@ __device__ __forceinline__ void load_widen(const T *__restrict__ p, float (&out)
 constexpr int KEYS_PER_BLOCK = 64;
 constexpr int QB = 4;  // queries per pass over the keys
 
+// Sums N values over the lanes that differ in bits 2..5 (the 16 slots of a wave): while their
+// number is even a round halves them, each lane keeping (and returning the index of) its half;
+// an odd number is added by a plain exchange.  Rounds: lane xor 32, 16, 8, 4.
+constexpr int slots_left(int n) {
+  for (int r = 0; r < 4 && n % 2 == 0; ++r) n /= 2;
+  return n;
+}
+template <int N, int OFF, int CAP>
+__device__ __forceinline__ int slots_reduce(float (&v)[CAP], int lane) {
+  if constexpr (OFF < 4) {
+    return 0;
+  } else if constexpr (N % 2 == 0) {
+    constexpr int H = N / 2;
+    const bool up = (lane & OFF) != 0;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const float keep = up ? v[H + i] : v[i], send = up ? v[i] : v[H + i];
+      v[i] = keep + __shfl_xor(send, OFF, 64);
+    }
+    return (up ? H : 0) + slots_reduce<H, OFF / 2>(v, lane);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += __shfl_xor(v[i], OFF, 64);
+    return slots_reduce<N, OFF / 2>(v, lane);
+  }
+}
+
 template <typename TKV, int D, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(AttnArgs a) {
   constexpr int DPL = D / 4;
@@ -106,25 +133,22 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(AttnArgs a
     float q[QB][DPL];
     int lim[QB];
     int maxlim = 0;
+    int64_t qo[QB];
 #pragma unroll
     for (int j = 0; j < QB; ++j) {
-      const int m = qb + j;
-      if (m < nq) {
-        const int t = m / G, g = m % G;
-        const int64_t qo = q_base + int64_t(h * G + g) * a.q_sh + int64_t(t) * a.q_st + e * DPL;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) q[j][i] = load_any(a.q, a.q_dtype, qo + i) * a.scale_log2;
-        int64_t l = kl + t;
-        if (l > a.span) l = a.span;
-        if (!row_ok || l < 0) l = 0;
-        lim[j] = int(l);
-      } else {
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) q[j][i] = 0.f;
-        lim[j] = 0;
-      }
+      const int m = min(qb + j, nq - 1), t = m / G, g = m % G;
+      qo[j] = q_base + int64_t(h * G + g) * a.q_sh + int64_t(t) * a.q_st + e * DPL;
+      int64_t l = kl + t;
+      if (l > a.span) l = a.span;
+      if (!row_ok || l < 0 || qb + j >= nq) l = 0;
+      lim[j] = int(l);
       maxlim = lim[j] > maxlim ? lim[j] : maxlim;
     }
+    load_runs(a.q, a.q_dtype, qo, q);
+#pragma unroll
+    for (int j = 0; j < QB; ++j)
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) q[j][i] *= a.scale_log2;
 
     float mx[QB], sum[QB], acc[QB][DPL];
 #pragma unroll
@@ -166,10 +190,10 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(AttnArgs a
       for (int j = 0; j < QB; ++j) {
         const float blk = fmaxf(fmaxf(s[0][j], s[1][j]), fmaxf(s[2][j], s[3][j]));
         const float mnew = fmaxf(mx[j], blk);
-        const float corr = exp2f(mx[j] - mnew);
+        const float corr = fast_exp2(mx[j] - mnew);
         float p[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p[r] = exp2f(s[r][j] - mnew);
+        for (int r = 0; r < 4; ++r) p[r] = fast_exp2(s[r][j] - mnew);
         sum[j] = sum[j] * corr + ((p[0] + p[1]) + (p[2] + p[3]));
 #pragma unroll
         for (int i = 0; i < DPL; ++i) {
@@ -184,75 +208,56 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(AttnArgs a
       }
     }
 
-    // Merge the 16 slots of the wave (lanes differing in bits 2..5).
+    // Merge the 16 slots of the wave (lanes differing in bits 2..5): a common maximum per
+    // query, then the sums halve over the lanes as they add (a lane keeps the half of the
+    // values that its bit names), 4 exchanges per query and dimension fewer than a full
+    // butterfly of every value.
+    float flat[QB * DPL];
 #pragma unroll
-    for (int off = 4; off < 64; off <<= 1) {
+    for (int j = 0; j < QB; ++j) {
+      float m = mx[j];
+#pragma unroll
+      for (int off = 4; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+      const float c = fast_exp2(mx[j] - m);
+      mx[j] = m;
+      sum[j] *= c;
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) flat[j * DPL + i] = acc[j][i] * c;
+#pragma unroll
+      for (int off = 4; off < 64; off <<= 1) sum[j] += __shfl_xor(sum[j], off, 64);
+    }
+    const int first = slots_reduce<QB * DPL, 32>(flat, lane);
+    if (lane == 0) {
 #pragma unroll
       for (int j = 0; j < QB; ++j) {
-        const float mo = __shfl_xor(mx[j], off, 64);
-        const float so = __shfl_xor(sum[j], off, 64);
-        const float mnew = fmaxf(mx[j], mo);
-        const float c1 = exp2f(mx[j] - mnew), c2 = exp2f(mo - mnew);
-        sum[j] = sum[j] * c1 + so * c2;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) {
-          const float ao = __shfl_xor(acc[j][i], off, 64);
-          acc[j][i] = acc[j][i] * c1 + ao * c2;
-        }
-        mx[j] = mnew;
+        merge_m[wave][j] = mx[j];
+        merge_l[wave][j] = sum[j];
       }
     }
-
-    if constexpr (WAVES > 1) {
-      if (slot == 0) {
 #pragma unroll
-        for (int j = 0; j < QB; ++j) {
-          if (e == 0) {
-            merge_m[wave][j] = mx[j];
-            merge_l[wave][j] = sum[j];
-          }
-#pragma unroll
-          for (int i = 0; i < DPL; ++i) merge_acc[wave][j][e * DPL + i] = acc[j][i];
-        }
-      }
-      __syncthreads();
-      if (wave == 0) {
-#pragma unroll
-        for (int j = 0; j < QB; ++j) {
-          float m = merge_m[0][j];
-#pragma unroll
-          for (int w = 1; w < WAVES; ++w) m = fmaxf(m, merge_m[w][j]);
-          float l = 0.f, o[DPL];
-#pragma unroll
-          for (int i = 0; i < DPL; ++i) o[i] = 0.f;
-#pragma unroll
-          for (int w = 0; w < WAVES; ++w) {
-            const float c = exp2f(merge_m[w][j] - m);
-            l += merge_l[w][j] * c;
-#pragma unroll
-            for (int i = 0; i < DPL; ++i) o[i] += merge_acc[w][j][e * DPL + i] * c;
-          }
-          sum[j] = l;
-#pragma unroll
-          for (int i = 0; i < DPL; ++i) acc[j][i] = o[i];
-        }
-      }
-      __syncthreads();
+    for (int i = 0; i < slots_left(QB * DPL); ++i) {
+      const int v = first + i;
+      merge_acc[wave][v / DPL][e * DPL + v % DPL] = flat[i];
     }
-
-    if (wave == 0 && slot == 0) {
+    __syncthreads();
+    for (int o = threadIdx.x; o < QB * D; o += 64 * WAVES) {
+      const int j = o / D, d = o % D, m = qb + j;
+      if (m >= nq) continue;
+      float top = merge_m[0][j];
 #pragma unroll
-      for (int j = 0; j < QB; ++j) {
-        const int m = qb + j;
-        if (m < nq) {
-          const int t = m / G, g = m % G;
-          const int64_t oo = o_base + int64_t(h * G + g) * a.o_sh + int64_t(t) * a.o_st + e * DPL;
-          const float inv = sum[j] > 0.f ? 1.0f / sum[j] : 0.f;
+      for (int w = 1; w < WAVES; ++w) top = fmaxf(top, merge_m[w][j]);
+      float l = 0.f, v = 0.f;
 #pragma unroll
-          for (int i = 0; i < DPL; ++i) store_any(a.out, a.out_dtype, oo + i, acc[j][i] * inv);
-        }
+      for (int w = 0; w < WAVES; ++w) {
+        const float c = fast_exp2(merge_m[w][j] - top);
+        l = fmaf(merge_l[w][j], c, l);
+        v = fmaf(merge_acc[w][j][d], c, v);
       }
+      const int t = m / G, g = m % G;
+      store_any(a.out, a.out_dtype, o_base + int64_t(h * G + g) * a.o_sh + int64_t(t) * a.o_st + d,
+                l > 0.f ? v / l : 0.f);
     }
+    __syncthreads();
   }
 }
 
@@ -310,7 +315,7 @@ __global__ __launch_bounds__(256) void decode_attention_mfma_kernel(AttnArgs a) 
   const TKV *__restrict__ vbase = static_cast<const TKV *>(a.v) + head_off;
 
   const int nq = int(count) * G;
-  for (int qg = 0; qg < nq; qg += NQT * 16) {
+  for (int qg = blockIdx.y * NQT * 16; qg < nq; qg += gridDim.y * NQT * 16) {
     // ---- queries of this group: column li of tile qt is query qg + 16 qt + li ----------
     int lim[NQT];
     float qf[NQT][DK][8];
@@ -321,11 +326,14 @@ __global__ __launch_bounds__(256) void decode_attention_mfma_kernel(AttnArgs a) 
       int l = 0;
       if (m < nq) {
         const int t = m / G, g = m % G;
-        const int64_t qo = q_base + int64_t(h * G + g) * a.q_sh + int64_t(t) * a.q_st;
+        int64_t qo[DK];
+#pragma unroll
+        for (int dk = 0; dk < DK; ++dk) qo[dk] = q_base + int64_t(h * G + g) * a.q_sh + int64_t(t) * a.q_st + 32 * dk + 8 * lg;
+        load_runs(a.q, a.q_dtype, qo, qf[qt]);
 #pragma unroll
         for (int dk = 0; dk < DK; ++dk)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) qf[qt][dk][e] = load_any(a.q, a.q_dtype, qo + 32 * dk + 8 * lg + e) * a.scale_log2;
+          for (int e = 0; e < 8; ++e) qf[qt][dk][e] *= a.scale_log2;
         int64_t lim64 = kl + t;
         if (lim64 > a.span) lim64 = a.span;
         l = (row_ok && lim64 > 0) ? int(lim64) : 0;
@@ -1338,6 +1346,15 @@ void launch_stream(const AttnArgs &a, hipStream_t s) {
   CG_LAUNCHED();
 }
 
+template <typename TKV, int D, int WAVES>
+void launch_d(const AttnArgs &a, hipStream_t s) {
+  decode_attention_kernel<TKV, D, WAVES><<<a.n_seqs * a.kv_heads, 64 * WAVES, 0, s>>>(a);
+  CG_LAUNCHED();
+}
+
+// Blocks along y for the query groups of a unit (the kernels stride over any beyond).
+unsigned groups(int queries, int per) { return unsigned(std::min((int64_t(queries) + per - 1) / per, int64_t(65535))); }
+
 template <typename TKV, int D>
 void launch_mfma(const AttnArgs &a, int queries, hipStream_t s) {
   const unsigned grid = unsigned((int64_t(a.n_seqs) * a.kv_heads + 3) / 4);
@@ -1352,18 +1369,25 @@ void launch_mfma(const AttnArgs &a, int queries, hipStream_t s) {
     if (qraw) return launch_tr<TKV, D, true>(a, queries, s);
     return launch_tr<TKV, D, false>(a, queries, s);
   } else {
-    if (queries <= 16) decode_attention_mfma_kernel<TKV, D, 1><<<grid, 256, 0, s>>>(a);
-    else if (queries <= 32) decode_attention_mfma_kernel<TKV, D, 2><<<grid, 256, 0, s>>>(a);
-    else decode_attention_mfma_kernel<TKV, D, 4><<<grid, 256, 0, s>>>(a);
+    const int64_t units = int64_t(a.n_seqs) * a.kv_heads;
+    // fp32 pools.  One-token rows of up to four heads per KV head: a block splits each unit's keys
+    // over its waves, four while the chip is not full of units (256 games of up to 256 keys: 9.1 us,
+    // two waves 10.4, the one-wave matrix-core kernel 20.2), two from 1024 units on (1024 games:
+    // 18.0 against 20.5 and 27.3).
+    if (D == 32 && queries <= QB && !a.seq_start) {
+      if (units < 1024) return launch_d<TKV, D, 4>(a, s);
+      return launch_d<TKV, D, 2>(a, s);
+    }
+    // More queries: one wave per 16 of a unit while that gives at most four waves per CU (64 rows x
+    // 16 tokens: 5.6 us, one wave per unit 11), else per 32 (256 x 64 tokens: 24 us against 47; 1024
+    // rows x 8 tokens on up to 480 keys: 54 against 92, 16 at a time 76).
+    if (queries <= 16 || units * ((queries + 15) / 16) <= 1024) {
+      decode_attention_mfma_kernel<TKV, D, 1><<<dim3(grid, groups(queries, 16)), 256, 0, s>>>(a);
+    } else {
+      decode_attention_mfma_kernel<TKV, D, 2><<<dim3(grid, groups(queries, 32)), 256, 0, s>>>(a);
+    }
     CG_LAUNCHED();
   }
-}
-
-template <typename TKV, int D>
-void launch_d(const AttnArgs &a, hipStream_t s) {
-  constexpr int WAVES = 4;
-  decode_attention_kernel<TKV, D, WAVES><<<a.n_seqs * a.kv_heads, 64 * WAVES, 0, s>>>(a);
-  CG_LAUNCHED();
 }
 
 template <typename TKV>
@@ -1374,15 +1398,11 @@ void launch_kv(const AttnArgs &a, hipStream_t s) {
   if (a.head_dim == 64) return launch_mfma<TKV, 64>(a, queries, s);
   switch (a.head_dim) {
     case 8:
-      return launch_d<TKV, 8>(a, s);
+      return launch_d<TKV, 8, 4>(a, s);
     case 16:
-      return launch_d<TKV, 16>(a, s);
+      return launch_d<TKV, 16, 4>(a, s);
     case 24:
-      return launch_d<TKV, 24>(a, s);
-    case 32:
-      return launch_d<TKV, 32>(a, s);
-    case 64:
-      return launch_d<TKV, 64>(a, s);
+      return launch_d<TKV, 24, 4>(a, s);
   }
   throw Error(CG_ERR_UNSUPPORTED,
               "decode attention is built for head_dim 8, 16, 24, 32 and 64, not " +

@@ -22,6 +22,21 @@ __device__ __forceinline__ float load_any(const void *p, int dtype, int64_t i) {
   }
 }
 
+// R runs of N consecutive elements at `at`: one branch on the type, then every load at once (a
+// branch per element makes each load wait for the one before).
+template <int R, int N>
+__device__ __forceinline__ void load_runs(const void *p, int dtype, const int64_t (&at)[R], float (&out)[R][N]) {
+  auto as = [&](auto *base) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int i = 0; i < N; ++i) out[r][i] = to_f32(base[at[r] + i]);
+  };
+  if (dtype == CG_F32) as(static_cast<const float *>(p));
+  else if (dtype == CG_BF16) as(static_cast<const bf16 *>(p));
+  else as(static_cast<const f16 *>(p));
+}
+
 __device__ __forceinline__ void store_any(void *p, int dtype, int64_t i, float v) {
   switch (dtype) {
     case CG_BF16:

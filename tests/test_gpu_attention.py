@@ -239,3 +239,23 @@ def test_packed_order_with_shared_work_and_many_units(device, B, distinct):
     work[rows >= capacity] = 0
     seq = work.repeat_interleave(kv_heads)[order.long()]
     assert bool((seq[:-1] >= seq[1:]).all())
+
+
+# fp32 pools on each side of the launch rules: whole-unit blocks of four and two waves (one token),
+# 16 and 32 queries per wave (padded runs), key counts around the 64-key blocks of the waves.
+@pytest.mark.parametrize("games, steps, longest", [(1, 1, 1), (3, 1, 64), (70, 1, 65), (511, 1, 257), (513, 1, 300),
+                                                   (5, 4, 63), (2, 17, 31), (150, 9, 130), (1, 130, 0)])
+def test_fp32_pool_launch_rules(device, games, steps, longest):
+    gen = torch.Generator(device=device).manual_seed(games * 1000 + steps)
+    randn = lambda *s: torch.randn(s, generator=gen, device=device)  # noqa: E731
+    max_len = longest + steps + 1
+    k, v, q = randn(games, 2, max_len, 32), randn(games, 2, max_len, 32), randn(games, 8, steps, 32)
+    rows = torch.randperm(games, generator=gen, device=device)
+    lengths = torch.randint(0, longest + 1, (games,), generator=gen, device=device) + 1
+    got = decode_attention(q, k, v, rows, lengths, max_len, 32**-0.5)
+    keys, values = (t[rows].double().repeat_interleave(4, 1) for t in (k, v))
+    scores = torch.matmul(q.double(), keys.transpose(-1, -2).contiguous()) * 32**-0.5
+    seen = lengths[:, None] + torch.arange(steps, device=device)
+    hidden = torch.arange(max_len, device=device)[None, None, None] >= seen[:, None, :, None]
+    want = torch.matmul(scores.masked_fill(hidden, float("-inf")).softmax(-1), values)
+    assert (got.double() - want).abs().max() <= 1e-5  # the fp32-pool bar of this file
