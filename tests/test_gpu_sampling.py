@@ -79,3 +79,35 @@ def test_rows_without_a_legal_entry_follow_numpy(device):
     uniforms = np.array([0.5, 0.5])
     assert (sample_rows(torch.from_numpy(got).to(device), torch.from_numpy(mask).to(device),
                         torch.from_numpy(uniforms).to(device)).cpu().numpy() == ref.sample_rows(want, mask, uniforms)).all()
+
+
+# Register-held rows (vector and scalar loads), wide rows, and 16 / 8 / 4 rows per sampling block,
+# with row counts that leave a block partly empty.
+@pytest.mark.parametrize("rows, width", [(1, 3), (17, 16), (5, 127), (66, 260), (33, 1020), (3, 1023), (9, 1025),
+                                         (7, 2047), (5, 4033), (6, 4096)])
+def test_every_row_shape_matches_the_oracle(device, rows, width):
+    logits, mask, rng = case(rows, width, 11 * rows + width)
+    mask[-1] = False
+    mask[-1, width // 2] = True  # one legal entry
+    got = masked_probabilities(torch.from_numpy(logits).to(device), torch.from_numpy(mask).to(device))
+    want = ref.masked_probabilities(logits, mask)
+    ulps = np.abs(got.cpu().numpy().view(np.int32).astype(np.int64) - want.view(np.int32).astype(np.int64))
+    assert ulps.max() <= 8 and (got.cpu().numpy()[~mask] == 0).all()
+    uniforms = rng.random(rows)
+    picked = sample_rows(torch.from_numpy(want).to(device), torch.from_numpy(mask).to(device),
+                         torch.from_numpy(uniforms).to(device)).cpu().numpy()
+    assert (picked == ref.sample_rows(want, mask, uniforms)).all()
+
+
+def test_pairwise_sum_order_is_numpys(device):
+    """With every logit equal the weights are 1, so the normaliser is exact in any order; with
+    logits of very different sizes its rounding shows the order of the additions."""
+
+    rng = np.random.default_rng(3)
+    for width in (9, 130, 500, 777, 1024, 1500, 4095):
+        logits = (rng.normal(size=(8, width)) * 4).astype(np.float32)
+        mask = np.ones((8, width), dtype=bool)
+        got = masked_probabilities(torch.from_numpy(logits).to(device), torch.from_numpy(mask).to(device)).cpu().numpy()
+        weights = torch.exp(torch.from_numpy(logits - logits.max(1, keepdims=True)).to(device)).cpu().numpy()
+        # torch's device exp is the same function, so only the order of the sum could differ
+        np.testing.assert_array_equal(got, weights / weights.sum(1, keepdims=True))
