@@ -4,7 +4,7 @@
 //
 //   * gemm_strided_kernel   C = alpha op(A) op(B) + beta C for any strides: the weight
 //                           gradients (dW = dY^T X) and input gradients (dX = dY W) of
-//                           every projection, on v_mfma_f32_16x16x4_f32;
+//                           every projection (split_tile.h);
 //   * layernorm_fwd / _bwd  LayerNorm keeping (mean, rstd) per row; the backward's input
 //                           gradient per row and per-block partial sums of dw / db;
 //   * rmsnorm_bwd           the input RMSNorm's backward (gain only);
@@ -13,8 +13,8 @@
 //                           the log-sum-exp of every (token, head);
 //   * attn_bwd_dq / _dkv    its backward: dQ (and D = rowsum(dO * O)) per (token, head),
 //                           dK / dV per (token, KV head) summed over the head group.
-// The attention kernels give each (token, head) one wave whose lanes take 64 keys (or
-// queries) at a time; head_dim is a template parameter (8 to 64).
+// The attention kernels work on 16 x 16 (query, key) tiles; head_dim is a template parameter
+// (8 to 64).
 #include <algorithm>
 #include <cmath>
 #include <string>
@@ -28,18 +28,12 @@ namespace {
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
 
 // bf16 (autocast) precision: values are kept in fp32 storage holding bf16 numbers.  A pair of
 // fp32 values to packed bf16, round to nearest even (v_cvt_pk_bf16_f32): a in the low half.
 __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
-}
-// Four consecutive k of an MFMA fragment as the bf16 operand of v_mfma_f32_16x16x16_bf16.
-__device__ __forceinline__ s16x4 bf16x4_of(f32x4 v) {
-  const u32x2 p = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
-  return __builtin_bit_cast(s16x4, p);
 }
 // The bf16 value nearest x, as fp32.
 __device__ __forceinline__ float round_bf16(float x) { return __builtin_bit_cast(float, pack_bf16(0.f, x) & 0xffff0000u); }
@@ -556,55 +550,71 @@ struct AttnTrain {
   const float *o, *dout, *lse;
   float *out, *lse_out, *dsum, *dq, *dk, *dv;
   int32_t round;  // bf16 outputs (o, dq, dk, dv), as SDPA on bf16 operands returns them
+  int32_t vec;    // output rows start 16-byte aligned
 };
 
 __device__ __forceinline__ float attn_out(const AttnTrain &a, float v) { return a.round ? round_bf16(v) : v; }
 
-// The three kernels work on 16 x 16 tiles of (query, key) pairs with v_mfma_f32_16x16x4_f32.
-// A contraction over head_dim gives lane (li, lg) the d slice [lg DC, (lg + 1) DC) (DC =
-// D / 4), one MFMA per d of the slice (the sum over d is the same whichever lane adds which
-// term).  A score tile leaves its MFMA with lane (li, lg) holding rows 4 lg + r, column li;
-// a contraction over those rows (keys or queries) is the four MFMAs r = 0..3, MFMA r taking
-// rows {4 lg + r} from the lane's own registers, so scores never leave the lane.  Outputs
-// over d come out transposed ([d][row]) so that each lane stores four consecutive d.
-constexpr int KT = 64;  // keys per staged K / V tile (forward and dQ)
+// The three kernels work on 16 x 16 tiles of (query, key) pairs with v_mfma_f32_16x16x32_bf16.
+// PARTS 3: fp32 operands in three bf16 parts (split.h); PARTS 1: operands that hold bf16 numbers
+// (the bf16 trunk's q, k, v and dO), so one part is exact.  Probabilities and dS are fp32 and
+// always multiplied in three parts.  A contraction over head_dim (padded to 32) takes both
+// operands with lane (li, lg) holding d = 8 lg .. 8 lg + 7.  A score tile leaves its MFMA with
+// lane (li, lg) holding rows 4 lg + r, column li; a contraction over those rows (keys or queries)
+// takes 32 of them, two score tiles, with lane group lg's k the rows {4 lg + r} of the one and
+// {16 + 4 lg + r} of the other, so scores never leave the lane.  Staged tiles are therefore kept
+// in up to two LDS layouts: by rows (a lane's eight d of a row) and by columns (a lane's eight
+// rows of a d).  Outputs over d come out transposed ([d][row]): each lane stores four consecutive
+// d.  What bounds them is the VALU work per score (exp, masks, splitting), so masks are only
+// evaluated in tiles that some query sees partly.
+constexpr int KT = 64;  // rows (keys, or queries of a dK / dV unit) per staged tile
 
-template <int D>
+template <int D, int PARTS>
 struct AttnDims {
-  static constexpr int DC = D / 4;                      // d per lane in a contraction over d
-  static constexpr int DT = (D + 15) / 16;              // 16-wide d tiles of an output
-  static constexpr int LD = DT * 16 + 4;                // LDS row, floats; d in [D, 16 DT) hold 0
-  static constexpr int C4 = D / 4;                      // float4 per row
-  static constexpr int PER_KV = (2 * KT * C4 + 255) / 256;  // float4 per thread, one K + V tile
-  static constexpr int QR = D <= 32 ? 64 : 32;             // query tokens per dK / dV unit (VGPRs bound it at 64)
-  static constexpr int QH = QR / 16;                        // its 16-query sub-tiles
-  static constexpr int PER_Q = (2 * QR * C4 + 255) / 256;   // float4 per thread, one Q + dO unit
+  static constexpr int DK = (D + 31) / 32;  // 32-wide d slices of a contraction over d
+  static constexpr int DT = (D + 15) / 16;  // 16-wide d tiles of an output
+  static constexpr int C4 = D / 4;
+  static constexpr int SLOTS = 32 * C4;                 // a slot: two rows x four d
+  static constexpr int PER = (SLOTS + 255) / 256;       // slots per thread
+  static constexpr int ROW_PART = 4096 * DK, COL_PART = 2048 * DT;  // bytes of one part of a tile
+  static constexpr int ROWS = PARTS * ROW_PART, COLS = PARTS * COL_PART;
 };
 
-template <int DC>
-__device__ __forceinline__ void lds_slice(const float *p, float (&out)[DC]) {
-  if constexpr (DC % 4 == 0) {
-#pragma unroll
-    for (int i = 0; i < DC; i += 4) {
-      const float4 v = *reinterpret_cast<const float4 *>(p + i);
-      out[i] = v.x;
-      out[i + 1] = v.y;
-      out[i + 2] = v.z;
-      out[i + 3] = v.w;
-    }
+// The parts of one MFMA operand.
+template <int PARTS>
+struct Operand {
+  split_u32x4 p[PARTS];
+};
+template <int D, int PARTS>
+using DimOperand = Operand<PARTS>[AttnDims<D, PARTS>::DK];
+// A thread's slots of a staged tile: two rows' four d each.
+template <int D, int PARTS>
+using SlotRegs = float4[AttnDims<D, PARTS>::PER][2];
+
+template <int PARTS>
+__device__ __forceinline__ Operand<PARTS> operand_of(const float (&v)[8]) {
+  Operand<PARTS> o;
+  const f32x4 x = {v[0], v[1], v[2], v[3]}, y = {v[4], v[5], v[6], v[7]};
+  if constexpr (PARTS == 3) {
+    const Split8 s = split8(x, y);
+    o.p[0] = s.hi, o.p[1] = s.mid, o.p[2] = s.lo;
   } else {
-    static_assert(DC % 2 == 0, "head_dim a multiple of 8");
-#pragma unroll
-    for (int i = 0; i < DC; i += 2) {
-      const float2 v = *reinterpret_cast<const float2 *>(p + i);
-      out[i] = v.x;
-      out[i + 1] = v.y;
-    }
+    o.p[0] = split_u32x4{split_pack(x[0], x[1]), split_pack(x[2], x[3]), split_pack(y[0], y[1]), split_pack(y[2], y[3])};
   }
+  return o;
 }
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+// c + a b, smallest products first.
+template <int PA, int PB>
+__device__ __forceinline__ f32x4 mma_parts(const Operand<PA> &a, const Operand<PB> &b, f32x4 c) {
+#pragma unroll
+  for (int order = 2; order >= 0; --order)
+#pragma unroll
+    for (int i = 0; i < PA; ++i)
+#pragma unroll
+      for (int j = 0; j < PB; ++j)
+        if (i + j == order) c = split_mma1(a.p[i], b.p[j], c);
+  return c;
 }
 
 __device__ __forceinline__ float max_over_rows(float x) {  // over lanes li, li + 16, li + 32, li + 48
@@ -617,44 +627,137 @@ __device__ __forceinline__ float sum_over_rows(float x) {
   return x + __shfl_xor(x, 32);
 }
 
-// Zeroes the d >= D columns of `rows` LDS rows (they feed output rows that are never stored).
-template <int D>
-__device__ __forceinline__ void zero_pad(float *t, int rows) {
-  using S = AttnDims<D>;
-  constexpr int W = S::DT * 16 - D;
-  if constexpr (W > 0)
-    for (int i = threadIdx.x; i < rows * W; i += blockDim.x) t[(i / W) * S::LD + D + i % W] = 0.f;
+// Clears LDS once: the d >= D padding of a staged tile is read (times zero or into output rows
+// that are never stored) and never written.
+__device__ __forceinline__ void clear_lds(char *lds, int bytes) {
+  for (int i = threadIdx.x * 16; i < bytes; i += 256 * 16) *reinterpret_cast<split_u32x4 *>(lds + i) = split_u32x4{0, 0, 0, 0};
 }
 
-// K / V tile of keys [j0, j0 + KT) of KV head hk (rows past n read 0), global -> registers -> LDS.
-template <int D>
-__device__ __forceinline__ void kv_load(const AttnTrain &a, int hk, int64_t j0, float4 (&r)[AttnDims<D>::PER_KV]) {
-  using S = AttnDims<D>;
+// Rows [r0, r0 + 64) of p (row stride ld floats, D used columns) into registers; rows outside
+// [0, last] read 0.
+template <int D, int PARTS>
+__device__ __forceinline__ void rows_load(SlotRegs<D, PARTS> &r, const float *__restrict__ p, int64_t ld,
+                                          int64_t r0, int64_t last) {
+  using S = AttnDims<D, PARTS>;
 #pragma unroll
-  for (int e = 0; e < S::PER_KV; ++e) {
-    const int i = threadIdx.x + 256 * e;
-    float4 x = {0.f, 0.f, 0.f, 0.f};
-    if (i < 2 * KT * S::C4) {
-      const bool isv = i >= KT * S::C4;
-      const int ii = isv ? i - KT * S::C4 : i, row = ii / S::C4, c = (ii % S::C4) * 4;
-      const int64_t j = j0 + row;
-      if (j < a.n) x = *reinterpret_cast<const float4 *>((isv ? a.v + j * a.ldv : a.k + j * a.ldk) + hk * D + c);
+  for (int e = 0; e < S::PER; ++e) {
+    const int slot = threadIdx.x + 256 * e, c = (slot % S::C4) * 4;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t row = r0 + 2 * (slot / S::C4) + h;
+      const bool in = slot < S::SLOTS && row <= last;
+      const float4 v = *reinterpret_cast<const float4 *>(p + (in ? row * ld + c : 0));
+      r[e][h] = in ? v : float4{0.f, 0.f, 0.f, 0.f};
     }
-    r[e] = x;
   }
 }
 
-template <int D>
-__device__ __forceinline__ void kv_store(float *kt, float *vt, const float4 (&r)[AttnDims<D>::PER_KV]) {
-  using S = AttnDims<D>;
+// The parts of a slot: per row (h), per part, its four d packed.
+template <int PARTS>
+__device__ __forceinline__ void slot_parts(const float4 (&v)[2], unsigned (&out)[2][PARTS][2]) {
 #pragma unroll
-  for (int e = 0; e < S::PER_KV; ++e) {
-    const int i = threadIdx.x + 256 * e;
-    if (i < 2 * KT * S::C4) {
-      const bool isv = i >= KT * S::C4;
-      const int ii = isv ? i - KT * S::C4 : i, row = ii / S::C4, c = (ii % S::C4) * 4;
-      *reinterpret_cast<float4 *>((isv ? vt : kt) + row * S::LD + c) = r[e];
+  for (int h = 0; h < 2; ++h) {
+    if constexpr (PARTS == 3) {
+      split_pair(v[h].x, v[h].y, out[h][0][0], out[h][1][0], out[h][2][0]);
+      split_pair(v[h].z, v[h].w, out[h][0][1], out[h][1][1], out[h][2][1]);
+    } else {
+      out[h][0][0] = split_pack(v[h].x, v[h].y);
+      out[h][0][1] = split_pack(v[h].z, v[h].w);
     }
+  }
+}
+
+// Registers -> LDS: by rows (tile_offset per 32-d slice) and / or by columns: row kappa of a
+// 32-row half u is value (kappa & 3) + 4 (kappa >> 4) of lane group (kappa >> 2) & 3, [u][16-d
+// tile][lane group][d, exclusive-or'ed with the lane group][8 rows].
+template <int D, int PARTS, bool BY_ROWS, bool BY_COLS>
+__device__ __forceinline__ void rows_store(char *rows, char *cols, const SlotRegs<D, PARTS> &r) {
+  using S = AttnDims<D, PARTS>;
+#pragma unroll
+  for (int e = 0; e < S::PER; ++e) {
+    const int slot = threadIdx.x + 256 * e;
+    if (slot >= S::SLOTS) continue;
+    const int c = (slot % S::C4) * 4, row = 2 * (slot / S::C4);
+    unsigned v[2][PARTS][2];
+    slot_parts<PARTS>(r[e], v);
+    if constexpr (BY_ROWS) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        char *to = rows + (c >> 5) * 4096 + tile_offset(row + h, (c >> 3) & 3) + (c & 4) * 2;
+#pragma unroll
+        for (int q = 0; q < PARTS; ++q) *reinterpret_cast<u32x2 *>(to + q * S::ROW_PART) = u32x2{v[h][q][0], v[h][q][1]};
+      }
+    }
+    if constexpr (BY_COLS) {
+      const int u = row >> 5, kappa = row & 31, lg = (kappa >> 2) & 3, at = (kappa & 3) + 4 * (kappa >> 4);
+      char *to = cols + u * 1024 * S::DT + (c >> 4) * 1024 + lg * 256 + at * 2;
+#pragma unroll
+      for (int q = 0; q < PARTS; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const unsigned a = v[0][q][i >> 1], b = v[1][q][i >> 1];
+          const unsigned w = i & 1 ? (a >> 16) | (b & 0xffff0000u) : (a & 0xffffu) | (b << 16);
+          *reinterpret_cast<unsigned *>(to + q * S::COL_PART + ((((c + i) & 15) ^ lg) << 4)) = w;
+        }
+    }
+  }
+}
+
+// A operand fragments: 16 rows `sub` of slice dk by rows; 16 d `dt` over the 32 rows `u` by columns.
+template <int D, int PARTS>
+__device__ __forceinline__ Operand<PARTS> row_frag(const char *rows, int sub, int dk, int li, int lg) {
+  Operand<PARTS> o;
+#pragma unroll
+  for (int q = 0; q < PARTS; ++q)
+    o.p[q] = *reinterpret_cast<const split_u32x4 *>(rows + q * AttnDims<D, PARTS>::ROW_PART + dk * 4096 +
+                                                    tile_offset(16 * sub + li, lg));
+  return o;
+}
+template <int D, int PARTS>
+__device__ __forceinline__ Operand<PARTS> col_frag(const char *cols, int u, int dt, int li, int lg) {
+  using S = AttnDims<D, PARTS>;
+  Operand<PARTS> o;
+#pragma unroll
+  for (int q = 0; q < PARTS; ++q)
+    o.p[q] = *reinterpret_cast<const split_u32x4 *>(cols + q * S::COL_PART + (u * S::DT + dt) * 1024 + lg * 256 +
+                                                    ((li ^ lg) << 4));
+  return o;
+}
+
+// A lane's eight d of one row (d = 32 dk + 8 lg ..) as a B operand; zero when !live or past D.
+template <int D, int PARTS>
+__device__ __forceinline__ void row_operand(DimOperand<D, PARTS> &o, const float *__restrict__ p,
+                                            bool live, int lg) {
+#pragma unroll
+  for (int dk = 0; dk < AttnDims<D, PARTS>::DK; ++dk) {
+    float v[8];
+    const int d = 32 * dk + 8 * lg;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float4 x = live && d < D ? *reinterpret_cast<const float4 *>(p + d + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
+      v[4 * h] = x.x, v[4 * h + 1] = x.y, v[4 * h + 2] = x.z, v[4 * h + 3] = x.w;
+    }
+    o[dk] = operand_of<PARTS>(v);
+  }
+}
+
+// Two score tiles' values as the B operand of a contraction over their 32 rows.
+__device__ __forceinline__ Operand<3> score_operand(const f32x4 &a, const f32x4 &b) {
+  const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  return operand_of<3>(v);
+}
+
+// Four consecutive d of an output row.
+__device__ __forceinline__ void store4(const AttnTrain &a, float *p, const f32x4 &v, float scale) {
+  const float4 o = {attn_out(a, v[0] * scale), attn_out(a, v[1] * scale), attn_out(a, v[2] * scale),
+                    attn_out(a, v[3] * scale)};
+  if (a.vec) {
+    *reinterpret_cast<float4 *>(p) = o;
+  } else {
+    p[0] = o.x;
+    p[1] = o.y;
+    p[2] = o.z;
+    p[3] = o.w;
   }
 }
 
@@ -681,13 +784,16 @@ __device__ __forceinline__ QueryStrip query_strip(const AttnTrain &a) {
   return q;
 }
 
-// Forward: online softmax over K / V tiles staged KT keys at a time.  S^T = K Q^T (keys on
+constexpr float LOG2E = 1.4426950408889634f;
+
+// Forward: online softmax (base 2) over K / V tiles staged KT keys at a time.  S^T = K Q^T (keys on
 // the rows, the lane's query li on the column), row statistics per query across the four
 // lanes li + 16 lg, O^T += V^T P^T.
-template <int D>
+template <int D, int PARTS>
 __global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnTrain a) {
-  using S = AttnDims<D>;
-  __shared__ __align__(16) float kt[2][KT * S::LD], vt[2][KT * S::LD];
+  using S = AttnDims<D, PARTS>;
+  __shared__ __align__(16) char lds[S::ROWS + S::COLS];
+  char *const kr = lds, *const vc = lds + S::ROWS;
   const int hk = blockIdx.y, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const QueryStrip w = query_strip(a);
   const int64_t t = w.t0 + li, w_last = min<int64_t>(a.n - 1, w.t0 + 15);
@@ -695,92 +801,87 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnTrain a) {
   const int64_t start = live ? a.seq_start[a.seq_of[t]] : 0;
   const int64_t w_first = w.active ? a.seq_start[a.seq_of[w.t0]] : 0;  // first key any query of the strip sees
   const int64_t k_lo = a.seq_start[a.seq_of[w.base]];
-  zero_pad<D>(kt[0], 2 * KT);
-  zero_pad<D>(vt[0], 2 * KT);
-  float qf[S::DC];
-#pragma unroll
-  for (int kk = 0; kk < S::DC; ++kk) qf[kk] = live ? a.q[t * a.ldq + w.h * D + lg * S::DC + kk] * a.scale : 0.f;
+  const float scale = a.scale * LOG2E;
+  clear_lds(lds, S::ROWS + S::COLS);
+  Operand<PARTS> qf[S::DK];
+  row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg);
   f32x4 acc[S::DT];
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -1e30f, l = 0.f;
-  float4 pre[S::PER_KV];
-  kv_load<D>(a, hk, k_lo, pre);
-  kv_store<D>(kt[0], vt[0], pre);
-  __syncthreads();
-  int buf = 0;
+  float4 kp[S::PER][2], vp[S::PER][2];
+  rows_load<D, PARTS>(kp, a.k + hk * D, a.ldk, k_lo, w.b_last);
+  rows_load<D, PARTS>(vp, a.v + hk * D, a.ldv, k_lo, w.b_last);
   for (int64_t j0 = k_lo; j0 <= w.b_last; j0 += KT) {
-    const bool more = j0 + KT <= w.b_last;
-    if (more) kv_load<D>(a, hk, j0 + KT, pre);  // the next tile's loads fly during this one's MFMAs
-    if (w.active && j0 <= w_last && j0 + KT - 1 >= w_first) {
-      const float *K = kt[buf], *V = vt[buf];
-      f32x4 s[4];
-      bool any[4];
-      float mt = -INFINITY;
+    __syncthreads();  // the tile before (and the clearing) is done with
+    rows_store<D, PARTS, true, false>(kr, nullptr, kp);
+    rows_store<D, PARTS, false, true>(nullptr, vc, vp);
+    __syncthreads();
+    if (j0 + KT <= w.b_last) {  // the next tile's loads fly during this one's products
+      rows_load<D, PARTS>(kp, a.k + hk * D, a.ldk, j0 + KT, w.b_last);
+      rows_load<D, PARTS>(vp, a.v + hk * D, a.ldv, j0 + KT, w.b_last);
+    }
+    if (!(w.active && j0 <= w_last && j0 + KT - 1 >= w_first)) continue;
+    // The lane's query sees the tile's keys lo .. hi.
+    const int lo = live ? int(max<int64_t>(start - j0, 0)) : KT, hi = live ? int(min<int64_t>(t - j0, KT - 1)) : -1;
+    const bool whole = __all(lo == 0 && hi == KT - 1);
+    f32x4 s[4];
+    bool any[4];
+    float mt = -INFINITY;
 #pragma unroll
-      for (int sub = 0; sub < 4; ++sub) {
-        const int64_t jb = j0 + 16 * sub;
-        any[sub] = jb <= w_last && jb + 15 >= w_first;
-        s[sub] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-        if (any[sub]) {
-          float kf[S::DC];
-          lds_slice<S::DC>(K + (16 * sub + li) * S::LD + lg * S::DC, kf);
-          f32x4 c = {0.f, 0.f, 0.f, 0.f};
+    for (int sub = 0; sub < 4; ++sub) {
+      const int64_t jb = j0 + 16 * sub;
+      any[sub] = jb <= w_last && jb + 15 >= w_first;
+      s[sub] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (!any[sub]) continue;
+      f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int kk = 0; kk < S::DC; ++kk) c = mfma4(kf[kk], qf[kk], c);
+      for (int dk = 0; dk < S::DK; ++dk) c = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(kr, sub, dk, li, lg), qf[dk], c);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int64_t j = jb + 4 * lg + r;
-            s[sub][r] = (live && j >= start && j <= t) ? c[r] : -INFINITY;
-            mt = fmaxf(mt, s[sub][r]);
-          }
-        }
-      }
-      mt = max_over_rows(mt);
-      const float mn = fmaxf(m, mt);
-      const float corr = __expf(m - mn);
-      m = mn;
-      l *= corr;
-#pragma unroll
-      for (int dt = 0; dt < S::DT; ++dt) acc[dt] *= corr;
-#pragma unroll
-      for (int sub = 0; sub < 4; ++sub) {
-        if (!any[sub]) continue;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[sub][r] = __expf(s[sub][r] - mn);
-          l += s[sub][r];
-        }
-#pragma unroll
-        for (int dt = 0; dt < S::DT; ++dt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[dt] = mfma4(V[(16 * sub + 4 * lg + r) * S::LD + dt * 16 + li], s[sub][r], acc[dt]);
+      for (int r = 0; r < 4; ++r) {
+        const int kk = 16 * sub + 4 * lg + r;
+        s[sub][r] = whole || (kk >= lo && kk <= hi) ? c[r] * scale : -INFINITY;
+        mt = fmaxf(mt, s[sub][r]);
       }
     }
-    if (more) kv_store<D>(kt[buf ^ 1], vt[buf ^ 1], pre);
-    __syncthreads();
-    buf ^= 1;
+    mt = max_over_rows(mt);
+    const float mn = fmaxf(m, mt);
+    const float corr = __builtin_amdgcn_exp2f(m - mn);
+    m = mn;
+    l *= corr;
+#pragma unroll
+    for (int dt = 0; dt < S::DT; ++dt) acc[dt] *= corr;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (!any[2 * u] && !any[2 * u + 1]) continue;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[2 * u + h][r] = __builtin_amdgcn_exp2f(s[2 * u + h][r] - mn);
+          l += s[2 * u + h][r];
+        }
+      const Operand<3> p = score_operand(s[2 * u], s[2 * u + 1]);
+#pragma unroll
+      for (int dt = 0; dt < S::DT; ++dt) acc[dt] = mma_parts<PARTS, 3>(col_frag<D, PARTS>(vc, u, dt, li, lg), p, acc[dt]);
+    }
   }
   l = sum_over_rows(l);
   if (!live) return;
-  const float inv = 1.0f / l;
   float *orow = a.out + (t * a.H + w.h) * D;
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = dt * 16 + 4 * lg + r;
-      if (d < D) orow[d] = attn_out(a, acc[dt][r] * inv);
-    }
-  if (lg == 0) a.lse_out[t * a.H + w.h] = m + logf(l);
+    if (dt * 16 + 4 * lg < D) store4(a, orow + dt * 16 + 4 * lg, acc[dt], 1.0f / l);
+  if (lg == 0) a.lse_out[t * a.H + w.h] = m * 0.6931471805599453f + logf(l);
 }
 
 // dQ (and D = rowsum(dO * O)) with the forward's blocks: S^T = K Q^T and dP^T = V dO^T per
 // 16-key tile, P from the saved log-sum-exp, dS = P (dP - D), dQ^T += K^T dS^T.
-template <int D>
+template <int D, int PARTS>
 __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const AttnTrain a) {
-  using S = AttnDims<D>;
-  __shared__ __align__(16) float kt[2][KT * S::LD], vt[2][KT * S::LD];
+  using S = AttnDims<D, PARTS>;
+  __shared__ __align__(16) char lds[2 * S::ROWS + S::COLS];
+  char *const kr = lds, *const vr = lds + S::ROWS, *const kc = lds + 2 * S::ROWS;
   const int hk = blockIdx.y, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const QueryStrip w = query_strip(a);
   const int64_t t = w.t0 + li, w_last = min<int64_t>(a.n - 1, w.t0 + 15);
@@ -789,136 +890,86 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const AttnTrain a) {
   const int64_t start = live ? a.seq_start[a.seq_of[t]] : 0;
   const int64_t w_first = w.active ? a.seq_start[a.seq_of[w.t0]] : 0;
   const int64_t k_lo = a.seq_start[a.seq_of[w.base]];
-  zero_pad<D>(kt[0], 2 * KT);
-  zero_pad<D>(vt[0], 2 * KT);
-  float qf[S::DC], gf[S::DC];
+  const float scale = a.scale * LOG2E;
+  clear_lds(lds, 2 * S::ROWS + S::COLS);
+  Operand<PARTS> qf[S::DK], gf[S::DK];
+  row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg);
+  row_operand<D, PARTS>(gf, a.dout + row * D, live, lg);
   float part = 0.f;
 #pragma unroll
-  for (int kk = 0; kk < S::DC; ++kk) {
-    const int d = lg * S::DC + kk;
-    qf[kk] = live ? a.q[t * a.ldq + w.h * D + d] * a.scale : 0.f;
-    gf[kk] = live ? a.dout[row * D + d] : 0.f;
-    part = fmaf(gf[kk], live ? a.o[row * D + d] : 0.f, part);
-  }
+  for (int dk = 0; dk < S::DK; ++dk)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int d = 32 * dk + 8 * lg + 4 * h;
+      if (!live || d >= D) continue;
+      const float4 g = *reinterpret_cast<const float4 *>(a.dout + row * D + d);
+      const float *o = a.o + row * D + d;
+      part = fmaf(g.x, o[0], fmaf(g.y, o[1], fmaf(g.z, o[2], fmaf(g.w, o[3], part))));
+    }
   const float dsum = sum_over_rows(part);
-  const float lse = live ? a.lse[row] : 0.f;
+  const float lse = live ? a.lse[row] * LOG2E : 0.f;
   f32x4 acc[S::DT];
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float4 pre[S::PER_KV];
-  kv_load<D>(a, hk, k_lo, pre);
-  kv_store<D>(kt[0], vt[0], pre);
-  __syncthreads();
-  int buf = 0;
+  float4 kp[S::PER][2], vp[S::PER][2];
+  rows_load<D, PARTS>(kp, a.k + hk * D, a.ldk, k_lo, w.b_last);
+  rows_load<D, PARTS>(vp, a.v + hk * D, a.ldv, k_lo, w.b_last);
   for (int64_t j0 = k_lo; j0 <= w.b_last; j0 += KT) {
-    const bool more = j0 + KT <= w.b_last;
-    if (more) kv_load<D>(a, hk, j0 + KT, pre);
-    if (w.active && j0 <= w_last && j0 + KT - 1 >= w_first) {
-      const float *K = kt[buf], *V = vt[buf];
+    __syncthreads();
+    rows_store<D, PARTS, true, true>(kr, kc, kp);
+    rows_store<D, PARTS, true, false>(vr, nullptr, vp);
+    __syncthreads();
+    if (j0 + KT <= w.b_last) {
+      rows_load<D, PARTS>(kp, a.k + hk * D, a.ldk, j0 + KT, w.b_last);
+      rows_load<D, PARTS>(vp, a.v + hk * D, a.ldv, j0 + KT, w.b_last);
+    }
+    if (!(w.active && j0 <= w_last && j0 + KT - 1 >= w_first)) continue;
+    const int lo = live ? int(max<int64_t>(start - j0, 0)) : KT, hi = live ? int(min<int64_t>(t - j0, KT - 1)) : -1;
+    const bool whole = __all(lo == 0 && hi == KT - 1);
 #pragma unroll
-      for (int sub = 0; sub < 4; ++sub) {
-        const int64_t jb = j0 + 16 * sub;
-        if (!(jb <= w_last && jb + 15 >= w_first)) continue;
-        float kf[S::DC], vf[S::DC];
-        lds_slice<S::DC>(K + (16 * sub + li) * S::LD + lg * S::DC, kf);
-        lds_slice<S::DC>(V + (16 * sub + li) * S::LD + lg * S::DC, vf);
+    for (int u = 0; u < 2; ++u) {
+      const int64_t jb = j0 + 32 * u;
+      if (!(jb <= w_last && jb + 31 >= w_first)) continue;
+      f32x4 ds[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int sub = 2 * u + h;
         f32x4 st = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kk = 0; kk < S::DC; ++kk) {
-          st = mfma4(kf[kk], qf[kk], st);
-          dp = mfma4(vf[kk], gf[kk], dp);
+        for (int dk = 0; dk < S::DK; ++dk) {
+          st = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(kr, sub, dk, li, lg), qf[dk], st);
+          dp = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(vr, sub, dk, li, lg), gf[dk], dp);
         }
-        f32x4 ds;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int64_t j = jb + 4 * lg + r;
-          const float p = (live && j >= start && j <= t) ? __expf(st[r] - lse) : 0.f;
-          ds[r] = p * (dp[r] - dsum);
+          const int kk = 16 * sub + 4 * lg + r;
+          const float p = whole || (kk >= lo && kk <= hi) ? __builtin_amdgcn_exp2f(fmaf(st[r], scale, -lse)) : 0.f;
+          ds[h][r] = p * (dp[r] - dsum);
         }
-#pragma unroll
-        for (int dt = 0; dt < S::DT; ++dt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[dt] = mfma4(K[(16 * sub + 4 * lg + r) * S::LD + dt * 16 + li], ds[r], acc[dt]);
       }
+      const Operand<3> dso = score_operand(ds[0], ds[1]);
+#pragma unroll
+      for (int dt = 0; dt < S::DT; ++dt) acc[dt] = mma_parts<PARTS, 3>(col_frag<D, PARTS>(kc, u, dt, li, lg), dso, acc[dt]);
     }
-    if (more) kv_store<D>(kt[buf ^ 1], vt[buf ^ 1], pre);
-    __syncthreads();
-    buf ^= 1;
   }
   if (!live) return;
   float *dqrow = a.dq + t * a.ldq + w.h * D;
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = dt * 16 + 4 * lg + r;
-      if (d < D) dqrow[d] = attn_out(a, acc[dt][r] * a.scale);
-    }
+    if (dt * 16 + 4 * lg < D) store4(a, dqrow + dt * 16 + 4 * lg, acc[dt], a.scale);
   if (lg == 0) a.dsum[row] = dsum;
 }
 
-// One staged query unit of the dK / dV kernel: QR tokens of one head (q scaled, dO, lse, D).
-template <int D>
-struct QueryUnit {
-  float4 v[AttnDims<D>::PER_Q];
-  float s;
-};
-
-template <int D>
-__device__ __forceinline__ QueryUnit<D> unit_load(const AttnTrain &a, int h, int64_t t0) {
-  using S = AttnDims<D>;
-  QueryUnit<D> u;
-#pragma unroll
-  for (int e = 0; e < S::PER_Q; ++e) {
-    const int i = threadIdx.x + 256 * e;
-    float4 x = {0.f, 0.f, 0.f, 0.f};
-    if (i < 2 * S::QR * S::C4) {
-      const bool isg = i >= S::QR * S::C4;
-      const int ii = isg ? i - S::QR * S::C4 : i, row = ii / S::C4, c = (ii % S::C4) * 4;
-      const int64_t t = t0 + row;
-      if (t < a.n) {
-        if (isg) {
-          x = *reinterpret_cast<const float4 *>(a.dout + (t * a.H + h) * D + c);
-        } else {
-          x = *reinterpret_cast<const float4 *>(a.q + t * a.ldq + h * D + c);
-          x.x *= a.scale;
-          x.y *= a.scale;
-          x.z *= a.scale;
-          x.w *= a.scale;
-        }
-      }
-    }
-    u.v[e] = x;
-  }
-  u.s = 0.f;
-  const int64_t t = t0 + (threadIdx.x % S::QR);
-  if (threadIdx.x < 2 * S::QR && t < a.n) u.s = threadIdx.x < S::QR ? a.lse[t * a.H + h] : a.dsum[t * a.H + h];
-  return u;
-}
-
-template <int D>
-__device__ __forceinline__ void unit_store(float *qs, float *gs, float *ls, const QueryUnit<D> &u) {
-  using S = AttnDims<D>;
-#pragma unroll
-  for (int e = 0; e < S::PER_Q; ++e) {
-    const int i = threadIdx.x + 256 * e;
-    if (i < 2 * S::QR * S::C4) {
-      const bool isg = i >= S::QR * S::C4;
-      const int ii = isg ? i - S::QR * S::C4 : i, row = ii / S::C4, c = (ii % S::C4) * 4;
-      *reinterpret_cast<float4 *>((isg ? gs : qs) + row * S::LD + c) = u.v[e];
-    }
-  }
-  if (threadIdx.x < 2 * S::QR) ls[threadIdx.x] = u.s;  // [0, S::QR) lse, [S::QR, 2 S::QR) D
-}
-
 // dK / dV: a block holds 64 keys of KV head blockIdx.y, wave w keys j0 + 16 w + li in
-// registers, and walks the units (16-token tile, head of the group) that can see them,
+// registers, and walks the units (KT tokens of one head of the group) that can see them,
 // staged through LDS.  S = Q K^T and dP = dO V^T (queries on the rows), P and dS per lane,
-// dV^T += dO^T P and dK^T += Q^T dS (q staged scaled, so dK needs no further scale).
-template <int D>
+// dV^T += dO^T P and dK^T += Q^T dS.
+template <int D, int PARTS>
 __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
-  using S = AttnDims<D>;
-  __shared__ __align__(16) float qs[2][S::QR * S::LD], gs[2][S::QR * S::LD], ls[2][2 * S::QR];
+  using S = AttnDims<D, PARTS>;
+  __shared__ __align__(16) char lds[2 * S::ROWS + 2 * S::COLS];
+  __shared__ __align__(16) float ls[2 * KT];
+  char *const qr = lds, *const gr = lds + S::ROWS, *const qc = lds + 2 * S::ROWS, *const gc = qc + S::COLS;
   const int G = a.H / a.KVH, hk = blockIdx.y;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int64_t j0 = int64_t(blockIdx.x) * 64, jw = j0 + 16 * wave, j = jw + li;
@@ -926,93 +977,80 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
   const int64_t end = live ? a.seq_start[a.seq_of[j] + 1] : 0;
   const int64_t w_hi = wave_live ? a.seq_start[a.seq_of[min<int64_t>(a.n - 1, jw + 15)] + 1] : 0;
   const int64_t q_hi = a.seq_start[a.seq_of[min<int64_t>(a.n - 1, j0 + 63)] + 1];
-  const int units = int((q_hi - j0 + S::QR - 1) / S::QR) * G;
-  zero_pad<D>(qs[0], 2 * S::QR);
-  zero_pad<D>(gs[0], 2 * S::QR);
-  float kf[S::DC], vf[S::DC];
-#pragma unroll
-  for (int kk = 0; kk < S::DC; ++kk) {
-    const int d = lg * S::DC + kk;
-    kf[kk] = live ? a.k[j * a.ldk + hk * D + d] : 0.f;
-    vf[kk] = live ? a.v[j * a.ldv + hk * D + d] : 0.f;
-  }
+  const int units = int((q_hi - j0 + KT - 1) / KT) * G;
+  const float scale = a.scale * LOG2E;
+  clear_lds(lds, 2 * S::ROWS + 2 * S::COLS);
+  Operand<PARTS> kf[S::DK], vf[S::DK];
+  row_operand<D, PARTS>(kf, a.k + j * a.ldk + hk * D, live, lg);
+  row_operand<D, PARTS>(vf, a.v + j * a.ldv + hk * D, live, lg);
   f32x4 dk[S::DT], dv[S::DT];
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt) {
     dk[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     dv[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  unit_store<D>(qs[0], gs[0], ls[0], unit_load<D>(a, hk * G, j0));
-  __syncthreads();
-  int buf = 0;
+  float4 qp[S::PER][2], gp[S::PER][2];
+  float sp = 0.f;
+  auto load = [&](int u) {
+    const int h = hk * G + u % G;
+    const int64_t t0 = j0 + KT * (u / G), last = min<int64_t>(a.n, q_hi) - 1;
+    rows_load<D, PARTS>(qp, a.q + h * D, a.ldq, t0, last);
+    rows_load<D, PARTS>(gp, a.dout + h * D, int64_t(a.H) * D, t0, last);
+    const int64_t t = t0 + (threadIdx.x & (KT - 1));
+    if (threadIdx.x < 2 * KT)
+      sp = t > last ? 0.f : threadIdx.x < KT ? a.lse[t * a.H + h] * LOG2E : a.dsum[t * a.H + h];
+  };
+  load(0);
   for (int u = 0; u < units; ++u) {
-    const bool more = u + 1 < units;
-    QueryUnit<D> next;
-    if (more) next = unit_load<D>(a, hk * G + (u + 1) % G, j0 + S::QR * ((u + 1) / G));
-    const int64_t t0 = j0 + S::QR * (u / G);
-    // The unit's 16-query sub-tiles: independent S / dP chains, then the dV / dK updates.
-    bool act[S::QH];
+    __syncthreads();
+    rows_store<D, PARTS, true, true>(qr, qc, qp);
+    rows_store<D, PARTS, true, true>(gr, gc, gp);
+    if (threadIdx.x < 2 * KT) ls[threadIdx.x] = sp;  // [0, KT) lse in base 2, [KT, 2 KT) D
+    __syncthreads();
+    if (u + 1 < units) load(u + 1);
+    const int64_t t0 = j0 + KT * (u / G);
+    if (!(wave_live && t0 + KT - 1 >= jw && t0 < w_hi)) continue;
+    // The lane's key is seen by the unit's queries lo .. hi.
+    const int lo = live ? int(max<int64_t>(j - t0, 0)) : KT, hi = live ? int(min<int64_t>(end - t0, KT)) - 1 : -1;
+    const bool whole = __all(lo == 0 && hi == KT - 1);
 #pragma unroll
-    for (int hf = 0; hf < S::QH; ++hf) act[hf] = wave_live && t0 + 16 * hf + 15 >= jw && t0 + 16 * hf < w_hi;
-    bool any = false;
+    for (int half = 0; half < 2; ++half) {
+      const int64_t tb = t0 + 32 * half;
+      if (!(tb + 31 >= jw && tb < w_hi)) continue;
+      f32x4 p[2], ds[2];
 #pragma unroll
-    for (int hf = 0; hf < S::QH; ++hf) any = any || act[hf];
-    if (any) {
-      const float *Q = qs[buf], *GO = gs[buf], *L = ls[buf];
-      f32x4 sc[S::QH], dp[S::QH], p[S::QH], ds[S::QH];
+      for (int x = 0; x < 2; ++x) {
+        const int sub = 2 * half + x;
+        f32x4 sc = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int hf = 0; hf < S::QH; ++hf) {
-        sc[hf] = f32x4{0.f, 0.f, 0.f, 0.f};
-        dp[hf] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (!act[hf]) continue;
-        float qa[S::DC], ga[S::DC];
-        lds_slice<S::DC>(Q + (16 * hf + li) * S::LD + lg * S::DC, qa);
-        lds_slice<S::DC>(GO + (16 * hf + li) * S::LD + lg * S::DC, ga);
-#pragma unroll
-        for (int kk = 0; kk < S::DC; ++kk) {
-          sc[hf] = mfma4(qa[kk], kf[kk], sc[hf]);
-          dp[hf] = mfma4(ga[kk], vf[kk], dp[hf]);
+        for (int k = 0; k < S::DK; ++k) {
+          sc = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(qr, sub, k, li, lg), kf[k], sc);
+          dp = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(gr, sub, k, li, lg), vf[k], dp);
         }
-      }
-#pragma unroll
-      for (int hf = 0; hf < S::QH; ++hf) {
-        const float4 lse4 = *reinterpret_cast<const float4 *>(L + 16 * hf + 4 * lg);
-        const float4 dsum4 = *reinterpret_cast<const float4 *>(L + S::QR + 16 * hf + 4 * lg);
-        const float lse[4] = {lse4.x, lse4.y, lse4.z, lse4.w}, dsm[4] = {dsum4.x, dsum4.y, dsum4.z, dsum4.w};
+        const f32x4 lse = *reinterpret_cast<const f32x4 *>(ls + 16 * sub + 4 * lg);
+        const f32x4 dsum = *reinterpret_cast<const f32x4 *>(ls + KT + 16 * sub + 4 * lg);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int64_t t = t0 + 16 * hf + 4 * lg + r;
-          p[hf][r] = (act[hf] && live && t >= j && t < end) ? __expf(sc[hf][r] - lse[r]) : 0.f;
-          ds[hf][r] = p[hf][r] * (dp[hf][r] - dsm[r]);
+          const int q = 16 * sub + 4 * lg + r;
+          p[x][r] = whole || (q >= lo && q <= hi) ? __builtin_amdgcn_exp2f(fmaf(sc[r], scale, -lse[r])) : 0.f;
+          ds[x][r] = p[x][r] * (dp[r] - dsum[r]);
         }
       }
+      const Operand<3> po = score_operand(p[0], p[1]), dso = score_operand(ds[0], ds[1]);
 #pragma unroll
-      for (int hf = 0; hf < S::QH; ++hf) {
-        if (!act[hf]) continue;
-#pragma unroll
-        for (int dt = 0; dt < S::DT; ++dt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            dv[dt] = mfma4(GO[(16 * hf + 4 * lg + r) * S::LD + dt * 16 + li], p[hf][r], dv[dt]);
-            dk[dt] = mfma4(Q[(16 * hf + 4 * lg + r) * S::LD + dt * 16 + li], ds[hf][r], dk[dt]);
-          }
+      for (int dt = 0; dt < S::DT; ++dt) {
+        dv[dt] = mma_parts<PARTS, 3>(col_frag<D, PARTS>(gc, half, dt, li, lg), po, dv[dt]);
+        dk[dt] = mma_parts<PARTS, 3>(col_frag<D, PARTS>(qc, half, dt, li, lg), dso, dk[dt]);
       }
     }
-    if (more) unit_store<D>(qs[buf ^ 1], gs[buf ^ 1], ls[buf ^ 1], next);
-    __syncthreads();
-    buf ^= 1;
   }
   if (!live) return;
   float *dkrow = a.dk + j * a.ldk + hk * D, *dvrow = a.dv + j * a.ldv + hk * D;
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = dt * 16 + 4 * lg + r;
-      if (d < D) {
-        dkrow[d] = attn_out(a, dk[dt][r]);
-        dvrow[d] = attn_out(a, dv[dt][r]);
-      }
+    if (dt * 16 + 4 * lg < D) {
+      store4(a, dkrow + dt * 16 + 4 * lg, dk[dt], a.scale);
+      store4(a, dvrow + dt * 16 + 4 * lg, dv[dt], 1.0f);
     }
 }
 
@@ -1194,6 +1232,63 @@ dim3 query_grid(const cg_attn_train &p) {
   return dim3(blocks_of(p.n, 16 * tpb), unsigned(p.KVH), unsigned((G + gpb - 1) / gpb));
 }
 
+// Attention launches; bf16_operands: q, k, v (and dout) hold bf16 numbers, so one part of each is
+// exact.
+void attn_fwd_launch(const cg_attn_train *p, bool bf16_operands, hipStream_t s) {
+  check_attn_train(p);
+  if (p->n == 0) return;
+  AttnTrain a{p->n, p->H, p->KVH, p->scale, p->seq_start, p->seq_of, p->q, p->k, p->v, p->ldq, p->ldk, p->ldv,
+              nullptr, nullptr, nullptr, p->o, p->lse, nullptr, nullptr, nullptr, nullptr, p->round_bf16, 1};
+  CG_REQUIRE(a.out && a.lse_out, CG_ERR_INVALID, "attention forward outputs are required");
+  CG_REQUIRE(aligned16(a.out), CG_ERR_INVALID, "attention output: 16-byte aligned");
+  const dim3 grid = query_grid(*p);
+  switch (p->head_dim) {
+#define CG_FWD_CASE(DD)                                                   \
+  case DD:                                                                \
+    if (bf16_operands) attn_fwd_kernel<DD, 1><<<grid, 256, 0, s>>>(a);    \
+    else attn_fwd_kernel<DD, 3><<<grid, 256, 0, s>>>(a);                  \
+    break;
+    CG_FWD_CASE(8)
+    CG_FWD_CASE(16)
+    CG_FWD_CASE(24)
+    CG_FWD_CASE(32)
+    CG_FWD_CASE(64)
+#undef CG_FWD_CASE
+    default: throw Error(CG_ERR_UNSUPPORTED, "training attention: head_dim 8, 16, 24, 32 or 64");
+  }
+  CG_LAUNCHED();
+}
+
+void attn_bwd_launch(const cg_attn_train *p, const float *dout, float *dsum, float *dq, float *dk, float *dv,
+                     bool bf16_operands, hipStream_t s) {
+  check_attn_train(p);
+  if (p->n == 0) return;
+  AttnTrain a{p->n, p->H, p->KVH, p->scale, p->seq_start, p->seq_of, p->q, p->k, p->v, p->ldq, p->ldk, p->ldv,
+              p->o, dout, p->lse, nullptr, nullptr, dsum, dq, dk, dv, p->round_bf16,
+              aligned16(dq) && aligned16(dk) && aligned16(dv)};
+  CG_REQUIRE(a.o && a.dout && a.lse && dsum && dq && dk && dv, CG_ERR_INVALID,
+             "attention backward operands are required");
+  CG_REQUIRE(aligned16(dout), CG_ERR_INVALID, "attention dO: 16-byte aligned");
+  const dim3 grid = query_grid(*p), grid_kv(blocks_of(p->n, 64), unsigned(p->KVH));
+  switch (p->head_dim) {
+#define CG_BWD_CASE(DD)                                                      \
+  case DD:                                                                   \
+    if (bf16_operands) attn_bwd_dq_kernel<DD, 1><<<grid, 256, 0, s>>>(a);    \
+    else attn_bwd_dq_kernel<DD, 3><<<grid, 256, 0, s>>>(a);                  \
+    CG_LAUNCHED();                                                           \
+    if (bf16_operands) attn_bwd_dkv_kernel<DD, 1><<<grid_kv, 256, 0, s>>>(a); \
+    else attn_bwd_dkv_kernel<DD, 3><<<grid_kv, 256, 0, s>>>(a);              \
+    break;
+    CG_BWD_CASE(8)
+    CG_BWD_CASE(16)
+    CG_BWD_CASE(24)
+    CG_BWD_CASE(32)
+    CG_BWD_CASE(64)
+#undef CG_BWD_CASE
+    default: throw Error(CG_ERR_UNSUPPORTED, "training attention: head_dim 8, 16, 24, 32 or 64");
+  }
+  CG_LAUNCHED();
+}
 
 }  // namespace
 }  // namespace cg
@@ -1337,56 +1432,12 @@ int cg_seq_of(const int64_t *seq_start, int32_t n_seqs, int32_t *seq_of, void *s
 }
 
 int cg_attn_train_fwd(const cg_attn_train *p, void *stream) {
-  return guarded([&] {
-    check_attn_train(p);
-    if (p->n == 0) return;
-    AttnTrain a{p->n, p->H, p->KVH, p->scale, p->seq_start, p->seq_of, p->q, p->k, p->v, p->ldq, p->ldk, p->ldv,
-                nullptr, nullptr, nullptr, p->o, p->lse, nullptr, nullptr, nullptr, nullptr, p->round_bf16};
-    CG_REQUIRE(a.out && a.lse_out, CG_ERR_INVALID, "attention forward outputs are required");
-    CG_REQUIRE(aligned16(a.out), CG_ERR_INVALID, "attention output: 16-byte aligned");
-    hipStream_t s = as_stream(stream);
-    const dim3 grid = query_grid(*p);
-    switch (p->head_dim) {
-      case 8: attn_fwd_kernel<8><<<grid, 256, 0, s>>>(a); break;
-      case 16: attn_fwd_kernel<16><<<grid, 256, 0, s>>>(a); break;
-      case 24: attn_fwd_kernel<24><<<grid, 256, 0, s>>>(a); break;
-      case 32: attn_fwd_kernel<32><<<grid, 256, 0, s>>>(a); break;
-      case 64: attn_fwd_kernel<64><<<grid, 256, 0, s>>>(a); break;
-      default: throw Error(CG_ERR_UNSUPPORTED, "training attention: head_dim 8, 16, 24, 32 or 64");
-    }
-    CG_LAUNCHED();
-  });
+  return guarded([&] { attn_fwd_launch(p, false, as_stream(stream)); });
 }
 
 int cg_attn_train_bwd(const cg_attn_train *p, const float *dout, float *dsum, float *dq, float *dk, float *dv,
                       void *stream) {
-  return guarded([&] {
-    check_attn_train(p);
-    if (p->n == 0) return;
-    AttnTrain a{p->n, p->H, p->KVH, p->scale, p->seq_start, p->seq_of, p->q, p->k, p->v, p->ldq, p->ldk, p->ldv,
-                p->o, dout, p->lse, nullptr, nullptr, dsum, dq, dk, dv, p->round_bf16};
-    CG_REQUIRE(a.o && a.dout && a.lse && dsum && dq && dk && dv, CG_ERR_INVALID,
-               "attention backward operands are required");
-    CG_REQUIRE(aligned16(dout), CG_ERR_INVALID, "attention dO: 16-byte aligned");
-    hipStream_t s = as_stream(stream);
-    const dim3 grid = query_grid(*p), grid_kv(blocks_of(p->n, 64), unsigned(p->KVH));
-    switch (p->head_dim) {
-#define CG_BWD_CASE(DD)                                  \
-  case DD:                                               \
-    attn_bwd_dq_kernel<DD><<<grid, 256, 0, s>>>(a);      \
-    CG_LAUNCHED();                                       \
-    attn_bwd_dkv_kernel<DD><<<grid_kv, 256, 0, s>>>(a);  \
-    break;
-      CG_BWD_CASE(8)
-      CG_BWD_CASE(16)
-      CG_BWD_CASE(24)
-      CG_BWD_CASE(32)
-      CG_BWD_CASE(64)
-#undef CG_BWD_CASE
-      default: throw Error(CG_ERR_UNSUPPORTED, "training attention: head_dim 8, 16, 24, 32 or 64");
-    }
-    CG_LAUNCHED();
-  });
+  return guarded([&] { attn_bwd_launch(p, dout, dsum, dq, dk, dv, false, as_stream(stream)); });
 }
 
 }  // extern "C"
@@ -1638,7 +1689,7 @@ int cg_trunk_train_forward(const cg_train_config *c, const cg_train_block *block
         }
       }
       const cg_attn_train at = attn_args(t, seq_start, tail.seq_of, a.qkv, a.o, a.lse);
-      ok(cg_attn_train_fwd(&at, st));
+      attn_fwd_launch(&at, t.bf, st);
       Epi res;  // x1 = xl + o W_out^T
       res.cin = a.xl;
       gm.nt(t.n, t.d, t.Q, a.o, w.out_w, a.x1, 1.f, res);
@@ -1711,7 +1762,7 @@ int cg_trunk_train_backward(const cg_train_config *c, const cg_train_block *bloc
       gm.tn(t.n, t.d, t.Q, s.dx1, a.o, gw.out_w);
       gm.nn(t.n, t.d, t.Q, s.dx1, w.out_w, s.dout);
       const cg_attn_train at = attn_args(t, seq_start, tail.seq_of, a.qkv, a.o, a.lse);
-      ok(cg_attn_train_bwd(&at, s.dout, s.dsum, s.dqkv, s.dqkv + t.Q, s.dqkv + t.Q + t.KVW, st));
+      attn_bwd_launch(&at, s.dout, s.dsum, s.dqkv, s.dqkv + t.Q, s.dqkv + t.Q + t.KVW, t.bf, st);
       const int32_t vi = c->value_index ? c->value_index[l] : -1;
       if (vi >= 0 && dvalues)
         ok(cg_add_strided(N, int32_t(t.KVW), 1.f, s.dqkv + t.Q + t.KVW, t.QKV, dvalues + vi * t.KVW, t.V, st));

@@ -353,3 +353,48 @@ def test_compiled_forward_hidden_packed_matches_eager(device):
             torch.testing.assert_close(compiled_g[name], eager_g[name], rtol=1e-5, atol=1e-7)
         else:
             assert torch.equal(eager_g[name], compiled_g[name]), name
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("lengths", [[16, 17, 31, 32, 33], [63, 64, 65, 1], [127, 2, 129, 200], [15, 1, 1, 1, 48, 96]])
+def test_attention_at_tile_edges(device, lengths, precision):
+    """Sequence ends around the 16-token strips, 32-row contractions and 64-row tiles; under bf16 the
+    trunk runs the one-part operands, so its gradients are compared with the three-part fp32 ones of
+    the same trunk at the bf16 bar."""
+
+    if precision == "fp32":
+        H, KVH, D, n = 8, 2, 32, sum(lengths)
+        g = torch.Generator().manual_seed(n)
+        ld = (H + 2 * KVH) * D
+        qkv = torch.randn(n, ld, generator=g, dtype=torch.float64)
+        q, k, v = (t.reshape(n, -1, D).clone().requires_grad_() for t in qkv.split([H * D, KVH * D, KVH * D], 1))
+        out = packed_attention_reference(q, k, v, lengths, H // KVH)
+        do = torch.randn(n, H, D, generator=g, dtype=torch.float64)
+        out.backward(do)
+        qkv_d, do_d = qkv.float().to(device), do.float().to(device)
+        seq_start = torch.tensor(np.concatenate([[0], np.cumsum(lengths)]), dtype=torch.int64, device=device)
+        seq_of = torch.empty(n, dtype=torch.int32, device=device)
+        stream = torch.cuda.current_stream().cuda_stream
+        nat.call("cg_seq_of", seq_start.data_ptr(), len(lengths), seq_of.data_ptr(), stream)
+        o, lse, dsum = torch.empty(n, H * D, device=device), torch.empty(n, H, device=device), torch.empty(n, H, device=device)
+        at = nat.AttnTrain(n, H, KVH, D, 1.0 / math.sqrt(D), seq_start.data_ptr(), seq_of.data_ptr(), qkv_d.data_ptr(),
+                           T._ptr(qkv_d, H * D), T._ptr(qkv_d, (H + KVH) * D), ld, ld, ld, o.data_ptr(), lse.data_ptr())
+        nat.call("cg_attn_train_fwd", ctypes.byref(at), stream)
+        close(o.view(n, H, D), out, what="o")
+        dqkv = torch.empty(n * ld + 1, device=device)[1:].view(n, ld)  # rows that are not 16-byte aligned
+        nat.call("cg_attn_train_bwd", ctypes.byref(at), do_d.data_ptr(), dsum.data_ptr(), dqkv.data_ptr(),
+                 T._ptr(dqkv, H * D), T._ptr(dqkv, (H + KVH) * D), stream)
+        for got, want, what in zip(dqkv.split([H * D, KVH * D, KVH * D], 1), (q, k, v), ("dq", "dk", "dv")):
+            close(got.reshape(want.shape), want.grad, what=what)
+        return
+    trunk = Trunk(TrunkConfig(d_model=256, n_layers=1, n_heads=8, n_kv_heads=2, d_ff=256)).to(device).train()
+    starts = np.concatenate([[0], np.cumsum(lengths)])
+    bounds = torch.from_numpy(np.repeat(np.stack([starts[:-1], starts[1:]], 1), lengths, axis=0))
+    x = torch.randn(sum(lengths), 256, generator=torch.Generator().manual_seed(1)).to(device).requires_grad_()
+    grads = []
+    for enabled in (False, True):
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=enabled):
+            hidden = trunk(x, None, None, bounds)
+        grads.append(torch.autograd.grad(hidden.square().sum(), [x, trunk.blocks[0].qkv_proj.weight]))
+    for exact, got in zip(*grads):
+        assert (got - exact).norm() <= 2e-2 * exact.norm()
