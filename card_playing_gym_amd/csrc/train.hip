@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <vector>
 
 #include "common.h"
 #include "split_tile.h"
@@ -212,9 +213,9 @@ __global__ void gemm_reduce_kernel(int32_t M, int32_t N, int32_t slices, float a
 }
 
 // Launch plan: row tile TM and split K.  A short reduction over few 128-row tiles takes
-// 64-row tiles (twice the blocks, no second pass); a long reduction into a small output (the
-// weight gradients reduce over every token) is split over k into enough (tile, slice) blocks
-// to fill the chip, and a second pass sums the slices.
+// 64-row tiles (twice the blocks, no second pass); a reduction whose tiles leave most of the chip
+// idle is split over k into enough (tile, slice) blocks to fill it, and a second pass sums the
+// slices.
 struct GemmPlan {
   int tm, slices, kc;
 };
@@ -223,13 +224,15 @@ GemmPlan gemm_plan(int32_t m, int32_t n, int32_t k, bool generic) {
   int tm = GT_M;
   if (!generic && m > 64 && tiles128 < 512 && !(k >= 1024 && tiles128 < 128)) tm = 64;
   const int64_t tiles = int64_t((m + tm - 1) / tm) * nt;
-  // Split K toward 512 blocks, but never past the 768 the chip holds at once (256 CUs x 3
-  // blocks): 408 tiles split in two would run as a full wave plus a 48-block tail, slower
-  // than the unsplit 408 tiles (13041-token packed batches hit this).
+  // Split K toward the 512 blocks that the chip holds at once (256 CUs x 2), never past them: 408
+  // tiles split in two would run as a full wave plus a tail, slower than unsplit (13041-token
+  // packed batches hit this).  A slice keeps four 32-k stages, two where the unsplit tiles would
+  // leave three CUs in four idle (256 x 256 over 792 tokens: 37 us unsplit).
+  const int stages = tiles <= 64 ? 2 : 4;
   int slices = 1;
-  if (tiles < 512 && k >= 4 * GT_K * 16) {
-    slices = int(std::min<int64_t>({(512 + tiles - 1) / tiles, 768 / tiles, k / (GT_K * 16)}));
-    slices = std::max(1, std::min(slices, 64));
+  if (tiles <= 256 && k >= 2 * stages * GT_K) {
+    slices = int(std::min<int64_t>(512 / tiles, k / (stages * GT_K)));
+    slices = std::max(1, std::min(slices, 32));
   }
   const int kc = ((k + slices - 1) / slices + GT_K - 1) / GT_K * GT_K;
   slices = (k + kc - 1) / kc;
@@ -972,7 +975,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
   char *const qr = lds, *const gr = lds + S::ROWS, *const qc = lds + 2 * S::ROWS, *const gc = qc + S::COLS;
   const int G = a.H / a.KVH, hk = blockIdx.y;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-  const int64_t j0 = int64_t(blockIdx.x) * 64, jw = j0 + 16 * wave, j = jw + li;
+  // Early keys of a sequence are seen by more queries: odd KV heads walk the key blocks backwards,
+  // so that the CU that got a long block first gets a short one next.
+  const int64_t jb = hk & 1 ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+  const int64_t j0 = jb * 64, jw = j0 + 16 * wave, j = jw + li;
   const bool live = j < a.n, wave_live = jw < a.n;
   const int64_t end = live ? a.seq_start[a.seq_of[j] + 1] : 0;
   const int64_t w_hi = wave_live ? a.seq_start[a.seq_of[min<int64_t>(a.n - 1, jw + 15)] + 1] : 0;
@@ -1070,6 +1076,36 @@ __global__ void add_strided_kernel(int32_t rows, int32_t cols, float alpha, cons
     const int c = int(i % cols);
     dst[r * ld_dst + c] += alpha * src[r * ld_src + c];
   }
+}
+
+// The per-layer embedding's update of the stream, x[r, c] += scale * ple[r, c % pd]
+// (Trunk._add_ple), and its gradient, dple[r, k] = scale * (dx[r, k] + dx[r, k + pd] + ...).
+__global__ void ple_add_kernel(int32_t rows, int32_t d, int32_t pd, float scale, const float *__restrict__ ple,
+                               int64_t ld_ple, float *__restrict__ x) {
+  const int64_t total = int64_t(rows) * d;
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t r = i / d;
+    x[i] += scale * ple[r * ld_ple + int(i % d) % pd];
+  }
+}
+__global__ void ple_grad_kernel(int32_t rows, int32_t d, int32_t pd, float scale, const float *__restrict__ dx,
+                                float *__restrict__ dple, int64_t ld_ple) {
+  const int64_t total = int64_t(rows) * pd;
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t r = i / pd;
+    const int k = int(i % pd);
+    float s = 0.f;
+    for (int c = k; c < d; c += pd) s += scale * dx[r * d + c];
+    dple[r * ld_ple + k] = s;
+  }
+}
+
+// dst[r, c] = src[r * ld_src + c].
+__global__ void copy_strided_kernel(int32_t rows, int32_t cols, const float *__restrict__ src, int64_t ld_src,
+                                    float *__restrict__ dst, int64_t ld_dst) {
+  const int64_t total = int64_t(rows) * cols;
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += int64_t(gridDim.x) * blockDim.x)
+    dst[i / cols * ld_dst + i % cols] = src[i / cols * ld_src + i % cols];
 }
 
 // Gain-only RMSNorm keeping rstd per row (one wave per row).
@@ -1604,17 +1640,8 @@ struct Gemm {
   }
 };
 
-// (column offset, width, scale) of each repeat of a per-layer embedding (trunk.py:318-333).
-template <typename F>
-void ple_slices(int64_t d, int64_t pd, F &&f) {
-  if (pd == d) {
-    f(int64_t(0), d, 1.0f);
-    return;
-  }
-  const int64_t reps = d % pd == 0 ? d / pd : (d + pd - 1) / pd;
-  const float scale = 1.0f / std::sqrt(float(reps));
-  for (int64_t r = 0; r < reps; ++r) f(r * pd, std::min(pd, d - r * pd), scale);
-}
+// Scale of each repeat of a per-layer embedding over the model width (trunk.py:318-333).
+float ple_scale(int64_t d, int64_t pd) { return pd == d ? 1.0f : 1.0f / std::sqrt(float((d + pd - 1) / pd)); }
 
 cg_attn_train attn_args(const TrainDims &t, const int64_t *seq_start, const int32_t *seq_of, const float *qkv,
                         float *o, float *lse) {
@@ -1703,10 +1730,11 @@ int cg_trunk_train_forward(const cg_train_config *c, const cg_train_block *block
       down.cin = a.x1;
       down.bias = w.down_b;
       gm.nt(t.n, t.d, t.F, a.g, w.down_w, x_next, 1.f, down);
-      if (ple)
-        ple_slices(t.d, t.pd, [&](int64_t off, int64_t width, float scale) {
-          ok(cg_add_strided(int32_t(t.n), int32_t(width), scale, ple + l * t.pd, t.P, x_next + off, t.d, st));
-        });
+      if (ple) {
+        ple_add_kernel<<<grid_1d(t.n * t.d), 256, 0, st>>>(int32_t(t.n), int32_t(t.d), int32_t(t.pd),
+                                                           ple_scale(t.d, t.pd), ple + l * t.pd, t.P, x_next);
+        CG_LAUNCHED();
+      }
     }
     ok(cg_layernorm_fwd(tail.x_last, final_w, final_b, c->eps, hidden, tail.mf, tail.rf, int32_t(t.n),
                         int32_t(t.d), st));
@@ -1732,22 +1760,30 @@ int cg_trunk_train_backward(const cg_train_config *c, const cg_train_block *bloc
     const int32_t N = int32_t(t.n);
     ok(cg_norm_bwd(tail.x_last, dhidden, final_w, tail.mf, tail.rf, s.dx, nullptr, grads->final_dw,
                    grads->final_db, N, int32_t(t.d), s.red, s.red_bytes, 0, st));
-    if (dple) {
-      zero_fill_kernel<<<grid_1d(t.n * t.P), 256, 0, st>>>(dple, t.n * t.P);
-      CG_LAUNCHED();
+    // Every layer writes its own columns of dple, and of dvalues where each slot has one layer; columns
+    // that no layer writes, or several add to, start from zero.
+    std::vector<int> users(size_t(t.V / std::max<int64_t>(t.KVW, 1)), 0);
+    bool own_slots = t.V % t.KVW == 0;
+    for (int64_t l = 0; l < t.L; ++l) {
+      const int32_t vi = c->value_index ? c->value_index[l] : -1;
+      if (vi >= 0 && size_t(vi) < users.size()) ++users[size_t(vi)];
     }
-    if (dvalues) {
-      zero_fill_kernel<<<grid_1d(t.n * t.V), 256, 0, st>>>(dvalues, t.n * t.V);
+    for (int u : users) own_slots = own_slots && u == 1;
+    auto zero = [&](float *p, int64_t cols) {
+      zero_fill_kernel<<<grid_1d(t.n * cols), 256, 0, st>>>(p, t.n * cols);
       CG_LAUNCHED();
-    }
+    };
+    if (dple && t.P != t.L * t.pd) zero(dple, t.P);
+    if (dvalues && !own_slots) zero(dvalues, t.V);
     for (int64_t l = t.L - 1; l >= 0; --l) {
       const cg_train_block &w = blocks[l];
       const cg_train_block_grads &gw = grads->blocks[l];
       const SavedLayer a = saved_layer(t, saved, l);
-      if (dple)
-        ple_slices(t.d, t.pd, [&](int64_t off, int64_t width, float scale) {
-          ok(cg_add_strided(N, int32_t(width), scale, s.dx + off, t.d, dple + l * t.pd, t.P, st));
-        });
+      if (dple) {
+        ple_grad_kernel<<<grid_1d(t.n * t.pd), 256, 0, st>>>(N, int32_t(t.d), int32_t(t.pd), ple_scale(t.d, t.pd), s.dx,
+                                                             dple + l * t.pd, t.P);
+        CG_LAUNCHED();
+      }
       gm.tn(t.n, t.d, t.F, s.dx, a.g, gw.down_w);
       column_sum_launch(s.dx, N, int32_t(t.d), t.d, gw.down_b, 0, s.red, s.red_bytes, t.bf, st);
       Epi dgelu;  // du = (dx W_down) gelu'(u)
@@ -1764,8 +1800,15 @@ int cg_trunk_train_backward(const cg_train_config *c, const cg_train_block *bloc
       const cg_attn_train at = attn_args(t, seq_start, tail.seq_of, a.qkv, a.o, a.lse);
       attn_bwd_launch(&at, s.dout, s.dsum, s.dqkv, s.dqkv + t.Q, s.dqkv + t.Q + t.KVW, t.bf, st);
       const int32_t vi = c->value_index ? c->value_index[l] : -1;
-      if (vi >= 0 && dvalues)
-        ok(cg_add_strided(N, int32_t(t.KVW), 1.f, s.dqkv + t.Q + t.KVW, t.QKV, dvalues + vi * t.KVW, t.V, st));
+      if (vi >= 0 && dvalues) {
+        const float *dv = s.dqkv + t.Q + t.KVW;
+        if (own_slots) {
+          copy_strided_kernel<<<grid_1d(t.n * t.KVW), 256, 0, st>>>(N, int32_t(t.KVW), dv, t.QKV, dvalues + vi * t.KVW, t.V);
+          CG_LAUNCHED();
+        } else {
+          ok(cg_add_strided(N, int32_t(t.KVW), 1.f, dv, t.QKV, dvalues + vi * t.KVW, t.V, st));
+        }
+      }
       gm.tn(t.n, t.QKV, t.d, s.dqkv, a.h1, gw.qkv_w);
       gm.nn(t.n, t.QKV, t.d, s.dqkv, w.qkv_w, s.dh);
       ok(cg_norm_bwd(a.xl, s.dh, w.ln_attn_w, a.m1, a.r1, s.dx, s.dx1, gw.ln_attn_w, gw.ln_attn_b, N, int32_t(t.d),
