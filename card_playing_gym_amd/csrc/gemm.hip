@@ -17,6 +17,8 @@
 // (l % 16) of a 16-column W tile, eight consecutive k values from 8 (l / 16); A and W use
 // the same lane -> k assignment, so every k is summed once (v_mfma_f32_16x16x32_bf16).
 // The 16x16 fp32 result sits in lane l as rows 4 (l / 16) + r, r < 4, column l % 16.
+#include <algorithm>
+
 #include "common.h"
 #include "gemm.h"
 #include "split_tile.h"
@@ -619,17 +621,18 @@ enum SplitTile : int { SPLIT_16 = 16, SPLIT_32 = 32, SPLIT_TILE_64 = 64, SPLIT_T
 // 32 x 32 tiles, 18.5 staged; at four per CU and k = 1024 they lead as well, 36 against 42).
 // Staged tiles are 128 rows high when that gives two per CU (16384 x 1024 x 256: 76 against
 // 84 us), else 64 (16384 x 256 x 1024: 67 against 69).
-SplitTile split_tile_of(int32_t m, int32_t n, int32_t k) {
+// (Rows too long for the staged tiles' 32-bit offsets keep the 32 x 32 ones.)
+SplitTile split_tile_of(int32_t m, int32_t n, int32_t k, int64_t lda) {
   auto tiles = [&](int64_t tm, int64_t tn) { return ((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
   if (tiles(16, 16) <= 512) return SPLIT_16;
   const int64_t t32 = tiles(32, 32);
-  if (t32 < 1024 || (t32 == 1024 && k <= 256)) return SPLIT_32;
+  if (t32 < 1024 || (t32 == 1024 && k <= 256) || std::max<int64_t>(k, lda) > TILE_MAX_STRIDE) return SPLIT_32;
   return tiles(128, 128) >= 512 ? SPLIT_TILE_128 : SPLIT_TILE_64;
 }
 
 template <int EPI, bool LN>
 void launch_split_tile(const GemmArgs &g, hipStream_t s) {
-  const SplitTile tile = split_tile_of(g.M, g.N, g.K);
+  const SplitTile tile = split_tile_of(g.M, g.N, g.K, g.lda);
   const int tn = tile >= SPLIT_TILE_64 ? ST_N : tile;
   const dim3 grid((g.N + tn - 1) / tn, (g.M + tile - 1) / tile);
   CG_REQUIRE(grid.y <= 65535u, CG_ERR_UNSUPPORTED, "too many rows for one launch");
@@ -766,7 +769,7 @@ void launch_gemm(const GemmArgs &g, hipStream_t s) {
 
 bool split_gemm_norms(int32_t m, int32_t n, int32_t k, const float *w, const float *b) {
   return k <= SPLIT_LN_K && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 &&
-         split_tile_of(m, n, k) <= SPLIT_32;
+         split_tile_of(m, n, k, k) <= SPLIT_32;
 }
 
 void launch_layernorm_rows(const float *x, const int32_t *index, const float *w, const float *b,

@@ -31,16 +31,71 @@ __device__ __forceinline__ int tile_offset(int row, int kg) {  // bytes inside o
   return (row >> 4) * 1024 + kg * 256 + (((row & 15) ^ (kg * 4)) << 4);
 }
 
-// Loads go to clamped, always valid addresses with no branches, so that a stage's loads fly at
-// once; rows >= rows_left are never stored by the caller and k >= k_left is zeroed at the LDS
-// write.
+// A thread's place in a tile: byte offsets from the tile's first row at a stage's first k (32 bits
+// beside a uniform pointer, so a load costs no vector address arithmetic).  MODE 1: one per
+// 64 rows; MODE 2: one, its eight k a uniform stride apart.
+template <int MODE, int ROWS>
+struct TilePlace {
+  unsigned at[ROWS / 64];
+};
+template <int MODE, int ROWS>
+__device__ __forceinline__ TilePlace<MODE, ROWS> tile_place(int64_t sr, int64_t sk, int rows_left, int tid) {
+  TilePlace<MODE, ROWS> t{};
+  if constexpr (MODE == 2) {
+    constexpr int W = ROWS / 64;  // consecutive rows per thread
+    const int row = W * (tid & 63);
+    t.at[0] = 4u * (unsigned(8 * (tid >> 6)) * unsigned(sk) +
+                    unsigned(W == 2 ? max(0, min(row, rows_left - 2)) : min(row, rows_left - 1)));
+  } else if constexpr (MODE == 1) {
+#pragma unroll
+    for (int e = 0; e < ROWS / 64; ++e)
+      t.at[e] = 4u * (unsigned(min((tid + e * 256) >> 2, rows_left - 1)) * unsigned(sr) + unsigned(8 * (tid & 3)));
+  }
+  return t;
+}
+
+// A whole stage (p at its first k): rows past the tile's are read from its last row and their
+// results never stored.
 template <int MODE, int ROWS, int NK>
-__device__ __forceinline__ void tile_load(TileRegs<MODE, ROWS, NK> &t, const float *__restrict__ p, int64_t sr,
-                                          int64_t sk, int rows_left, int k_left, int tid) {
+__device__ __forceinline__ void tile_load(TileRegs<MODE, ROWS, NK> &t, const TilePlace<MODE, ROWS> &place,
+                                          const float *__restrict__ p, int64_t sk) {
+  auto at = [](const float *q, unsigned bytes) { return reinterpret_cast<const char *>(q) + bytes; };
 #pragma unroll
   for (int s = 0; s < NK; ++s) {
     if constexpr (MODE == 2) {
-      constexpr int W = ROWS / 64;  // consecutive rows per thread
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const char *q = at(p + int64_t(32 * s + i) * sk, place.at[0]);
+        if constexpr (ROWS == 128) {
+          const split_f32x2 x = *reinterpret_cast<const split_f32x2 *>(q);
+          t.v[(s * 2 + 0) * 8 + i] = x[0];
+          t.v[(s * 2 + 1) * 8 + i] = x[1];
+        } else {
+          t.v[s * 8 + i] = *reinterpret_cast<const float *>(q);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < ROWS / 64; ++e) {
+        const char *q = at(p + 32 * s, place.at[e]);
+        const split_f32x4 x = *reinterpret_cast<const split_f32x4 *>(q), y = *reinterpret_cast<const split_f32x4 *>(q + 16);
+        float *o = t.v + (s * (ROWS / 64) + e) * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = x[i], o[4 + i] = y[i];
+      }
+    }
+  }
+}
+
+// The last stage of a ragged k, and every stage of MODE 0: clamped, always valid addresses with
+// no branches; k >= k_left is zeroed at the LDS write.
+template <int MODE, int ROWS, int NK>
+__device__ __forceinline__ void tile_load_tail(TileRegs<MODE, ROWS, NK> &t, const float *__restrict__ p, int64_t sr,
+                                               int64_t sk, int rows_left, int k_left, int tid) {
+#pragma unroll
+  for (int s = 0; s < NK; ++s) {
+    if constexpr (MODE == 2) {
+      constexpr int W = ROWS / 64;
       const int row = W * (tid & 63), kg = tid >> 6;
       const int rc = W == 2 ? max(0, min(row, rows_left - 2)) : min(row, rows_left - 1);
 #pragma unroll
@@ -73,6 +128,9 @@ __device__ __forceinline__ void tile_load(TileRegs<MODE, ROWS, NK> &t, const flo
     }
   }
 }
+
+// The largest row stride (MODE 1) or k stride (MODE 2) whose offsets inside a tile fit 32 bits.
+constexpr int64_t TILE_MAX_STRIDE = int64_t(1) << 22;
 
 // Converts the stage's values and writes them to `lds`: part p of k step s at byte
 // (s PLANES + p) plane.  TAIL: k >= k_left is zeroed (the last stage of a ragged k).
@@ -144,10 +202,17 @@ __device__ __forceinline__ void tile_product(const float *__restrict__ a, int64_
   TileRegs<AM, TM, NK> ra;
   TileRegs<BM, ST_N, NK> rb;
   const int last = kbeg + (kend - kbeg - 1) / KS * KS;  // first k of the last stage
+  const TilePlace<AM, TM> pa = tile_place<AM, TM>(sam, sak, ma, tid);
+  const TilePlace<BM, ST_N> pb = tile_place<BM, ST_N>(sbn, sbk, nb, tid);
   auto load = [&](int k0) {
     k0 = min(k0, last);
-    tile_load<AM, TM, NK>(ra, a + int64_t(k0) * sak, sam, sak, ma, kend - k0, tid);
-    tile_load<BM, ST_N, NK>(rb, b + int64_t(k0) * sbk, sbn, sbk, nb, kend - k0, tid);
+    if (AM != 0 && k0 + KS <= kend) {
+      tile_load<AM, TM, NK>(ra, pa, a + int64_t(k0) * sak, sak);
+      tile_load<BM, ST_N, NK>(rb, pb, b + int64_t(k0) * sbk, sbk);
+    } else {
+      tile_load_tail<AM, TM, NK>(ra, a + int64_t(k0) * sak, sam, sak, ma, kend - k0, tid);
+      tile_load_tail<BM, ST_N, NK>(rb, b + int64_t(k0) * sbk, sbn, sbk, nb, kend - k0, tid);
+    }
   };
   auto store = [&](auto tail, char *to, int k_left) {
     tile_store<AM, TM, NK, PLANES, decltype(tail)::value>(to, PLANE, ra, k_left, tid);

@@ -147,41 +147,64 @@ __global__ __launch_bounds__(256, 2) void gemm_strided_kernel(int32_t M, int32_t
         }
     return;
   }
-  // Epilogue: every operand it reads (prior C or cin, bias, aux_in) is loaded for a whole
-  // 16-row block at once from clamped, always valid addresses, and unused values are dropped by
-  // selects, so the loads overlap instead of waiting one by one behind per-element branches.
-  const bool prior = beta != 0.f, fwd_gelu = epi.mode == EPI_GELU;
-  const float *pin = epi.cin ? epi.cin : C, *ain = epi.mode == EPI_GELU_GRAD ? epi.aux_in : C;
+  // Epilogue, a 16-row block at a time: every operand it reads (prior C or cin, bias, aux_in; only
+  // those this product has) is loaded at once, from addresses a uniform pointer plus 32 bits per
+  // lane; tiles that hang over an edge clamp them.
+  const bool prior = beta != 0.f, grad = epi.mode == EPI_GELU_GRAD, fwd_gelu = epi.mode == EPI_GELU;
+  const float *pin = epi.cin ? epi.cin : C;
   float bj[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int n = min(n0 + wn * 64 + j * 16 + li, N - 1);
     bj[j] = epi.bias ? epi.bias[n] : 0.f;
   }
+  const bool inside = m0 + TM <= M && n0 + GT_N <= N && ldc <= TILE_MAX_STRIDE;
+  auto finish = [&](auto whole) {
+    constexpr bool WHOLE = decltype(whole)::value;
 #pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    float pv[4][4], av[4][4];
+    for (int i = 0; i < FM; ++i) {
+      const int64_t base = int64_t(m0 + i * 16) * ldc + n0;
+      unsigned at[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t m = min(m0 + wm * (TM / 2) + i * 16 + 4 * lg + r, M - 1), n = min(n0 + wn * 64 + j * 16 + li, N - 1);
-        pv[j][r] = pin[m * ldc + n];
-        av[j][r] = ain[m * ldc + n];
-      }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm * (TM / 2) + i * 16 + 4 * lg + r, n = n0 + wn * 64 + j * 16 + li;
-        const float v = epi_value(epi, alpha * acc[i][j][r], beta, prior ? pv[j][r] : 0.f, bj[j], av[j][r]);
-        if (m < M && n < N) {
-          const int64_t o = int64_t(m) * ldc + n;
-          C[o] = v;
-          if (fwd_gelu) epi.aux_out[o] = epi.round ? round_bf16(gelu_exact(v)) : gelu_exact(v);
+      for (int r = 0; r < 4; ++r) at[r] = 4u * (unsigned(wm * (TM / 2) + 4 * lg + r) * unsigned(ldc) + unsigned(wn * 64 + li));
+      auto place = [&](auto *p, int j, int r) {
+        using T = std::remove_pointer_t<decltype(p)>;
+        if constexpr (WHOLE) {
+          using B = std::conditional_t<std::is_const_v<T>, const char, char>;
+          return reinterpret_cast<T *>(reinterpret_cast<B *>(p + base + 16 * j) + at[r]);
+        } else {
+          const int64_t m = min(m0 + wm * (TM / 2) + i * 16 + 4 * lg + r, M - 1), n = min(n0 + wn * 64 + j * 16 + li, N - 1);
+          return p + m * ldc + n;
         }
+      };
+      float pv[4][4], av[4][4];
+      if (prior) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pv[j][r] = *place(pin, j, r);
       }
-  }
+      if (grad) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) av[j][r] = *place(epi.aux_in, j, r);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + wm * (TM / 2) + i * 16 + 4 * lg + r, n = n0 + wn * 64 + j * 16 + li;
+          const float v = epi_value(epi, alpha * acc[i][j][r], beta, prior ? pv[j][r] : 0.f, bj[j], grad ? av[j][r] : 0.f);
+          if (WHOLE || (m < M && n < N)) {
+            *place(C, j, r) = v;
+            if (fwd_gelu) *place(epi.aux_out, j, r) = epi.round ? round_bf16(gelu_exact(v)) : gelu_exact(v);
+          }
+        }
+    }
+  };
+  if (inside) finish(std::true_type{});
+  else finish(std::false_type{});
 }
 
 // C[m, n] = epilogue(alpha * sum_z part[z][m, n]).  A thread takes four consecutive entries
@@ -636,21 +659,24 @@ __device__ __forceinline__ void clear_lds(char *lds, int bytes) {
   for (int i = threadIdx.x * 16; i < bytes; i += 256 * 16) *reinterpret_cast<split_u32x4 *>(lds + i) = split_u32x4{0, 0, 0, 0};
 }
 
-// Rows [r0, r0 + 64) of p (row stride ld floats, D used columns) into registers; rows outside
-// [0, last] read 0.
+// Rows [r0, r0 + 64) of p (row stride ld floats, D used columns) into registers; rows past `last` are
+// read as the last (their scores are masked).  The row base is uniform, the rest 32 bits.
 template <int D, int PARTS>
-__device__ __forceinline__ void rows_load(SlotRegs<D, PARTS> &r, const float *__restrict__ p, int64_t ld,
-                                          int64_t r0, int64_t last) {
+__device__ __forceinline__ void rows_load(SlotRegs<D, PARTS> &r, const float *__restrict__ p, int64_t ld, int64_t r0,
+                                          int64_t last) {
   using S = AttnDims<D, PARTS>;
+  const char *base = reinterpret_cast<const char *>(p + r0 * ld);  // (strides are not negative)
+  const int left = int(min<int64_t>(last - r0, KT - 1));
 #pragma unroll
   for (int e = 0; e < S::PER; ++e) {
-    const int slot = threadIdx.x + 256 * e, c = (slot % S::C4) * 4;
+    const int slot = min(int(threadIdx.x) + 256 * e, S::SLOTS - 1), row = 2 * (slot / S::C4), c = (slot % S::C4) * 4;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int64_t row = r0 + 2 * (slot / S::C4) + h;
-      const bool in = slot < S::SLOTS && row <= last;
-      const float4 v = *reinterpret_cast<const float4 *>(p + (in ? row * ld + c : 0));
-      r[e][h] = in ? v : float4{0.f, 0.f, 0.f, 0.f};
+      const int at = min(row + h, left);
+      if (ld <= TILE_MAX_STRIDE)
+        r[e][h] = *reinterpret_cast<const float4 *>(base + 4u * (unsigned(at) * unsigned(ld) + unsigned(c)));
+      else
+        r[e][h] = *reinterpret_cast<const float4 *>(base + 4 * (at * ld + c));
     }
   }
 }
@@ -729,8 +755,8 @@ __device__ __forceinline__ Operand<PARTS> col_frag(const char *cols, int u, int 
 
 // A lane's eight d of one row (d = 32 dk + 8 lg ..) as a B operand; zero when !live or past D.
 template <int D, int PARTS>
-__device__ __forceinline__ void row_operand(DimOperand<D, PARTS> &o, const float *__restrict__ p,
-                                            bool live, int lg) {
+__device__ __forceinline__ void row_operand(DimOperand<D, PARTS> &o, const float *__restrict__ p, bool live, int lg,
+                                            float scale = 1.0f) {
 #pragma unroll
   for (int dk = 0; dk < AttnDims<D, PARTS>::DK; ++dk) {
     float v[8];
@@ -738,7 +764,7 @@ __device__ __forceinline__ void row_operand(DimOperand<D, PARTS> &o, const float
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const float4 x = live && d < D ? *reinterpret_cast<const float4 *>(p + d + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
-      v[4 * h] = x.x, v[4 * h + 1] = x.y, v[4 * h + 2] = x.z, v[4 * h + 3] = x.w;
+      v[4 * h] = x.x * scale, v[4 * h + 1] = x.y * scale, v[4 * h + 2] = x.z * scale, v[4 * h + 3] = x.w * scale;
     }
     o[dk] = operand_of<PARTS>(v);
   }
@@ -806,8 +832,8 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnTrain a) {
   const int64_t k_lo = a.seq_start[a.seq_of[w.base]];
   const float scale = a.scale * LOG2E;
   clear_lds(lds, S::ROWS + S::COLS);
-  Operand<PARTS> qf[S::DK];
-  row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg);
+  Operand<PARTS> qf[S::DK];  // (scaling bf16 queries would take more than one part)
+  row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg, PARTS == 3 ? scale : 1.0f);
   f32x4 acc[S::DT];
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -827,7 +853,8 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnTrain a) {
     if (!(w.active && j0 <= w_last && j0 + KT - 1 >= w_first)) continue;
     // The lane's query sees the tile's keys lo .. hi.
     const int lo = live ? int(max<int64_t>(start - j0, 0)) : KT, hi = live ? int(min<int64_t>(t - j0, KT - 1)) : -1;
-    const bool whole = __all(lo == 0 && hi == KT - 1);
+    const unsigned seen = unsigned(max(hi - lo + 1, 0));
+    const bool whole = __all(seen == KT);
     f32x4 s[4];
     bool any[4];
     float mt = -INFINITY;
@@ -840,12 +867,12 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnTrain a) {
       f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int dk = 0; dk < S::DK; ++dk) c = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(kr, sub, dk, li, lg), qf[dk], c);
+      s[sub] = PARTS == 3 ? c : c * scale;
+      if (!whole) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kk = 16 * sub + 4 * lg + r;
-        s[sub][r] = whole || (kk >= lo && kk <= hi) ? c[r] * scale : -INFINITY;
-        mt = fmaxf(mt, s[sub][r]);
+        for (int r = 0; r < 4; ++r) s[sub][r] = unsigned(4 * lg - lo + 16 * sub + r) < seen ? s[sub][r] : -INFINITY;
       }
+      mt = fmaxf(fmaxf(mt, fmaxf(s[sub][0], s[sub][1])), fmaxf(s[sub][2], s[sub][3]));
     }
     mt = max_over_rows(mt);
     const float mn = fmaxf(m, mt);
@@ -928,7 +955,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const AttnTrain a) {
     }
     if (!(w.active && j0 <= w_last && j0 + KT - 1 >= w_first)) continue;
     const int lo = live ? int(max<int64_t>(start - j0, 0)) : KT, hi = live ? int(min<int64_t>(t - j0, KT - 1)) : -1;
-    const bool whole = __all(lo == 0 && hi == KT - 1);
+    const unsigned seen = unsigned(max(hi - lo + 1, 0));
+    const bool whole = __all(seen == KT);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int64_t jb = j0 + 32 * u;
@@ -943,12 +971,15 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const AttnTrain a) {
           st = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(kr, sub, dk, li, lg), qf[dk], st);
           dp = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(vr, sub, dk, li, lg), gf[dk], dp);
         }
+        f32x4 p;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int kk = 16 * sub + 4 * lg + r;
-          const float p = whole || (kk >= lo && kk <= hi) ? __builtin_amdgcn_exp2f(fmaf(st[r], scale, -lse)) : 0.f;
-          ds[h][r] = p * (dp[r] - dsum);
+        for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(st[r], scale, -lse));
+        if (!whole) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) p[r] = unsigned(4 * lg - lo + 16 * sub + r) < seen ? p[r] : 0.f;
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ds[h][r] = p[r] * (dp[r] - dsum);
       }
       const Operand<3> dso = score_operand(ds[0], ds[1]);
 #pragma unroll
@@ -1018,7 +1049,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
     if (!(wave_live && t0 + KT - 1 >= jw && t0 < w_hi)) continue;
     // The lane's key is seen by the unit's queries lo .. hi.
     const int lo = live ? int(max<int64_t>(j - t0, 0)) : KT, hi = live ? int(min<int64_t>(end - t0, KT)) - 1 : -1;
-    const bool whole = __all(lo == 0 && hi == KT - 1);
+    const unsigned seen = unsigned(max(hi - lo + 1, 0));
+    const bool whole = __all(seen == KT);
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int64_t tb = t0 + 32 * half;
@@ -1036,11 +1068,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
         const f32x4 lse = *reinterpret_cast<const f32x4 *>(ls + 16 * sub + 4 * lg);
         const f32x4 dsum = *reinterpret_cast<const f32x4 *>(ls + KT + 16 * sub + 4 * lg);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int q = 16 * sub + 4 * lg + r;
-          p[x][r] = whole || (q >= lo && q <= hi) ? __builtin_amdgcn_exp2f(fmaf(sc[r], scale, -lse[r])) : 0.f;
-          ds[x][r] = p[x][r] * (dp[r] - dsum[r]);
+        for (int r = 0; r < 4; ++r) p[x][r] = __builtin_amdgcn_exp2f(fmaf(sc[r], scale, -lse[r]));
+        if (!whole) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) p[x][r] = unsigned(4 * lg - lo + 16 * sub + r) < seen ? p[x][r] : 0.f;
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ds[x][r] = p[x][r] * (dp[r] - dsum[r]);
       }
       const Operand<3> po = score_operand(p[0], p[1]), dso = score_operand(ds[0], ds[1]);
 #pragma unroll
@@ -1142,15 +1176,15 @@ void check_attn_train(const cg_attn_train *p) {
   CG_REQUIRE(p->q && p->k && p->v && p->seq_start && p->seq_of, CG_ERR_INVALID,
              "attention q, k, v, seq_start and seq_of are required");
   CG_REQUIRE(aligned16(p->q) && aligned16(p->k) && aligned16(p->v) && p->ldq % 4 == 0 && p->ldk % 4 == 0 &&
-                 p->ldv % 4 == 0,
+                 p->ldv % 4 == 0 && p->ldq >= 0 && p->ldk >= 0 && p->ldv >= 0,
              CG_ERR_INVALID, "attention q / k / v: 16-byte aligned rows (pointers and row strides)");
 }
 
 // Operand mode (rows, k) of a GEMM input: 1 k contiguous, 2 rows contiguous, 0 any strides.
 int operand_mode(const float *p, int64_t sr, int64_t sk, int32_t rows, int32_t kk) {
   if (!aligned16(p)) return 0;
-  if (sk == 1 && sr % 4 == 0 && kk % 4 == 0) return 1;
-  if (sr == 1 && sk % 4 == 0 && rows % 4 == 0) return 2;
+  if (sk == 1 && sr % 4 == 0 && kk % 4 == 0 && sr >= 0 && sr <= TILE_MAX_STRIDE) return 1;
+  if (sr == 1 && sk % 4 == 0 && rows % 4 == 0 && sk >= 0 && sk <= TILE_MAX_STRIDE) return 2;
   return 0;
 }
 
