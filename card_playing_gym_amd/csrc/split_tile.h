@@ -134,8 +134,10 @@ constexpr int64_t TILE_MAX_STRIDE = int64_t(1) << 22;
 
 // Converts the stage's values and writes them to `lds`: part p of k step s at byte
 // (s PLANES + p) plane.  TAIL: k >= k_left is zeroed (the last stage of a ragged k).
+// `sums` (one per row of the thread, or NULL) receives the values as multiplied.
 template <int MODE, int ROWS, int NK, int PLANES, bool TAIL>
-__device__ __forceinline__ void tile_store(char *lds, int plane, const TileRegs<MODE, ROWS, NK> &t, int k_left, int tid) {
+__device__ __forceinline__ void tile_store(char *lds, int plane, const TileRegs<MODE, ROWS, NK> &t, int k_left, int tid,
+                                           float *sums = nullptr) {
 #pragma unroll
   for (int s = 0; s < NK; ++s)
 #pragma unroll
@@ -162,9 +164,15 @@ __device__ __forceinline__ void tile_store(char *lds, int plane, const TileRegs<
         *reinterpret_cast<split_u32x4 *>(o) = p.hi;
         *reinterpret_cast<split_u32x4 *>(o + plane) = p.mid;
         *reinterpret_cast<split_u32x4 *>(o + 2 * plane) = p.lo;
+        if (sums) sums[e] += ((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]));
       } else {
-        *reinterpret_cast<split_u32x4 *>(o) = split_u32x4{split_pack(x[0], x[1]), split_pack(x[2], x[3]),
-                                                          split_pack(y[0], y[1]), split_pack(y[2], y[3])};
+        const split_u32x4 p = {split_pack(x[0], x[1]), split_pack(x[2], x[3]), split_pack(y[0], y[1]),
+                               split_pack(y[2], y[3])};
+        *reinterpret_cast<split_u32x4 *>(o) = p;
+        if (sums) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sums[e] += __uint_as_float(p[i] << 16) + __uint_as_float(p[i] & 0xffff0000u);
+        }
       }
     }
 }
@@ -183,10 +191,12 @@ constexpr int tile_lds_bytes() {
 // acc[i][j] = the wave's 16 x 16 tiles of A[m0 .., kbeg .. kend) B: lane (li, lg) holds rows
 // 16 i + 4 lg + r, column 16 j + li of the wave's TM / 2 x 64 part.  a / b point at the tile's
 // first row and column; ma / nb are the rows and columns left there.  All 256 threads call it.
-template <int AM, int BM, int TM, int PLANES, int NK>
+// With SUMS and `row_sums` set, row_sums[r] = sum over k of A's row r as it was multiplied (r < ma).
+template <int AM, int BM, int TM, int PLANES, int NK, bool SUMS = false>
 __device__ __forceinline__ void tile_product(const float *__restrict__ a, int64_t sam, int64_t sak, int ma,
                                              const float *__restrict__ b, int64_t sbk, int64_t sbn, int nb, int kbeg,
-                                             int kend, char *lds, split_f32x4 (&acc)[TM / 32][4]) {
+                                             int kend, char *lds, split_f32x4 (&acc)[TM / 32][4],
+                                             float *__restrict__ row_sums = nullptr) {
   constexpr int FM = TM / 32, KS = 32 * NK;
   constexpr int PLANE = (TM + ST_N) * 64;  // bytes of one part of one 32-k step, A rows then B rows
   constexpr int STAGE = PLANE * PLANES * NK;
@@ -198,7 +208,8 @@ __device__ __forceinline__ void tile_product(const float *__restrict__ a, int64_
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = cor[i][j] = split_f32x4{0.f, 0.f, 0.f, 0.f};
-  if (kbeg >= kend) return;
+  if (kbeg >= kend) return;  // (never with SUMS: slices are not empty)
+  float sums[TM / 64] = {};
   TileRegs<AM, TM, NK> ra;
   TileRegs<BM, ST_N, NK> rb;
   const int last = kbeg + (kend - kbeg - 1) / KS * KS;  // first k of the last stage
@@ -215,7 +226,12 @@ __device__ __forceinline__ void tile_product(const float *__restrict__ a, int64_
     }
   };
   auto store = [&](auto tail, char *to, int k_left) {
-    tile_store<AM, TM, NK, PLANES, decltype(tail)::value>(to, PLANE, ra, k_left, tid);
+    if constexpr (SUMS) {
+      if (row_sums) tile_store<AM, TM, NK, PLANES, decltype(tail)::value>(to, PLANE, ra, k_left, tid, sums);
+      else tile_store<AM, TM, NK, PLANES, decltype(tail)::value>(to, PLANE, ra, k_left, tid);
+    } else {
+      tile_store<AM, TM, NK, PLANES, decltype(tail)::value>(to, PLANE, ra, k_left, tid);
+    }
     tile_store<BM, ST_N, NK, PLANES, decltype(tail)::value>(to + TM * 64, PLANE, rb, k_left, tid);
   };
   auto multiply = [&](const char *from) {
@@ -281,6 +297,26 @@ __device__ __forceinline__ void tile_product(const float *__restrict__ a, int64_
     nxt = t;
   }
   multiply(cur);
+  if constexpr (SUMS) {
+    if (row_sums) {  // a row's four k groups meet: four lanes (MODE 0, 1) or four waves (MODE 2)
+      if constexpr (AM == 2) {
+        __syncthreads();
+        float *meet = reinterpret_cast<float *>(lds);  // [4][TM]
+#pragma unroll
+        for (int e = 0; e < TM / 64; ++e) meet[wave * TM + (TM / 64) * lane + e] = sums[e];
+        __syncthreads();
+        if (tid < TM && tid < ma) row_sums[tid] = (meet[tid] + meet[TM + tid]) + (meet[2 * TM + tid] + meet[3 * TM + tid]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < TM / 64; ++e) {
+          float v = sums[e] + __shfl_xor(sums[e], 1);
+          v += __shfl_xor(v, 2);
+          const int row = (tid + e * 256) >> 2;
+          if ((tid & 3) == 0 && row < ma) row_sums[row] = v;
+        }
+      }
+    }
+  }
   if constexpr (PLANES == 3) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)

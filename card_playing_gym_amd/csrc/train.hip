@@ -74,6 +74,8 @@ struct Epi {
   const float *cin = nullptr;
   const float *aux_in = nullptr;
   float *aux_out = nullptr;
+  float *row_sum = nullptr;  // [M]: also the sums of A's rows over k (a weight gradient's bias gradient;
+                             // under `round` of the rounded operands, rounded)
   int32_t mode = EPI_PLAIN;
   int32_t round = 0;  // bf16 operands (the GEMM rounds them as it stages) and bf16 outputs
 };
@@ -106,7 +108,7 @@ __device__ __forceinline__ void epilogue(const Epi &e, float v, float beta, floa
 // them.
 constexpr int GT_M = 128, GT_N = ST_N, GT_K = 32;
 
-template <int AM, int BM, int TM, bool BF>
+template <int AM, int BM, int TM, bool BF, bool SUMS>
 __global__ __launch_bounds__(256, 2) void gemm_strided_kernel(int32_t M, int32_t N, int32_t K, int32_t kc, float alpha,
                                                            const float *__restrict__ A, int64_t sam, int64_t sak,
                                                            const float *__restrict__ B, int64_t sbk, int64_t sbn,
@@ -130,8 +132,17 @@ __global__ __launch_bounds__(256, 2) void gemm_strided_kernel(int32_t M, int32_t
   const int m0 = mt * TM, n0 = nt * GT_N;
   const int kbeg = blockIdx.z * kc, kend = min(K, kbeg + kc);
   f32x4 acc[FM][4];
-  tile_product<AM, BM, TM, PLANES, NK>(A + int64_t(m0) * sam, sam, sak, M - m0, B + int64_t(n0) * sbn, sbk, sbn, N - n0,
-                                       kbeg, kend, lds, acc);
+  // Row sums: the first column of tiles leaves them beside its slice's partial products.
+  float *sums = nullptr;
+  if constexpr (SUMS)
+    if (nt == 0) sums = part ? part + int64_t(gridDim.z) * M * N + int64_t(blockIdx.z) * M + m0 : epi.row_sum + m0;
+  tile_product<AM, BM, TM, PLANES, NK, SUMS>(A + int64_t(m0) * sam, sam, sak, M - m0, B + int64_t(n0) * sbn, sbk, sbn,
+                                             N - n0, kbeg, kend, lds, acc, sums);
+  if constexpr (SUMS && BF)
+    if (sums && !part) {  // the sums' own threads wrote them
+      __syncthreads();
+      if (int(threadIdx.x) < min(TM, M - m0)) sums[threadIdx.x] = round_bf16(sums[threadIdx.x]);
+    }
   if constexpr (!BF)
     tile_repair<FM>(acc, A + int64_t(kbeg) * sak, sam, sak, B + int64_t(kbeg) * sbk, sbk, sbn, m0 + wm * (TM / 2),
                     n0 + wn * 64, M, N, kend - kbeg);
@@ -213,6 +224,14 @@ __global__ void gemm_reduce_kernel(int32_t M, int32_t N, int32_t slices, float a
                                    float beta, float *__restrict__ C, int64_t ldc, const Epi epi) {
   const int64_t total = int64_t(M) * N, quads = (total + 3) / 4;
   const bool vec = (N & 3) == 0;
+  if (epi.row_sum) {
+    const float *sums = part + int64_t(slices) * total;
+    for (int m = blockIdx.x * blockDim.x + threadIdx.x; m < M; m += gridDim.x * blockDim.x) {
+      float v = 0.f;
+      for (int z = 0; z < slices; ++z) v += sums[int64_t(z) * M + m];
+      epi.row_sum[m] = epi.round ? round_bf16(v) : v;
+    }
+  }
   for (int64_t q = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; q < quads; q += int64_t(gridDim.x) * blockDim.x) {
     const int64_t i0 = 4 * q;
     f32x4 s[4] = {};
@@ -515,7 +534,7 @@ __global__ __launch_bounds__(1024) void norm_params_kernel(const float *__restri
 // chunk lands in out[y][c] (a second pass sums the chunks).
 __global__ __launch_bounds__(256) void column_sum_kernel(const float *__restrict__ in, int32_t rows, int32_t cols,
                                                          int64_t ld, float *__restrict__ out, int32_t accumulate,
-                                                         int32_t chunk, int32_t round_in, int32_t round_out) {
+                                                         int32_t chunk) {
   __shared__ float red[4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = blockIdx.x * 64 + lane;
@@ -523,10 +542,7 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const float *__restrict
   float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
   if (c < cols) {
     int r = r0 + wave;
-    auto at = [&](int rr) {
-      const float v = in[int64_t(rr) * ld + c];
-      return round_in ? round_bf16(v) : v;
-    };
+    auto at = [&](int rr) { return in[int64_t(rr) * ld + c]; };
     for (; r + 12 < r1; r += 16) {
       s0 += at(r);
       s1 += at(r + 4);
@@ -539,7 +555,6 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const float *__restrict
   __syncthreads();
   if (wave == 0 && c < cols) {
     float s = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
-    if (round_out) s = round_bf16(s);
     float *o = out + int64_t(blockIdx.y) * cols + c;
     *o = accumulate ? *o + s : s;
   }
@@ -1188,6 +1203,9 @@ int operand_mode(const float *p, int64_t sr, int64_t sk, int32_t rows, int32_t k
   return 0;
 }
 
+// A split product's partial results and partial row sums.
+size_t slice_bytes(const GemmPlan &pl, int32_t m, int32_t n) { return size_t(pl.slices) * size_t(m) * (size_t(n) + 1) * 4; }
+
 GemmPlan plan_of(int32_t m, int32_t n, int32_t k, const float *a, int64_t sam, int64_t sak, const float *b,
                  int64_t sbk, int64_t sbn, int *am, int *bm) {
   *am = operand_mode(a, sam, sak, m, k);
@@ -1206,7 +1224,8 @@ void gemm_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, i
              "GEMM epilogue: GELU needs its second output, GELU' its pre-activation");
   int am, bm;
   const GemmPlan pl = plan_of(m, n, k, a, sam, sak, b, sbk, sbn, &am, &bm);
-  const size_t need = pl.slices > 1 ? size_t(pl.slices) * size_t(m) * size_t(n) * 4 : 0;
+  const size_t need = pl.slices > 1 ? slice_bytes(pl, m, n) : 0;
+  CG_REQUIRE(k > 0 || !epi.row_sum, CG_ERR_INVALID, "GEMM: row sums of an empty product");
   CG_REQUIRE(need == 0 || (workspace && workspace_size >= need), CG_ERR_INVALID,
              "GEMM: workspace too small, need " + std::to_string(need) + " bytes");
   const dim3 grid(unsigned((n + GT_N - 1) / GT_N), unsigned((m + pl.tm - 1) / pl.tm), unsigned(pl.slices));
@@ -1214,15 +1233,20 @@ void gemm_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, i
   hipStream_t s = as_stream(stream);
   float *part = pl.slices > 1 ? static_cast<float *>(workspace) : nullptr;
   const int32_t kc = pl.kc;
-  const bool bf = epi.round != 0;
-#define CG_GEMM_CASE(A_, B_, T_)                                                                                 \
-  if (am == A_ && bm == B_ && pl.tm == T_) {                                                                     \
-    if (bf)                                                                                                      \
-      gemm_strided_kernel<A_, B_, T_, true><<<grid, 256, 0, s>>>(m, n, k, kc, alpha, a, sam, sak, b, sbk, sbn, beta, \
-                                                                 c, ldc, part, epi);                             \
-    else                                                                                                         \
-      gemm_strided_kernel<A_, B_, T_, false><<<grid, 256, 0, s>>>(m, n, k, kc, alpha, a, sam, sak, b, sbk, sbn,    \
-                                                                  beta, c, ldc, part, epi);                      \
+  const bool bf = epi.round != 0, sums = epi.row_sum != nullptr;
+  CG_REQUIRE(!sums || (am == 2 && bm == 2) || (am == 0 && bm == 0), CG_ERR_UNSUPPORTED, "GEMM: row sums of this layout");
+#define CG_GEMM_RUN(A_, B_, T_, BF_, S_)                                                                        \
+  gemm_strided_kernel<A_, B_, T_, BF_, S_><<<grid, 256, 0, s>>>(m, n, k, kc, alpha, a, sam, sak, b, sbk, sbn, beta, c, \
+                                                                ldc, part, epi)
+#define CG_GEMM_CASE(A_, B_, T_)                     \
+  if (!sums && am == A_ && bm == B_ && pl.tm == T_) { \
+    if (bf) CG_GEMM_RUN(A_, B_, T_, true, false);    \
+    else CG_GEMM_RUN(A_, B_, T_, false, false);      \
+  }
+#define CG_GEMM_SUMS(A_, B_, T_)                    \
+  if (sums && am == A_ && bm == B_ && pl.tm == T_) { \
+    if (bf) CG_GEMM_RUN(A_, B_, T_, true, true);    \
+    else CG_GEMM_RUN(A_, B_, T_, false, true);      \
   }
   CG_GEMM_CASE(1, 1, 128)
   CG_GEMM_CASE(1, 2, 128)
@@ -1233,6 +1257,11 @@ void gemm_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, i
   CG_GEMM_CASE(2, 1, 64)
   CG_GEMM_CASE(2, 2, 64)
   CG_GEMM_CASE(0, 0, 128)
+  CG_GEMM_SUMS(2, 2, 128)  // weight gradients: A = dY^T, B = X, both token-major
+  CG_GEMM_SUMS(2, 2, 64)
+  CG_GEMM_SUMS(0, 0, 128)
+#undef CG_GEMM_RUN
+#undef CG_GEMM_SUMS
 #undef CG_GEMM_CASE
   CG_LAUNCHED();
   if (part) {
@@ -1249,7 +1278,7 @@ size_t gemm_workspace_bytes(int32_t m, int32_t n, int32_t k) {
   size_t most = 0;
   for (bool generic : {false, true}) {
     const GemmPlan pl = gemm_plan(m, n, k, generic);
-    if (pl.slices > 1) most = std::max(most, size_t(pl.slices) * size_t(m) * size_t(n) * 4);
+    if (pl.slices > 1) most = std::max(most, slice_bytes(pl, m, n));
   }
   return most;
 }
@@ -1258,16 +1287,14 @@ size_t column_sum_ws(int32_t rows, int32_t cols) {
   return rows > 2048 ? size_t((rows + 255) / 256) * size_t(std::max(cols, 0)) * 4 : 0;
 }
 
-// out[c] (+)= sum_r x[r * ld + c]; with `bf16`, the sum of the bf16-rounded entries, rounded to
-// bf16 (a bias gradient under autocast: the sum of a bf16 gradient, returned in bf16).
+// out[c] (+)= sum_r x[r * ld + c].
 void column_sum_launch(const float *x, int32_t rows, int32_t cols, int64_t ld, float *out, int32_t accumulate,
-                       void *workspace, size_t workspace_size, bool bf16, void *stream) {
+                       void *workspace, size_t workspace_size, void *stream) {
   if (cols == 0) return;
   CG_REQUIRE(x && out && rows >= 0, CG_ERR_INVALID, "column sum operands are required");
   hipStream_t s = as_stream(stream);
-  const int32_t r = bf16 ? 1 : 0;
   if (rows <= 2048) {
-    column_sum_kernel<<<dim3(blocks_of(cols, 64), 1), 256, 0, s>>>(x, rows, cols, ld, out, accumulate, rows, r, r);
+    column_sum_kernel<<<dim3(blocks_of(cols, 64), 1), 256, 0, s>>>(x, rows, cols, ld, out, accumulate, rows);
     CG_LAUNCHED();
     return;
   }
@@ -1275,10 +1302,9 @@ void column_sum_launch(const float *x, int32_t rows, int32_t cols, int64_t ld, f
   CG_REQUIRE(workspace && workspace_size >= need, CG_ERR_INVALID, "column sum: workspace too small");
   const int chunks = (rows + 255) / 256;
   float *part = static_cast<float *>(workspace);
-  column_sum_kernel<<<dim3(blocks_of(cols, 64), unsigned(chunks)), 256, 0, s>>>(x, rows, cols, ld, part, 0, 256, r, 0);
+  column_sum_kernel<<<dim3(blocks_of(cols, 64), unsigned(chunks)), 256, 0, s>>>(x, rows, cols, ld, part, 0, 256);
   CG_LAUNCHED();
-  column_sum_kernel<<<dim3(blocks_of(cols, 64), 1), 256, 0, s>>>(part, chunks, cols, cols, out, accumulate, chunks, 0,
-                                                                 r);
+  column_sum_kernel<<<dim3(blocks_of(cols, 64), 1), 256, 0, s>>>(part, chunks, cols, cols, out, accumulate, chunks);
   CG_LAUNCHED();
 }
 
@@ -1450,7 +1476,7 @@ size_t cg_column_sum_workspace_size(int32_t rows, int32_t cols) { return column_
 
 int cg_column_sum(const float *x, int32_t rows, int32_t cols, int64_t ld, float *out, int32_t accumulate,
                   void *workspace, size_t workspace_size, void *stream) {
-  return guarded([&] { column_sum_launch(x, rows, cols, ld, out, accumulate, workspace, workspace_size, false, stream); });
+  return guarded([&] { column_sum_launch(x, rows, cols, ld, out, accumulate, workspace, workspace_size, stream); });
 }
 
 int cg_gelu_fwd(const float *u, float *g, int64_t n, void *stream) {
@@ -1605,7 +1631,7 @@ size_t max_gemm_ws(const TrainDims &t) {
 }
 
 // Scratch of one call: GEMM split-K partials, then (backward) dx, dx1, dh (d each), du (F), do (Q),
-// dqkv (QKV), dsum (H), norm / column-sum partials.
+// dqkv (QKV), dsum (H), norm partials.
 struct Scratch {
   float *gemm_ws;
   size_t gemm_bytes;
@@ -1613,11 +1639,7 @@ struct Scratch {
   size_t red_bytes;
 };
 
-size_t red_bytes_of(const TrainDims &t) {
-  const int64_t cols = std::max({t.d, t.F, t.QKV});
-  return std::max(cg_norm_bwd_workspace_size(int32_t(t.n), int32_t(t.d)),
-                  cg_column_sum_workspace_size(int32_t(t.n), int32_t(cols)));
-}
+size_t red_bytes_of(const TrainDims &t) { return cg_norm_bwd_workspace_size(int32_t(t.n), int32_t(t.d)); }
 
 Scratch scratch_of(const TrainDims &t, void *base) {
   Scratch s{};
@@ -1667,10 +1689,12 @@ struct Gemm {
     gemm_launch(int32_t(M), int32_t(K), int32_t(N), 1.f, dy, N, 1, w, K, 1, 0.f, out, K, s.gemm_ws, s.gemm_bytes,
                 with(e), st);
   }
-  // out[N, K] = dy[M, N]^T x[M, K]
-  void tn(int64_t M, int64_t N, int64_t K, const float *dy, const float *x, float *out) const {
+  // out[N, K] = dy[M, N]^T x[M, K]; dbias[N] (when set) the column sums of dy
+  void tn(int64_t M, int64_t N, int64_t K, const float *dy, const float *x, float *out, float *dbias = nullptr) const {
+    Epi e;
+    e.row_sum = dbias;
     gemm_launch(int32_t(N), int32_t(K), int32_t(M), 1.f, dy, 1, N, x, K, 1, 0.f, out, K, s.gemm_ws, s.gemm_bytes,
-                with(Epi{}), st);
+                with(e), st);
   }
 };
 
@@ -1818,14 +1842,12 @@ int cg_trunk_train_backward(const cg_train_config *c, const cg_train_block *bloc
                                                              dple + l * t.pd, t.P);
         CG_LAUNCHED();
       }
-      gm.tn(t.n, t.d, t.F, s.dx, a.g, gw.down_w);
-      column_sum_launch(s.dx, N, int32_t(t.d), t.d, gw.down_b, 0, s.red, s.red_bytes, t.bf, st);
+      gm.tn(t.n, t.d, t.F, s.dx, a.g, gw.down_w, gw.down_b);
       Epi dgelu;  // du = (dx W_down) gelu'(u)
       dgelu.aux_in = a.u;
       dgelu.mode = EPI_GELU_GRAD;
       gm.nn(t.n, t.d, t.F, s.dx, w.down_w, s.du, dgelu);
-      gm.tn(t.n, t.F, t.d, s.du, a.h2, gw.up_w);
-      column_sum_launch(s.du, N, int32_t(t.F), t.F, gw.up_b, 0, s.red, s.red_bytes, t.bf, st);
+      gm.tn(t.n, t.F, t.d, s.du, a.h2, gw.up_w, gw.up_b);
       gm.nn(t.n, t.F, t.d, s.du, w.up_w, s.dh);
       ok(cg_norm_bwd(a.x1, s.dh, w.ln_mlp_w, a.m2, a.r2, s.dx1, s.dx, gw.ln_mlp_w, gw.ln_mlp_b, N, int32_t(t.d),
                      s.red, s.red_bytes, 0, st));
