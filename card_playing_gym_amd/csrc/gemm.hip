@@ -612,12 +612,13 @@ __global__ __launch_bounds__(256, 2) void split_tile_kernel(GemmArgs g) {
   }
 }
 
-enum SplitTile : int { SPLIT_16 = 16, SPLIT_32 = 32, SPLIT_TILE_64 = 64, SPLIT_TILE_128 = 128 };
+enum SplitTile : int { SPLIT_16, SPLIT_32, SPLIT_32x64, SPLIT_TILE_64, SPLIT_TILE_128 };
 
 // Which kernel a fp32 product takes.  16 x 16 tiles of split_rows_kernel while they are two per
 // CU or fewer (64 x 256 x 1024: 7.1 us, 32 x 32 tiles 10.5; 512 x 256 x 1024: both 10.9), 32 x 32
 // tiles up to four per CU (1024 x 256 x 1024: 12.2 us, 16 x 16 19.6, the 64-row staged tiles 36.9;
-// 1024 x 1024 x 256: 15.3 against 17.8), the staged tiles beyond (2048 x 1024 x 256: 26 us in
+// 1024 x 1024 x 256: 15.3 against 17.8; from two per CU and up to k = 256, 32 x 64 tiles with k over
+// four waves convert half as much: 12.3), the staged tiles beyond (2048 x 1024 x 256: 26 us in
 // 32 x 32 tiles, 18.5 staged; at four per CU and k = 1024 they lead as well, 36 against 42).
 // Staged tiles are 128 rows high when that gives two per CU (16384 x 1024 x 256: 76 against
 // 84 us), else 64 (16384 x 256 x 1024: 67 against 69).
@@ -626,20 +627,24 @@ SplitTile split_tile_of(int32_t m, int32_t n, int32_t k, int64_t lda) {
   auto tiles = [&](int64_t tm, int64_t tn) { return ((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
   if (tiles(16, 16) <= 512) return SPLIT_16;
   const int64_t t32 = tiles(32, 32);
-  if (t32 < 1024 || (t32 == 1024 && k <= 256) || std::max<int64_t>(k, lda) > TILE_MAX_STRIDE) return SPLIT_32;
+  if (t32 > 512 && t32 <= 1024 && k <= SPLIT_LN_K && n >= 64 && lda == k) return SPLIT_32x64;
+  if (t32 < 1024 || std::max<int64_t>(k, lda) > TILE_MAX_STRIDE) return SPLIT_32;
   return tiles(128, 128) >= 512 ? SPLIT_TILE_128 : SPLIT_TILE_64;
 }
 
 template <int EPI, bool LN>
 void launch_split_tile(const GemmArgs &g, hipStream_t s) {
   const SplitTile tile = split_tile_of(g.M, g.N, g.K, g.lda);
-  const int tn = tile >= SPLIT_TILE_64 ? ST_N : tile;
-  const dim3 grid((g.N + tn - 1) / tn, (g.M + tile - 1) / tile);
+  const int tm = tile == SPLIT_16 ? 16 : tile <= SPLIT_32x64 ? 32 : tile == SPLIT_TILE_64 ? 64 : 128;
+  const int tn = tile <= SPLIT_32 ? tm : tile == SPLIT_32x64 ? 64 : ST_N;
+  const dim3 grid((g.N + tn - 1) / tn, (g.M + tm - 1) / tm);
   CG_REQUIRE(grid.y <= 65535u, CG_ERR_UNSUPPORTED, "too many rows for one launch");
   if (tile == SPLIT_16) {
     split_rows_kernel<16, 16, 1, 1, 8, EPI, LN><<<grid, 512, 0, s>>>(g);
   } else if (tile == SPLIT_32) {
     split_rows_kernel<32, 32, 1, 1, 8, EPI, LN><<<grid, 512, 0, s>>>(g);
+  } else if (tile == SPLIT_32x64) {
+    split_rows_kernel<32, 64, 1, 1, 4, EPI, LN><<<grid, 256, 0, s>>>(g);
   } else {
     CG_REQUIRE(!LN, CG_ERR_UNSUPPORTED, "the staged product takes rows that are already normalised");
     if (tile == SPLIT_TILE_64) split_tile_kernel<64, EPI><<<grid, 256, 0, s>>>(g);
@@ -746,6 +751,46 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(const float *__rest
   }
 }
 
+// The same for d a multiple of 4 up to 256 and 16-byte aligned rows: a lane holds four consecutive
+// columns of a row, a wave four rows with all their loads in flight (16384 x 256: 9.1 -> 8.6 us).
+__global__ __launch_bounds__(256) void layernorm_rows4_kernel(const float *__restrict__ x,
+                                                              const int32_t *__restrict__ index,
+                                                              const float *__restrict__ w,
+                                                              const float *__restrict__ b, float eps,
+                                                              void *__restrict__ y, int32_t y_dtype, int32_t n,
+                                                              int32_t d) {
+  const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 4, k = 4 * (threadIdx.x & 63);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  const bool in = k < d;
+  f32x4 v[4];
+  int src[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = min(row0 + r, n - 1);
+    src[r] = index ? index[row] : row;
+    v[r] = src[r] >= 0 && in ? *reinterpret_cast<const f32x4 *>(x + int64_t(src[r]) * d + k) : zero;
+  }
+  const f32x4 g = in ? *reinterpret_cast<const f32x4 *>(w + k) : zero, o = in ? *reinterpret_cast<const f32x4 *>(b + k) : zero;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float mean = wave_sum((v[r][0] + v[r][1]) + (v[r][2] + v[r][3])) / float(d);
+    float q = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float t = in ? v[r][e] - mean : 0.f;
+      q = fmaf(t, t, q);
+    }
+    const float rstd = rsqrtf(wave_sum(q) / float(d) + eps);
+    if (row0 + r >= n || !in) continue;
+    f32x4 out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = src[r] >= 0 ? fmaf((v[r][e] - mean) * rstd, g[e], o[e]) : 0.f;
+    const int64_t at = int64_t(row0 + r) * d + k;
+    if (y_dtype == CG_BF16) *reinterpret_cast<u32x2 *>(static_cast<bf16 *>(y) + at) = cvt4<bf16>(out);
+    else *reinterpret_cast<f32x4 *>(static_cast<float *>(y) + at) = out;
+  }
+}
+
 __global__ void convert_kernel(const float *__restrict__ x, void *__restrict__ y, int32_t dtype, int64_t n) {
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
     if (dtype == CG_BF16) static_cast<bf16 *>(y)[i] = from_f32<bf16>(x[i]);
@@ -769,7 +814,7 @@ void launch_gemm(const GemmArgs &g, hipStream_t s) {
 
 bool split_gemm_norms(int32_t m, int32_t n, int32_t k, const float *w, const float *b) {
   return k <= SPLIT_LN_K && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 &&
-         split_tile_of(m, n, k, k) <= SPLIT_32;
+         split_tile_of(m, n, k, k) <= SPLIT_32x64;
 }
 
 void launch_layernorm_rows(const float *x, const int32_t *index, const float *w, const float *b,
@@ -777,7 +822,11 @@ void launch_layernorm_rows(const float *x, const int32_t *index, const float *w,
                            hipStream_t s) {
   if (n <= 0) return;
   const unsigned grid = unsigned((n + 3) / 4);
-  if (d <= 256) layernorm_rows_kernel<4><<<grid, 256, 0, s>>>(x, index, w, b, eps, y, y_dtype, n, d);
+  const uintptr_t at = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(b) |
+                       reinterpret_cast<uintptr_t>(y);
+  if (d <= 256 && d % 4 == 0 && (at & 15) == 0)
+    layernorm_rows4_kernel<<<unsigned((int64_t(n) + 15) / 16), 256, 0, s>>>(x, index, w, b, eps, y, y_dtype, n, d);
+  else if (d <= 256) layernorm_rows_kernel<4><<<grid, 256, 0, s>>>(x, index, w, b, eps, y, y_dtype, n, d);
   else if (d <= 512) layernorm_rows_kernel<8><<<grid, 256, 0, s>>>(x, index, w, b, eps, y, y_dtype, n, d);
   else if (d <= 1024) layernorm_rows_kernel<16><<<grid, 256, 0, s>>>(x, index, w, b, eps, y, y_dtype, n, d);
   else throw Error(CG_ERR_UNSUPPORTED, "LayerNorm width above 1024");

@@ -592,6 +592,10 @@ struct AttnTrain {
   float *out, *lse_out, *dsum, *dq, *dk, *dv;
   int32_t round;  // bf16 outputs (o, dq, dk, dv), as SDPA on bf16 operands returns them
   int32_t vec;    // output rows start 16-byte aligned
+  // dK / dV of `splits` parts of each head group, [split][n][dk | dv of every KV head], summed (and
+  // rounded) by merge_dkv_kernel; NULL: one part, written to dk / dv.
+  float *parts;
+  int32_t splits;
 };
 
 __device__ __forceinline__ float attn_out(const AttnTrain &a, float v) { return a.round ? round_bf16(v) : v; }
@@ -834,7 +838,7 @@ constexpr float LOG2E = 1.4426950408889634f;
 // the rows, the lane's query li on the column), row statistics per query across the four
 // lanes li + 16 lg, O^T += V^T P^T.
 template <int D, int PARTS>
-__global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnTrain a) {
+__global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_fwd_kernel(const AttnTrain a) {
   using S = AttnDims<D, PARTS>;
   __shared__ __align__(16) char lds[S::ROWS + S::COLS];
   char *const kr = lds, *const vc = lds + S::ROWS;
@@ -923,7 +927,7 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnTrain a) {
 // dQ (and D = rowsum(dO * O)) with the forward's blocks: S^T = K Q^T and dP^T = V dO^T per
 // 16-key tile, P from the saved log-sum-exp, dS = P (dP - D), dQ^T += K^T dS^T.
 template <int D, int PARTS>
-__global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const AttnTrain a) {
+__global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_bwd_dq_kernel(const AttnTrain a) {
   using S = AttnDims<D, PARTS>;
   __shared__ __align__(16) char lds[2 * S::ROWS + S::COLS];
   char *const kr = lds, *const vr = lds + S::ROWS, *const kc = lds + 2 * S::ROWS;
@@ -1012,14 +1016,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const AttnTrain a) {
 // dK / dV: a block holds 64 keys of KV head blockIdx.y, wave w keys j0 + 16 w + li in
 // registers, and walks the units (KT tokens of one head of the group) that can see them,
 // staged through LDS.  S = Q K^T and dP = dO V^T (queries on the rows), P and dS per lane,
-// dV^T += dO^T P and dK^T += Q^T dS.
+// dV^T += dO^T P and dK^T += Q^T dS.  A block's walk is its critical path (the first keys of a
+// 256-token sequence see 16 units of four heads), so the heads of a group may be split over
+// blockIdx.z.
 template <int D, int PARTS>
 __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
   using S = AttnDims<D, PARTS>;
   __shared__ __align__(16) char lds[2 * S::ROWS + 2 * S::COLS];
   __shared__ __align__(16) float ls[2 * KT];
   char *const qr = lds, *const gr = lds + S::ROWS, *const qc = lds + 2 * S::ROWS, *const gc = qc + S::COLS;
-  const int G = a.H / a.KVH, hk = blockIdx.y;
+  const int G = a.H / a.KVH / a.splits, hk = blockIdx.y, h0 = hk * (a.H / a.KVH) + blockIdx.z * G;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   // Early keys of a sequence are seen by more queries: odd KV heads walk the key blocks backwards,
   // so that the CU that got a long block first gets a short one next.
@@ -1044,7 +1050,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
   float4 qp[S::PER][2], gp[S::PER][2];
   float sp = 0.f;
   auto load = [&](int u) {
-    const int h = hk * G + u % G;
+    const int h = h0 + u % G;
     const int64_t t0 = j0 + KT * (u / G), last = min<int64_t>(a.n, q_hi) - 1;
     rows_load<D, PARTS>(qp, a.q + h * D, a.ldq, t0, last);
     rows_load<D, PARTS>(gp, a.dout + h * D, int64_t(a.H) * D, t0, last);
@@ -1100,6 +1106,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
     }
   }
   if (!live) return;
+  if (a.parts) {
+    float *row = a.parts + (int64_t(blockIdx.z) * a.n + j) * 2 * a.KVH * D + hk * D;
+#pragma unroll
+    for (int dt = 0; dt < S::DT; ++dt)
+      if (dt * 16 + 4 * lg < D) {
+        *reinterpret_cast<f32x4 *>(row + dt * 16 + 4 * lg) = dk[dt] * a.scale;
+        *reinterpret_cast<f32x4 *>(row + a.KVH * D + dt * 16 + 4 * lg) = dv[dt];
+      }
+    return;
+  }
   float *dkrow = a.dk + j * a.ldk + hk * D, *dvrow = a.dv + j * a.ldv + hk * D;
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
@@ -1107,6 +1123,20 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
       store4(a, dkrow + dt * 16 + 4 * lg, dk[dt], a.scale);
       store4(a, dvrow + dt * 16 + 4 * lg, dv[dt], 1.0f);
     }
+}
+
+// dk / dv = the sum of the head parts (width = KVH * D columns each, a multiple of 4), rounded like the
+// attention's other outputs.
+__global__ void merge_dkv_kernel(const AttnTrain a, int32_t width) {
+  const int quads = 2 * width / 4;
+  const int64_t total = int64_t(a.n) * quads;
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t t = i / quads;
+    const int c = int(i % quads) * 4;
+    f32x4 v = *reinterpret_cast<const f32x4 *>(a.parts + t * 2 * width + c);
+    for (int z = 1; z < a.splits; ++z) v += *reinterpret_cast<const f32x4 *>(a.parts + (z * int64_t(a.n) + t) * 2 * width + c);
+    store4(a, c < width ? a.dk + t * a.ldk + c : a.dv + t * a.ldv + c - width, v, 1.0f);
+  }
 }
 
 // dst[i] = 0: clears the accumulated gradients (a kernel rather than a memset node, so a
@@ -1334,7 +1364,7 @@ void attn_fwd_launch(const cg_attn_train *p, bool bf16_operands, hipStream_t s) 
   check_attn_train(p);
   if (p->n == 0) return;
   AttnTrain a{p->n, p->H, p->KVH, p->scale, p->seq_start, p->seq_of, p->q, p->k, p->v, p->ldq, p->ldk, p->ldv,
-              nullptr, nullptr, nullptr, p->o, p->lse, nullptr, nullptr, nullptr, nullptr, p->round_bf16, 1};
+              nullptr, nullptr, nullptr, p->o, p->lse, nullptr, nullptr, nullptr, nullptr, p->round_bf16, 1, nullptr, 1};
   CG_REQUIRE(a.out && a.lse_out, CG_ERR_INVALID, "attention forward outputs are required");
   CG_REQUIRE(aligned16(a.out), CG_ERR_INVALID, "attention output: 16-byte aligned");
   const dim3 grid = query_grid(*p);
@@ -1355,17 +1385,29 @@ void attn_fwd_launch(const cg_attn_train *p, bool bf16_operands, hipStream_t s) 
   CG_LAUNCHED();
 }
 
+// Backward; `parts` (16-byte aligned, part_floats floats; NULL: none) lets few key blocks split their head
+// groups.
 void attn_bwd_launch(const cg_attn_train *p, const float *dout, float *dsum, float *dq, float *dk, float *dv,
-                     bool bf16_operands, hipStream_t s) {
+                     bool bf16_operands, hipStream_t s, float *parts = nullptr, int64_t part_floats = 0) {
   check_attn_train(p);
   if (p->n == 0) return;
   AttnTrain a{p->n, p->H, p->KVH, p->scale, p->seq_start, p->seq_of, p->q, p->k, p->v, p->ldq, p->ldk, p->ldv,
               p->o, dout, p->lse, nullptr, nullptr, dsum, dq, dk, dv, p->round_bf16,
-              aligned16(dq) && aligned16(dk) && aligned16(dv)};
+              aligned16(dq) && aligned16(dk) && aligned16(dv), nullptr, 1};
   CG_REQUIRE(a.o && a.dout && a.lse && dsum && dq && dk && dv, CG_ERR_INVALID,
              "attention backward operands are required");
   CG_REQUIRE(aligned16(dout), CG_ERR_INVALID, "attention dO: 16-byte aligned");
-  const dim3 grid = query_grid(*p), grid_kv(blocks_of(p->n, 64), unsigned(p->KVH));
+  // Heads split while the blocks stay within eight per CU (13.8 k ragged tokens fp32: 432 blocks 77 us,
+  // 1728 blocks 52 and the merge 9), with one-part operands, whose walk is shorter, within two (64 x 256
+  // tokens: 512 blocks 45 us, 2048 blocks 37 and the merge 10).
+  const int64_t blocks = int64_t(blocks_of(p->n, 64)) * p->KVH, width = int64_t(p->KVH) * p->head_dim;
+  for (int z = 4; z > 1 && parts; z /= 2)
+    if (p->H / p->KVH % z == 0 && blocks * z <= (bf16_operands ? 512 : 2048) && z * 2 * width * p->n <= part_floats) {
+      a.splits = z;
+      a.parts = parts;
+      break;
+    }
+  const dim3 grid = query_grid(*p), grid_kv(blocks_of(p->n, 64), unsigned(p->KVH), unsigned(a.splits));
   switch (p->head_dim) {
 #define CG_BWD_CASE(DD)                                                      \
   case DD:                                                                   \
@@ -1384,6 +1426,10 @@ void attn_bwd_launch(const cg_attn_train *p, const float *dout, float *dsum, flo
     default: throw Error(CG_ERR_UNSUPPORTED, "training attention: head_dim 8, 16, 24, 32 or 64");
   }
   CG_LAUNCHED();
+  if (a.parts) {
+    merge_dkv_kernel<<<grid_1d(int64_t(p->n) * width / 2), 256, 0, s>>>(a, int32_t(width));
+    CG_LAUNCHED();
+  }
 }
 
 }  // namespace
@@ -1854,7 +1900,8 @@ int cg_trunk_train_backward(const cg_train_config *c, const cg_train_block *bloc
       gm.tn(t.n, t.d, t.Q, s.dx1, a.o, gw.out_w);
       gm.nn(t.n, t.d, t.Q, s.dx1, w.out_w, s.dout);
       const cg_attn_train at = attn_args(t, seq_start, tail.seq_of, a.qkv, a.o, a.lse);
-      attn_bwd_launch(&at, s.dout, s.dsum, s.dqkv, s.dqkv + t.Q, s.dqkv + t.Q + t.KVW, t.bf, st);
+      attn_bwd_launch(&at, s.dout, s.dsum, s.dqkv, s.dqkv + t.Q, s.dqkv + t.Q + t.KVW, t.bf, st, s.du,
+                      t.n * t.F);  // (du has been used up)
       const int32_t vi = c->value_index ? c->value_index[l] : -1;
       if (vi >= 0 && dvalues) {
         const float *dv = s.dqkv + t.Q + t.KVW;
