@@ -218,6 +218,143 @@ __global__ __launch_bounds__(256, 2) void gemm_strided_kernel(int32_t M, int32_t
   else finish(std::false_type{});
 }
 
+// ---- products of few rows --------------------------------------------------------------
+// A microbatch of hundreds of rows is bound by launches and by the latency of each: a staged product
+// split over k takes a second launch for its slices (792 x 256 x 512: 9.6 + 4 us).  Here one launch
+// spreads k over the eight waves of a 32 x 32 tile's block, each reading its operand fragments straight
+// from global memory (lane (li, lg): row li, k 8 lg .. 8 lg + 7 of a 32-k step) and the partial tiles
+// meeting in LDS.
+template <int MODE>
+__device__ __forceinline__ void rows_frag(const float *__restrict__ p, int64_t sk, int k0, int K, split_f32x4 (&v)[2]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int k = k0 + 4 * h;
+    if constexpr (MODE == 1) {  // K is a multiple of 4
+      const split_f32x4 x = *reinterpret_cast<const split_f32x4 *>(p + min(k, K - 4));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[h][e] = k < K ? x[e] : 0.f;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = p[int64_t(min(k + e, K - 1)) * sk];
+        v[h][e] = k + e < K ? x : 0.f;
+      }
+    }
+  }
+}
+
+constexpr int ROWS_K = 1024;  // longest reduction and most tiles of the kernel below
+constexpr int64_t ROWS_TILES = 512;
+
+template <int AM, int BM, bool BF, bool SUMS>
+__global__ __launch_bounds__(512) void gemm_rows_kernel(int32_t M, int32_t N, int32_t K, float alpha,
+                                                        const float *__restrict__ A, int64_t sam, int64_t sak,
+                                                        const float *__restrict__ B, int64_t sbk, int64_t sbn, float beta,
+                                                        float *__restrict__ C, int64_t ldc, const Epi epi) {
+  constexpr int T = 32, PITCH = T + 4, WAVES = 8, PARTS = BF ? 1 : 3;
+  __shared__ float red[WAVES][T * PITCH];
+  __shared__ float sums[SUMS ? WAVES : 1][T];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
+  const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+  const float *ar[2], *br[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    ar[i] = A + int64_t(min(m0 + 16 * i + li, M - 1)) * sam;
+    br[i] = B + int64_t(min(n0 + 16 * i + li, N - 1)) * sbn;
+  }
+  f32x4 acc[2][2], cor[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = cor[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float rs[2] = {0.f, 0.f};
+  for (int k0 = 32 * wave; k0 < K; k0 += 2 * 32 * WAVES) {
+    split_f32x4 a[2][2][2], b[2][2][2];  // two steps' operands in flight
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int k = k0 + t * 32 * WAVES;
+      if (k >= K) continue;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        rows_frag<AM>(ar[i], sak, k + 8 * lg, K, a[t][i]);
+        rows_frag<BM>(br[i], sbk, k + 8 * lg, K, b[t][i]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      if (k0 + t * 32 * WAVES >= K) continue;
+      if constexpr (BF) {
+        split_u32x4 af[2], bf[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            af[i][e] = split_pack(a[t][i][e >> 1][2 * (e & 1)], a[t][i][e >> 1][2 * (e & 1) + 1]);
+            bf[i][e] = split_pack(b[t][i][e >> 1][2 * (e & 1)], b[t][i][e >> 1][2 * (e & 1) + 1]);
+            if constexpr (SUMS) rs[i] += __uint_as_float(af[i][e] << 16) + __uint_as_float(af[i][e] & 0xffff0000u);
+          }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = split_mma1(af[i], bf[j], acc[i][j]);
+      } else {
+        Split8 as[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          as[i] = split8(a[t][i][0], a[t][i][1]);
+          if constexpr (SUMS) {
+            const split_f32x4 s = a[t][i][0] + a[t][i][1];
+            rs[i] += (s[0] + s[1]) + (s[2] + s[3]);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const Split8 bs = split8(b[t][j][0], b[t][j][1]);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) split_mma(as[i], bs, acc[i][j], cor[i][j]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[wave][(16 * i + 4 * lg + r) * PITCH + 16 * j + li] = PARTS == 3 ? acc[i][j][r] + cor[i][j][r] : acc[i][j][r];
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      rs[i] += __shfl_xor(rs[i], 16);
+      rs[i] += __shfl_xor(rs[i], 32);
+      if (lg == 0) sums[wave][16 * i + li] = rs[i];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = tid; e < T * T; e += 64 * WAVES) {
+    const int r = e / T, c = e % T, m = m0 + r, n = n0 + c;
+    float v = red[0][r * PITCH + c];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) v += red[w][r * PITCH + c];
+    if (m >= M || n >= N) continue;
+    if (!BF && !split_finite(v)) {  // see split.h
+      v = 0.f;
+      for (int k = 0; k < K; ++k) v = fmaf(A[m * sam + k * sak], B[k * sbk + n * sbn], v);
+    }
+    epilogue(epi, alpha * v, beta, C, ldc, m, n);
+  }
+  if constexpr (SUMS) {
+    if (blockIdx.x == 0 && tid < T && m0 + tid < M) {
+      float v = sums[0][tid];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) v += sums[w][tid];
+      epi.row_sum[m0 + tid] = BF ? round_bf16(v) : v;
+    }
+  }
+}
+
 // C[m, n] = epilogue(alpha * sum_z part[z][m, n]).  A thread takes four consecutive entries
 // (float4 loads when N is a multiple of 4) and keeps four slices in flight.
 __global__ void gemm_reduce_kernel(int32_t M, int32_t N, int32_t slices, float alpha, const float *__restrict__ part,
@@ -1244,6 +1381,31 @@ GemmPlan plan_of(int32_t m, int32_t n, int32_t k, const float *a, int64_t sam, i
   return gemm_plan(m, n, k, *am == 0);
 }
 
+void rows_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, int64_t sam, int64_t sak, const float *b,
+                 int64_t sbk, int64_t sbn, float beta, float *c, int64_t ldc, const Epi &epi, int am, int bm,
+                 hipStream_t s) {
+  const dim3 grid(unsigned((n + 31) / 32), unsigned((m + 31) / 32));
+  const bool bf = epi.round != 0, sums = epi.row_sum != nullptr;
+#define CG_ROWS_RUN(A_, B_, BF_, S_) \
+  gemm_rows_kernel<A_, B_, BF_, S_><<<grid, 512, 0, s>>>(m, n, k, alpha, a, sam, sak, b, sbk, sbn, beta, c, ldc, epi)
+#define CG_ROWS_CASE(A_, B_, S_)               \
+  if (sums == S_ && am == A_ && bm == B_) {    \
+    if (bf) CG_ROWS_RUN(A_, B_, true, S_);     \
+    else CG_ROWS_RUN(A_, B_, false, S_);       \
+  }
+  CG_REQUIRE(!sums || (am == 2 && bm == 2) || (am == 0 && bm == 0), CG_ERR_UNSUPPORTED, "GEMM: row sums of this layout");
+  CG_ROWS_CASE(1, 1, false)
+  CG_ROWS_CASE(1, 2, false)
+  CG_ROWS_CASE(2, 1, false)
+  CG_ROWS_CASE(2, 2, false)
+  CG_ROWS_CASE(0, 0, false)
+  CG_ROWS_CASE(2, 2, true)
+  CG_ROWS_CASE(0, 0, true)
+#undef CG_ROWS_CASE
+#undef CG_ROWS_RUN
+  CG_LAUNCHED();
+}
+
 void gemm_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, int64_t sam, int64_t sak,
                  const float *b, int64_t sbk, int64_t sbn, float beta, float *c, int64_t ldc, void *workspace,
                  size_t workspace_size, const Epi &epi, void *stream) {
@@ -1254,6 +1416,10 @@ void gemm_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, i
              "GEMM epilogue: GELU needs its second output, GELU' its pre-activation");
   int am, bm;
   const GemmPlan pl = plan_of(m, n, k, a, sam, sak, b, sbk, sbn, &am, &bm);
+  if (k > 0 && k <= ROWS_K && int64_t((m + 31) / 32) * ((n + 31) / 32) <= ROWS_TILES) {
+    rows_launch(m, n, k, alpha, a, sam, sak, b, sbk, sbn, beta, c, ldc, epi, am, bm, as_stream(stream));
+    return;
+  }
   const size_t need = pl.slices > 1 ? slice_bytes(pl, m, n) : 0;
   CG_REQUIRE(k > 0 || !epi.row_sum, CG_ERR_INVALID, "GEMM: row sums of an empty product");
   CG_REQUIRE(need == 0 || (workspace && workspace_size >= need), CG_ERR_INVALID,
