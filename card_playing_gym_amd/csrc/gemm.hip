@@ -261,6 +261,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs g) {
   }
 }
 
+// (C + addend) * scale with the addend's rounding (EPI_SCALE_ADD).
+__device__ __forceinline__ float scale_add(const GemmArgs &g, float c, float addend) {
+  if (g.round_c) c = to_f32(from_f32<bf16>(c));
+  if (g.add_dtype != CG_BF16) return (c + addend) * g.scale;
+  return to_f32(from_f32<bf16>(to_f32(from_f32<bf16>(c + addend)) * g.scale));
+}
+
 // ---- fp32 products of few rows -----------------------------------------------------------
 // What bounds a decode wave's product is latency, not rate: 64 rows x 1024 x 256 is 1 MB of
 // weights and 0.03 GFLOP.  So the k of one small output tile is spread over the WK waves of a
@@ -271,49 +278,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs g) {
 // rows of A are normalised on the way in (every wave holds its k of the tile's rows, so the
 // statistics cost one exchange through LDS), which saves the whole-row tiles, and the launches,
 // that a LayerNorm in the producer's epilogue needs.
-template <int EPI>
-__device__ __forceinline__ void split_store(const GemmArgs &g, int m, int n, float c) {
-  if (g.bias) c += g.bias[n];
-  if constexpr (EPI == EPI_RESID) {
-    if (g.ple) c = fmaf(g.ple[int64_t(m) * g.ld_ple + g.ple_off + n % g.ple_dim], g.ple_scale, c);
-    float *dst = g.resid + int64_t(m) * g.ldr + n;
-    *dst += c;
-  } else if constexpr (EPI == EPI_QKV) {
-    const int kvw = g.kv_heads * g.head_dim;
-    if (n < g.q_cols) {
-      static_cast<float *>(g.out)[int64_t(m) * g.ldo + n] = c;
-      return;
-    }
-    const int row = g.tok_row[m];
-    if (row < 0) return;
-    const bool is_v = n >= g.q_cols + kvw;
-    const int kv = n - g.q_cols - (is_v ? kvw : 0);
-    const int h = kv / g.head_dim, d = kv % g.head_dim;
-    if (is_v && g.vemb_off >= 0) c += g.vemb[int64_t(m) * g.ld_vemb + g.vemb_off + kv];
-    const int64_t dst = ((int64_t(row) * g.kv_heads + h) * g.max_len + g.tok_pos[m]) * g.head_dim + d;
-    void *base = is_v ? g.vc : g.kc;
-    if (g.kv_dtype == CG_BF16) static_cast<bf16 *>(base)[dst] = from_f32<bf16>(c);
-    else if (g.kv_dtype == CG_F16) static_cast<f16 *>(base)[dst] = from_f32<f16>(c);
-    else static_cast<float *>(base)[dst] = c;
-  } else {
-    float v = c;
-    if constexpr (EPI == EPI_GELU) v = gelu_erf(c);
-    if constexpr (EPI == EPI_SCALE_ADD) {
-      const float cc = g.round_c ? to_f32(from_f32<bf16>(c)) : c;
-      const int64_t ai = int64_t(m) * g.ld_add + n;
-      if (g.add_dtype == CG_BF16) {
-        const float sum = to_f32(from_f32<bf16>(cc + to_f32(static_cast<const bf16 *>(g.addend)[ai])));
-        v = to_f32(from_f32<bf16>(sum * g.scale));
-      } else {
-        v = (cc + static_cast<const float *>(g.addend)[ai]) * g.scale;
-      }
-    }
-    const int64_t o = int64_t(m) * g.ldo + n;
-    if (g.out_dtype == CG_BF16) static_cast<bf16 *>(g.out)[o] = from_f32<bf16>(v);
-    else static_cast<float *>(g.out)[o] = v;
-  }
-}
-
 constexpr int SPLIT_LN_K = 256;  // widest A row that a block normalises by itself
 
 template <int BM, int BN, int WM, int WN, int WK, int EPI, bool LN>
@@ -472,24 +436,106 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void split_rows_kernel(GemmArgs 
       for (int r = 0; r < 4; ++r)
         red[wk][(wm * FM * 16 + i * 16 + 4 * lg + r) * PITCH + wn * FN * 16 + j * 16 + li] = acc[i][j][r] + cor[i][j][r];
   __syncthreads();
+  // A thread's results, then everything their epilogue reads at once, then the epilogue: read
+  // element by element, each load waited for the store before it (a 1024-row fp32 decode step of
+  // 41 launches: 550 us, 539 so).
+  constexpr int E = (BM * BN + THREADS - 1) / THREADS;
+  float v[E];
+  int mr[E], nc[E];
+  bool ok[E];
 #pragma unroll
-  for (int e = tid; e < BM * BN; e += THREADS) {
-    const int r = e / BN, c = e % BN, m = m0 + r, n = n0 + c;
-    float v = red[0][r * PITCH + c];
+  for (int e = 0; e < E; ++e) {
+    const int at = min(tid + e * THREADS, BM * BN - 1), r = at / BN, c = at % BN, m = m0 + r, n = n0 + c;
+    ok[e] = tid + e * THREADS < BM * BN && m < g.M && n < g.N;
+    mr[e] = min(m, g.M - 1);
+    nc[e] = min(n, g.N - 1);
+    v[e] = red[0][r * PITCH + c];
 #pragma unroll
-    for (int w = 1; w < WK; ++w) v += red[w][r * PITCH + c];
-    if (m >= g.M || n >= g.N) continue;
-    if (!split_finite(v)) {  // see split.h
+    for (int w = 1; w < WK; ++w) v[e] += red[w][r * PITCH + c];
+    if (ok[e] && !split_finite(v[e])) {  // see split.h
       const float *ar = static_cast<const float *>(g.A) + int64_t(m) * g.lda;
       const float *wr = static_cast<const float *>(g.W) + int64_t(n) * g.K;
-      v = 0.f;
+      v[e] = 0.f;
       for (int k = 0; k < g.K; ++k) {
         float x = ar[k];
         if constexpr (LN) x = fmaf((x - norm[0][r]) * norm[1][r], g.a_ln_w[k], g.a_ln_b[k]);
-        v = fmaf(x, wr[k], v);
+        v[e] = fmaf(x, wr[k], v[e]);
       }
     }
-    split_store<EPI>(g, m, n, v);
+  }
+  if (g.bias) {
+    float bias[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) bias[e] = g.bias[nc[e]];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] += bias[e];
+  }
+  if constexpr (EPI == EPI_RESID) {
+    if (g.ple) {
+      float p[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) p[e] = g.ple[int64_t(mr[e]) * g.ld_ple + g.ple_off + nc[e] % g.ple_dim];
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = fmaf(p[e], g.ple_scale, v[e]);
+    }
+    float x[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = g.resid[int64_t(mr[e]) * g.ldr + nc[e]];
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (ok[e]) g.resid[int64_t(mr[e]) * g.ldr + nc[e]] = x[e] + v[e];
+  } else if constexpr (EPI == EPI_QKV) {
+    const int kvw = g.kv_heads * g.head_dim;
+    int row[E], pos[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      row[e] = g.tok_row[mr[e]];
+      pos[e] = g.tok_pos[mr[e]];
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (!ok[e]) continue;
+      const int m = mr[e], n = nc[e];
+      if (n < g.q_cols) {
+        static_cast<float *>(g.out)[int64_t(m) * g.ldo + n] = v[e];
+        continue;
+      }
+      if (row[e] < 0) continue;
+      const bool is_v = n >= g.q_cols + kvw;
+      const int kv = n - g.q_cols - (is_v ? kvw : 0);
+      const int h = kv / g.head_dim, d = kv % g.head_dim;
+      float c = v[e];
+      if (is_v && g.vemb_off >= 0) c += g.vemb[int64_t(m) * g.ld_vemb + g.vemb_off + kv];
+      const int64_t dst = ((int64_t(row[e]) * g.kv_heads + h) * g.max_len + pos[e]) * g.head_dim + d;
+      void *base = is_v ? g.vc : g.kc;
+      if (g.kv_dtype == CG_BF16) static_cast<bf16 *>(base)[dst] = from_f32<bf16>(c);
+      else if (g.kv_dtype == CG_F16) static_cast<f16 *>(base)[dst] = from_f32<f16>(c);
+      else static_cast<float *>(base)[dst] = c;
+    }
+  } else {
+    if constexpr (EPI == EPI_GELU) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = gelu_erf(v[e]);
+    }
+    if constexpr (EPI == EPI_SCALE_ADD) {
+      float x[E];
+      if (g.add_dtype == CG_BF16) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = to_f32(static_cast<const bf16 *>(g.addend)[int64_t(mr[e]) * g.ld_add + nc[e]]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = static_cast<const float *>(g.addend)[int64_t(mr[e]) * g.ld_add + nc[e]];
+      }
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = scale_add(g, v[e], x[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (!ok[e]) continue;
+      const int64_t o = int64_t(mr[e]) * g.ldo + nc[e];
+      if (g.out_dtype == CG_BF16) static_cast<bf16 *>(g.out)[o] = from_f32<bf16>(v[e]);
+      else static_cast<float *>(g.out)[o] = v[e];
+    }
   }
 }
 
@@ -592,11 +638,28 @@ __global__ __launch_bounds__(256, 2) void split_tile_kernel(GemmArgs g) {
         }
       }
     } else if constexpr (EPI == EPI_SCALE_ADD) {
+      float e[4][4];
+      if (g.add_dtype == CG_BF16) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) e[j][r] = to_f32(static_cast<const bf16 *>(g.addend)[mr[r] * g.ld_add + nj[j]]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) e[j][r] = static_cast<const float *>(g.addend)[mr[r] * g.ld_add + nj[j]];
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (nok[j] && ok[r]) split_store<EPI>(g, int(mr[r]), nj[j], acc[i][j][r]);
+        for (int r = 0; r < 4; ++r) {
+          if (!nok[j] || !ok[r]) continue;
+          const float v = scale_add(g, c[j][r], e[j][r]);
+          const int64_t o = mr[r] * g.ldo + nj[j];
+          if (f32_out) static_cast<float *>(g.out)[o] = v;
+          else static_cast<bf16 *>(g.out)[o] = from_f32<bf16>(v);
+        }
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
