@@ -413,8 +413,8 @@ GemmPlan gemm_plan(int32_t m, int32_t n, int32_t k, bool generic) {
     slices = int(std::min<int64_t>(512 / tiles, k / (stages * GT_K)));
     slices = std::max(1, std::min(slices, 32));
   }
-  const int kc = ((k + slices - 1) / slices + GT_K - 1) / GT_K * GT_K;
-  slices = (k + kc - 1) / kc;
+  const int kc = std::max((k + slices - 1) / slices + GT_K - 1, GT_K) / GT_K * GT_K;  // (k 0: one empty slice)
+  slices = std::max((k + kc - 1) / kc, 1);
   return {tm, slices, kc};
 }
 

@@ -55,6 +55,18 @@ def test_gemm_layouts(device, size):
     close(out, dy.double().T @ x.double(), what="tn")
 
 
+@pytest.mark.parametrize("m, n", [(5, 7), (2048, 512)], ids=["one-tile", "many"])
+def test_empty_reduction_leaves_the_prior_value(device, m, n):
+    """k = 0: out = alpha * 0 + beta * out."""
+
+    out = torch.randn(m, n, device=device)
+    want = 3.0 * out
+    operand = torch.empty(8, device=device)
+    nat.call("cg_gemm_strided", m, n, 0, 0.5, operand.data_ptr(), 0, 1, operand.data_ptr(), 1, 0, 3.0, out.data_ptr(), n,
+             nat.CG_F32, None, 0, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("d", [64, 66, 240, 256, 600])
 def test_norms_and_gelu(device, d):
     g = torch.Generator().manual_seed(d)
