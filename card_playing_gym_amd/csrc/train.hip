@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256, 2) void gemm_strided_kernel(int32_t M, int32_t
     const int n = min(n0 + wn * 64 + j * 16 + li, N - 1);
     bj[j] = epi.bias ? epi.bias[n] : 0.f;
   }
-  const bool inside = m0 + TM <= M && n0 + GT_N <= N && ldc <= TILE_MAX_STRIDE;
+  const bool inside = m0 + TM <= M && n0 + GT_N <= N && ldc >= 0 && ldc <= TILE_MAX_STRIDE;
   auto finish = [&](auto whole) {
     constexpr bool WHOLE = decltype(whole)::value;
 #pragma unroll

@@ -67,6 +67,22 @@ def test_empty_reduction_leaves_the_prior_value(device, m, n):
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("m, n, k", [(9, 5, 16), (2048, 512, 64), (2050, 513, 64), (128, 256, 2048)],
+                         ids=["rows", "whole-tiles", "edge-tiles", "split-k"])
+def test_output_rows_in_any_order(device, m, n, k):
+    """A negative row stride of C (its last row first in memory) gives the same rows, bit for bit."""
+
+    gen = torch.Generator(device=device).manual_seed(m)
+    x, w, prior = (torch.randn(s, generator=gen, device=device) for s in ((m, k), (n, k), (m, n)))
+    want, out = prior.clone(), prior.flip(0).contiguous()
+    T.linear_nt(x, w, want, beta=1.0)
+    size = nat.lib().cg_gemm_workspace_size(m, n, k)
+    workspace = torch.empty(max(size, 1), dtype=torch.uint8, device=device)
+    nat.call("cg_gemm_strided", m, n, k, 1.0, x.data_ptr(), k, 1, w.data_ptr(), 1, k, 1.0, T._ptr(out, (m - 1) * n), -n,
+             nat.CG_F32, workspace.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(out.flip(0), want)
+
+
 @pytest.mark.parametrize("d", [64, 66, 240, 256, 600])
 def test_norms_and_gelu(device, d):
     g = torch.Generator().manual_seed(d)
