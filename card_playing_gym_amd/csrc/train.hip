@@ -816,12 +816,14 @@ __device__ __forceinline__ void clear_lds(char *lds, int bytes) {
 }
 
 // Rows [r0, r0 + 64) of p (row stride ld floats, D used columns) into registers; rows past `last` are
-// read as the last (their scores are masked).  The row base is uniform, the rest 32 bits.
+// read as the last (their scores are masked).  The row base is uniform, the rest 32 bits where the
+// stride allows.
 template <int D, int PARTS>
 __device__ __forceinline__ void rows_load(SlotRegs<D, PARTS> &r, const float *__restrict__ p, int64_t ld, int64_t r0,
                                           int64_t last) {
   using S = AttnDims<D, PARTS>;
-  const char *base = reinterpret_cast<const char *>(p + r0 * ld);  // (strides are not negative)
+  const char *base = reinterpret_cast<const char *>(p + r0 * ld);
+  const bool near = ld >= 0 && ld <= TILE_MAX_STRIDE;
   const int left = int(min<int64_t>(last - r0, KT - 1));
 #pragma unroll
   for (int e = 0; e < S::PER; ++e) {
@@ -829,7 +831,7 @@ __device__ __forceinline__ void rows_load(SlotRegs<D, PARTS> &r, const float *__
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int at = min(row + h, left);
-      if (ld <= TILE_MAX_STRIDE)
+      if (near)
         r[e][h] = *reinterpret_cast<const float4 *>(base + 4u * (unsigned(at) * unsigned(ld) + unsigned(c)));
       else
         r[e][h] = *reinterpret_cast<const float4 *>(base + 4 * (at * ld + c));
@@ -1358,7 +1360,7 @@ void check_attn_train(const cg_attn_train *p) {
   CG_REQUIRE(p->q && p->k && p->v && p->seq_start && p->seq_of, CG_ERR_INVALID,
              "attention q, k, v, seq_start and seq_of are required");
   CG_REQUIRE(aligned16(p->q) && aligned16(p->k) && aligned16(p->v) && p->ldq % 4 == 0 && p->ldk % 4 == 0 &&
-                 p->ldv % 4 == 0 && p->ldq >= 0 && p->ldk >= 0 && p->ldv >= 0,
+                 p->ldv % 4 == 0,
              CG_ERR_INVALID, "attention q / k / v: 16-byte aligned rows (pointers and row strides)");
 }
 

@@ -174,6 +174,34 @@ def test_attention_forward_backward(device, D, H, KVH):
     close(dqkv[:, Q + KVW :].view(n, KVH, D), v.grad, what="dv")
 
 
+@pytest.mark.parametrize("D,H,KVH", [(32, 8, 2), (64, 4, 4), (8, 4, 2)])
+def test_attention_rows_in_any_order(device, D, H, KVH):
+    """Negative row strides of q / k / v and their gradients (the last token first in memory) give
+    the same numbers, bit for bit."""
+
+    lengths = [5, 70, 1, 130]
+    n, ld = sum(lengths), (H + 2 * KVH) * D
+    gen = torch.Generator(device=device).manual_seed(D)
+    qkv, do = torch.randn(n, ld, generator=gen, device=device), torch.randn(n, H * D, generator=gen, device=device)
+    seq_start = torch.tensor(np.concatenate([[0], np.cumsum(lengths)]), dtype=torch.int64, device=device)
+    seq_of = torch.arange(len(lengths), device=device, dtype=torch.int32).repeat_interleave(torch.tensor(lengths, device=device))
+    stream = torch.cuda.current_stream().cuda_stream
+    results = []
+    for step in (1, -1):
+        rows = qkv if step == 1 else qkv.flip(0).contiguous()
+        first = 0 if step == 1 else (n - 1) * ld
+        o, lse, dsum = (torch.empty(n, c, device=device) for c in (H * D, H, H))
+        grads = torch.empty_like(rows)
+        at = nat.AttnTrain(n, H, KVH, D, 1.0 / math.sqrt(D), seq_start.data_ptr(), seq_of.data_ptr(),
+                           *(T._ptr(rows, first + c) for c in (0, H * D, (H + KVH) * D)), *[step * ld] * 3,
+                           o.data_ptr(), lse.data_ptr())
+        nat.call("cg_attn_train_fwd", ctypes.byref(at), stream)
+        nat.call("cg_attn_train_bwd", ctypes.byref(at), do.data_ptr(), dsum.data_ptr(),
+                 *(T._ptr(grads, first + c) for c in (0, H * D, (H + KVH) * D)), stream)
+        results.append((o, lse, grads if step == 1 else grads.flip(0)))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
 CONFIGS = [
     dict(d_model=64, n_layers=2, n_heads=4, n_kv_heads=2, d_ff=128, per_layer_dim=16, value_embeddings="alternating"),
     dict(d_model=96, n_layers=1, n_heads=3, n_kv_heads=1, d_ff=160, per_layer_dim=0, value_embeddings="all"),
