@@ -786,18 +786,39 @@ __device__ __forceinline__ Operand<PARTS> operand_of(const float (&v)[8]) {
   return o;
 }
 
-// c + a b, smallest products first.
-template <int PA, int PB>
+// c + a b, smallest products first; of one order the last part of `b` first, or with `A_FIRST` of `a`:
+// mma_parts(a, b) and mma_parts<.., true>(b, a) add the same terms in the same order.
+template <int PA, int PB, bool A_FIRST = false>
 __device__ __forceinline__ f32x4 mma_parts(const Operand<PA> &a, const Operand<PB> &b, f32x4 c) {
 #pragma unroll
   for (int order = 2; order >= 0; --order)
 #pragma unroll
-    for (int i = 0; i < PA; ++i)
-#pragma unroll
-      for (int j = 0; j < PB; ++j)
-        if (i + j == order) c = split_mma1(a.p[i], b.p[j], c);
+    for (int i = 0; i <= order; ++i) {
+      const int ia = A_FIRST ? order - i : i, ib = order - ia;
+      if (ia < PA && ib < PB) c = split_mma1(a.p[ia], b.p[ib], c);
+    }
   return c;
 }
+
+// A score tile in natural units: three parts hold scaled queries already; bf16 queries are scaled
+// here, rounded before anything is subtracted.  The backward forms a score with the forward's own
+// operations, so that P = exp(score - lse) carries the rounding of lse alone: a score of any size that
+// the forward took as its maximum comes back as exp(0).
+template <int PARTS>
+__device__ __forceinline__ f32x4 natural_score(f32x4 c, float scale) {
+#pragma clang fp contract(off)
+  if constexpr (PARTS == 1) c = c * scale;
+  return c;
+}
+__device__ __forceinline__ float4 scaled_query(const float4 &q, float scale) {
+#pragma clang fp contract(off)
+  return float4{q.x * scale, q.y * scale, q.z * scale, q.w * scale};
+}
+
+constexpr float LOG2E = 1.4426950408889634f;
+
+// e^x (v_exp_f32 is 2^x).
+__device__ __forceinline__ float exp_natural(float x) { return __builtin_amdgcn_exp2f(x * LOG2E); }
 
 __device__ __forceinline__ float max_over_rows(float x) {  // over lanes li, li + 16, li + 32, li + 48
   x = fmaxf(x, __shfl_xor(x, 16));
@@ -921,8 +942,9 @@ __device__ __forceinline__ void row_operand(DimOperand<D, PARTS> &o, const float
     const int d = 32 * dk + 8 * lg;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const float4 x = live && d < D ? *reinterpret_cast<const float4 *>(p + d + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
-      v[4 * h] = x.x * scale, v[4 * h + 1] = x.y * scale, v[4 * h + 2] = x.z * scale, v[4 * h + 3] = x.w * scale;
+      const float4 x = scaled_query(
+          live && d < D ? *reinterpret_cast<const float4 *>(p + d + 4 * h) : float4{0.f, 0.f, 0.f, 0.f}, scale);
+      v[4 * h] = x.x, v[4 * h + 1] = x.y, v[4 * h + 2] = x.z, v[4 * h + 3] = x.w;
     }
     o[dk] = operand_of<PARTS>(v);
   }
@@ -971,13 +993,11 @@ __device__ __forceinline__ QueryStrip query_strip(const AttnTrain &a) {
   return q;
 }
 
-constexpr float LOG2E = 1.4426950408889634f;
-
-// Forward: online softmax (base 2) over K / V tiles staged KT keys at a time.  S^T = K Q^T (keys on
+// Forward: online softmax over K / V tiles staged KT keys at a time.  S^T = K Q^T (keys on
 // the rows, the lane's query li on the column), row statistics per query across the four
 // lanes li + 16 lg, O^T += V^T P^T.
 template <int D, int PARTS>
-__global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_fwd_kernel(const AttnTrain a) {
+__global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_fwd_kernel(const AttnTrain a) {
   using S = AttnDims<D, PARTS>;
   __shared__ __align__(16) char lds[S::ROWS + S::COLS];
   char *const kr = lds, *const vc = lds + S::ROWS;
@@ -988,10 +1008,9 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_
   const int64_t start = live ? a.seq_start[a.seq_of[t]] : 0;
   const int64_t w_first = w.active ? a.seq_start[a.seq_of[w.t0]] : 0;  // first key any query of the strip sees
   const int64_t k_lo = a.seq_start[a.seq_of[w.base]];
-  const float scale = a.scale * LOG2E;
   clear_lds(lds, S::ROWS + S::COLS);
   Operand<PARTS> qf[S::DK];  // (scaling bf16 queries would take more than one part)
-  row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg, PARTS == 3 ? scale : 1.0f);
+  row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg, PARTS == 3 ? a.scale : 1.0f);
   f32x4 acc[S::DT];
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1025,7 +1044,7 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_
       f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int dk = 0; dk < S::DK; ++dk) c = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(kr, sub, dk, li, lg), qf[dk], c);
-      s[sub] = PARTS == 3 ? c : c * scale;
+      s[sub] = natural_score<PARTS>(c, a.scale);
       if (!whole) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) s[sub][r] = unsigned(4 * lg - lo + 16 * sub + r) < seen ? s[sub][r] : -INFINITY;
@@ -1034,7 +1053,7 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_
     }
     mt = max_over_rows(mt);
     const float mn = fmaxf(m, mt);
-    const float corr = __builtin_amdgcn_exp2f(m - mn);
+    const float corr = exp_natural(m - mn);
     m = mn;
     l *= corr;
 #pragma unroll
@@ -1046,7 +1065,7 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[2 * u + h][r] = __builtin_amdgcn_exp2f(s[2 * u + h][r] - mn);
+          s[2 * u + h][r] = exp_natural(s[2 * u + h][r] - mn);
           l += s[2 * u + h][r];
         }
       const Operand<3> p = score_operand(s[2 * u], s[2 * u + 1]);
@@ -1060,13 +1079,13 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
     if (dt * 16 + 4 * lg < D) store4(a, orow + dt * 16 + 4 * lg, acc[dt], 1.0f / l);
-  if (lg == 0) a.lse_out[t * a.H + w.h] = m * 0.6931471805599453f + logf(l);
+  if (lg == 0) a.lse_out[t * a.H + w.h] = m + logf(l);
 }
 
 // dQ (and D = rowsum(dO * O)) with the forward's blocks: S^T = K Q^T and dP^T = V dO^T per
 // 16-key tile, P from the saved log-sum-exp, dS = P (dP - D), dQ^T += K^T dS^T.
 template <int D, int PARTS>
-__global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_bwd_dq_kernel(const AttnTrain a) {
+__global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_bwd_dq_kernel(const AttnTrain a) {
   using S = AttnDims<D, PARTS>;
   __shared__ __align__(16) char lds[2 * S::ROWS + S::COLS];
   char *const kr = lds, *const vr = lds + S::ROWS, *const kc = lds + 2 * S::ROWS;
@@ -1078,10 +1097,9 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_
   const int64_t start = live ? a.seq_start[a.seq_of[t]] : 0;
   const int64_t w_first = w.active ? a.seq_start[a.seq_of[w.t0]] : 0;
   const int64_t k_lo = a.seq_start[a.seq_of[w.base]];
-  const float scale = a.scale * LOG2E;
   clear_lds(lds, 2 * S::ROWS + S::COLS);
   Operand<PARTS> qf[S::DK], gf[S::DK];
-  row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg);
+  row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg, PARTS == 3 ? a.scale : 1.0f);
   row_operand<D, PARTS>(gf, a.dout + row * D, live, lg);
   float part = 0.f;
 #pragma unroll
@@ -1095,7 +1113,7 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_
       part = fmaf(g.x, o[0], fmaf(g.y, o[1], fmaf(g.z, o[2], fmaf(g.w, o[3], part))));
     }
   const float dsum = sum_over_rows(part);
-  const float lse = live ? a.lse[row] * LOG2E : 0.f;
+  const float lse = live ? a.lse[row] : 0.f;
   f32x4 acc[S::DT];
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1129,9 +1147,10 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 4 : 3) : 2) void attn_
           st = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(kr, sub, dk, li, lg), qf[dk], st);
           dp = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(vr, sub, dk, li, lg), gf[dk], dp);
         }
+        st = natural_score<PARTS>(st, a.scale);
         f32x4 p;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(st[r], scale, -lse));
+        for (int r = 0; r < 4; ++r) p[r] = exp_natural(st[r] - lse);
         if (!whole) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) p[r] = unsigned(4 * lg - lo + 16 * sub + r) < seen ? p[r] : 0.f;
@@ -1175,7 +1194,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
   const int64_t w_hi = wave_live ? a.seq_start[a.seq_of[min<int64_t>(a.n - 1, jw + 15)] + 1] : 0;
   const int64_t q_hi = a.seq_start[a.seq_of[min<int64_t>(a.n - 1, j0 + 63)] + 1];
   const int units = int((q_hi - j0 + KT - 1) / KT) * G;
-  const float scale = a.scale * LOG2E;
   clear_lds(lds, 2 * S::ROWS + 2 * S::COLS);
   Operand<PARTS> kf[S::DK], vf[S::DK];
   row_operand<D, PARTS>(kf, a.k + j * a.ldk + hk * D, live, lg);
@@ -1195,14 +1213,20 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
     rows_load<D, PARTS>(gp, a.dout + h * D, int64_t(a.H) * D, t0, last);
     const int64_t t = t0 + (threadIdx.x & (KT - 1));
     if (threadIdx.x < 2 * KT)
-      sp = t > last ? 0.f : threadIdx.x < KT ? a.lse[t * a.H + h] * LOG2E : a.dsum[t * a.H + h];
+      sp = t > last ? 0.f : threadIdx.x < KT ? a.lse[t * a.H + h] : a.dsum[t * a.H + h];
   };
   load(0);
   for (int u = 0; u < units; ++u) {
     __syncthreads();
+    if constexpr (PARTS == 3) {
+#pragma unroll
+      for (int e = 0; e < S::PER; ++e)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) qp[e][h] = scaled_query(qp[e][h], a.scale);
+    }
     rows_store<D, PARTS, true, true>(qr, qc, qp);
     rows_store<D, PARTS, true, true>(gr, gc, gp);
-    if (threadIdx.x < 2 * KT) ls[threadIdx.x] = sp;  // [0, KT) lse in base 2, [KT, 2 KT) D
+    if (threadIdx.x < 2 * KT) ls[threadIdx.x] = sp;  // [0, KT) lse, [KT, 2 KT) D
     __syncthreads();
     if (u + 1 < units) load(u + 1);
     const int64_t t0 = j0 + KT * (u / G);
@@ -1222,13 +1246,14 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
         f32x4 sc = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < S::DK; ++k) {
-          sc = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(qr, sub, k, li, lg), kf[k], sc);
+          sc = mma_parts<PARTS, PARTS, true>(row_frag<D, PARTS>(qr, sub, k, li, lg), kf[k], sc);
           dp = mma_parts<PARTS, PARTS>(row_frag<D, PARTS>(gr, sub, k, li, lg), vf[k], dp);
         }
+        sc = natural_score<PARTS>(sc, a.scale);
         const f32x4 lse = *reinterpret_cast<const f32x4 *>(ls + 16 * sub + 4 * lg);
         const f32x4 dsum = *reinterpret_cast<const f32x4 *>(ls + KT + 16 * sub + 4 * lg);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p[x][r] = __builtin_amdgcn_exp2f(fmaf(sc[r], scale, -lse[r]));
+        for (int r = 0; r < 4; ++r) p[x][r] = exp_natural(sc[r] - lse[r]);
         if (!whole) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) p[x][r] = unsigned(4 * lg - lo + 16 * sub + r) < seen ? p[x][r] : 0.f;
@@ -1245,12 +1270,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
     }
   }
   if (!live) return;
+  const float dk_scale = PARTS == 3 ? 1.0f : a.scale;  // (of the staged queries)
   if (a.parts) {
     float *row = a.parts + (int64_t(blockIdx.z) * a.n + j) * 2 * a.KVH * D + hk * D;
 #pragma unroll
     for (int dt = 0; dt < S::DT; ++dt)
       if (dt * 16 + 4 * lg < D) {
-        *reinterpret_cast<f32x4 *>(row + dt * 16 + 4 * lg) = dk[dt] * a.scale;
+        *reinterpret_cast<f32x4 *>(row + dt * 16 + 4 * lg) = dk[dt] * dk_scale;
         *reinterpret_cast<f32x4 *>(row + a.KVH * D + dt * 16 + 4 * lg) = dv[dt];
       }
     return;
@@ -1259,7 +1285,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
     if (dt * 16 + 4 * lg < D) {
-      store4(a, dkrow + dt * 16 + 4 * lg, dk[dt], a.scale);
+      store4(a, dkrow + dt * 16 + 4 * lg, dk[dt], dk_scale);
       store4(a, dvrow + dt * 16 + 4 * lg, dv[dt], 1.0f);
     }
 }

@@ -202,6 +202,27 @@ def test_attention_rows_in_any_order(device, D, H, KVH):
     assert all(torch.equal(a, b) for a, b in zip(*results))
 
 
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("size", [1.0, 37.0, 1e5])
+def test_backward_weights_are_the_forwards(device, precision, size):
+    """Sequences of one token: the softmax weight is 1 whatever the score, in the backward as in the
+    forward, so o = v and dv (the value rows' gradient) are those of scores of 0, bit for bit."""
+
+    results = []
+    for scale in (0.0, size):
+        torch.manual_seed(0)
+        trunk = Trunk(TrunkConfig(d_model=256, n_layers=1, n_heads=8, n_kv_heads=2, d_ff=256)).to(device).train()
+        weight = trunk.blocks[0].qkv_proj.weight
+        with torch.no_grad():
+            weight[: 256 + 64].mul_(scale / 0.02)  # LayerNorm rows times these: scores of up to ~size^2 * 256
+        x = torch.randn(300, 256, generator=torch.Generator().manual_seed(1)).to(device)
+        bounds = torch.stack([torch.arange(300), torch.arange(1, 301)], 1)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=precision == "bf16"):
+            hidden = trunk(x, None, None, bounds)
+        results.append((hidden.detach(), torch.autograd.grad(hidden.square().sum(), weight)[0][256 + 64 :]))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
 CONFIGS = [
     dict(d_model=64, n_layers=2, n_heads=4, n_kv_heads=2, d_ff=128, per_layer_dim=16, value_embeddings="alternating"),
     dict(d_model=96, n_layers=1, n_heads=3, n_kv_heads=1, d_ff=160, per_layer_dim=0, value_embeddings="all"),
