@@ -800,6 +800,32 @@ __device__ __forceinline__ f32x4 mma_parts(const Operand<PA> &a, const Operand<P
   return c;
 }
 
+// A sum over rows: the leading products, and (fp32 operands) the corrections apart from them.  Small
+// terms added to a large sum lose their low bits downwards in the matrix unit, every term the same way:
+// with one sum the gradients' column sums were three times as far off (64 x 256 tokens: dq 9.5e-7
+// relative, 2.7e-7 so; dk and dv themselves 6.1e-7, 3.4e-7).  bf16 results hide it (sum in one).
+template <int PARTS>
+struct RowSum {
+  f32x4 part[PARTS == 3 ? 2 : 1];
+  __device__ __forceinline__ void scale(float x) {
+#pragma unroll
+    for (f32x4 &v : part) v *= x;
+  }
+  __device__ __forceinline__ f32x4 total() const { return PARTS == 3 ? part[0] + part[PARTS == 3] : part[0]; }
+};
+
+template <int PARTS>
+__device__ __forceinline__ void mma_add(const Operand<PARTS> &a, const Operand<3> &b, RowSum<PARTS> &sum) {
+#pragma unroll
+  for (int order = 2; order >= 0; --order)
+#pragma unroll
+    for (int i = 0; i <= order; ++i)
+      if (i < PARTS) {
+        f32x4 &to = sum.part[PARTS == 3 && order != 0];
+        to = split_mma1(a.p[i], b.p[order - i], to);
+      }
+}
+
 // A score tile in natural units: three parts hold scaled queries already; bf16 queries are scaled
 // here, rounded before anything is subtracted.  The backward forms a score with the forward's own
 // operations, so that P = exp(score - lse) carries the rounding of lse alone: a score of any size that
@@ -1011,9 +1037,7 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_
   clear_lds(lds, S::ROWS + S::COLS);
   Operand<PARTS> qf[S::DK];  // (scaling bf16 queries would take more than one part)
   row_operand<D, PARTS>(qf, a.q + t * a.ldq + w.h * D, live, lg, PARTS == 3 ? a.scale : 1.0f);
-  f32x4 acc[S::DT];
-#pragma unroll
-  for (int dt = 0; dt < S::DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  RowSum<PARTS> sum[S::DT] = {};
   float m = -1e30f, l = 0.f;
   float4 kp[S::PER][2], vp[S::PER][2];
   rows_load<D, PARTS>(kp, a.k + hk * D, a.ldk, k_lo, w.b_last);
@@ -1057,7 +1081,7 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_
     m = mn;
     l *= corr;
 #pragma unroll
-    for (int dt = 0; dt < S::DT; ++dt) acc[dt] *= corr;
+    for (int dt = 0; dt < S::DT; ++dt) sum[dt].scale(corr);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       if (!any[2 * u] && !any[2 * u + 1]) continue;
@@ -1070,11 +1094,14 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_
         }
       const Operand<3> p = score_operand(s[2 * u], s[2 * u + 1]);
 #pragma unroll
-      for (int dt = 0; dt < S::DT; ++dt) acc[dt] = mma_parts<PARTS, 3>(col_frag<D, PARTS>(vc, u, dt, li, lg), p, acc[dt]);
+      for (int dt = 0; dt < S::DT; ++dt) mma_add<PARTS>(col_frag<D, PARTS>(vc, u, dt, li, lg), p, sum[dt]);
     }
   }
   l = sum_over_rows(l);
   if (!live) return;
+  f32x4 acc[S::DT];
+#pragma unroll
+  for (int dt = 0; dt < S::DT; ++dt) acc[dt] = sum[dt].total();
   float *orow = a.out + (t * a.H + w.h) * D;
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
@@ -1114,9 +1141,7 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_
     }
   const float dsum = sum_over_rows(part);
   const float lse = live ? a.lse[row] : 0.f;
-  f32x4 acc[S::DT];
-#pragma unroll
-  for (int dt = 0; dt < S::DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  RowSum<PARTS> sum[S::DT] = {};
   float4 kp[S::PER][2], vp[S::PER][2];
   rows_load<D, PARTS>(kp, a.k + hk * D, a.ldk, k_lo, w.b_last);
   rows_load<D, PARTS>(vp, a.v + hk * D, a.ldv, k_lo, w.b_last);
@@ -1160,10 +1185,13 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_
       }
       const Operand<3> dso = score_operand(ds[0], ds[1]);
 #pragma unroll
-      for (int dt = 0; dt < S::DT; ++dt) acc[dt] = mma_parts<PARTS, 3>(col_frag<D, PARTS>(kc, u, dt, li, lg), dso, acc[dt]);
+      for (int dt = 0; dt < S::DT; ++dt) mma_add<PARTS>(col_frag<D, PARTS>(kc, u, dt, li, lg), dso, sum[dt]);
     }
   }
   if (!live) return;
+  f32x4 acc[S::DT];
+#pragma unroll
+  for (int dt = 0; dt < S::DT; ++dt) acc[dt] = sum[dt].total();
   float *dqrow = a.dq + t * a.ldq + w.h * D;
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
@@ -1198,12 +1226,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
   Operand<PARTS> kf[S::DK], vf[S::DK];
   row_operand<D, PARTS>(kf, a.k + j * a.ldk + hk * D, live, lg);
   row_operand<D, PARTS>(vf, a.v + j * a.ldv + hk * D, live, lg);
-  f32x4 dk[S::DT], dv[S::DT];
-#pragma unroll
-  for (int dt = 0; dt < S::DT; ++dt) {
-    dk[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dv[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  RowSum<PARTS> dk_sum[S::DT] = {}, dv_sum[S::DT] = {};
   float4 qp[S::PER][2], gp[S::PER][2];
   float sp = 0.f;
   auto load = [&](int u) {
@@ -1264,12 +1287,18 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
       const Operand<3> po = score_operand(p[0], p[1]), dso = score_operand(ds[0], ds[1]);
 #pragma unroll
       for (int dt = 0; dt < S::DT; ++dt) {
-        dv[dt] = mma_parts<PARTS, 3>(col_frag<D, PARTS>(gc, half, dt, li, lg), po, dv[dt]);
-        dk[dt] = mma_parts<PARTS, 3>(col_frag<D, PARTS>(qc, half, dt, li, lg), dso, dk[dt]);
+        mma_add<PARTS>(col_frag<D, PARTS>(gc, half, dt, li, lg), po, dv_sum[dt]);
+        mma_add<PARTS>(col_frag<D, PARTS>(qc, half, dt, li, lg), dso, dk_sum[dt]);
       }
     }
   }
   if (!live) return;
+  f32x4 dk[S::DT], dv[S::DT];
+#pragma unroll
+  for (int dt = 0; dt < S::DT; ++dt) {
+    dk[dt] = dk_sum[dt].total();
+    dv[dt] = dv_sum[dt].total();
+  }
   const float dk_scale = PARTS == 3 ? 1.0f : a.scale;  // (of the staged queries)
   if (a.parts) {
     float *row = a.parts + (int64_t(blockIdx.z) * a.n + j) * 2 * a.KVH * D + hk * D;
