@@ -1007,8 +1007,8 @@ struct QueryStrip {
   int64_t b_last;  // last token of the block
 };
 
-__device__ __forceinline__ QueryStrip query_strip(const AttnTrain &a) {
-  const int G = a.H / a.KVH, gpb = min(G, 4), tpb = 4 / gpb, wave = threadIdx.x >> 6;
+__device__ __forceinline__ QueryStrip query_strip(const AttnTrain &a, int tid) {
+  const int G = a.H / a.KVH, gpb = min(G, 4), tpb = 4 / gpb, wave = tid >> 6;
   const int strip = wave / gpb, g = blockIdx.z * gpb + wave % gpb;
   QueryStrip q;
   q.base = int64_t(blockIdx.x) * 16 * tpb;
@@ -1019,16 +1019,97 @@ __device__ __forceinline__ QueryStrip query_strip(const AttnTrain &a) {
   return q;
 }
 
+// Plain fp32 forms of the three kernels' results, one lane's query (or key) and d = 16 dt + 4 lg + r at
+// a time, over the rows that it sees alone.  A part of an infinity or of a value past bf16's largest
+// number is not finite, and a hidden row's zero weight times it is NaN, so results that are not finite
+// are formed again here (split.h); finite ones never come here.  The callers find their lane's place
+// again from `fresh_thread`, so that the main loops keep nothing alive for this.
+__device__ __forceinline__ int fresh_thread() {
+  int tid = threadIdx.x;
+  asm("" : "+v"(tid));
+  return tid;
+}
+
+template <int D>
+__device__ __forceinline__ float plain_dot(const float *__restrict__ x, const float *__restrict__ y) {
+  float s = 0.f;
+#pragma unroll 1  // (few registers: the kernels' occupancy is the main loops')
+  for (int d = 0; d < D; d += 4) {
+    const float4 a = *reinterpret_cast<const float4 *>(x + d), b = *reinterpret_cast<const float4 *>(y + d);
+    s = fmaf(a.x, b.x, fmaf(a.y, b.y, fmaf(a.z, b.z, fmaf(a.w, b.w, s))));
+  }
+  return s;
+}
+
+template <int DT>
+__device__ __forceinline__ bool all_finite(const f32x4 (&v)[DT]) {
+  bool ok = true;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ok = ok && split_finite(v[dt][r]);
+  return ok;
+}
+
+// acc += w x[d] over the lane's d.
+template <int D, int DT>
+__device__ __forceinline__ void plain_add(f32x4 (&acc)[DT], float w, const float *__restrict__ x, int lg) {
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    if (dt * 16 + 4 * lg >= D) continue;
+    const float4 v = *reinterpret_cast<const float4 *>(x + dt * 16 + 4 * lg);
+    acc[dt] = f32x4{fmaf(w, v.x, acc[dt][0]), fmaf(w, v.y, acc[dt][1]), fmaf(w, v.z, acc[dt][2]), fmaf(w, v.w, acc[dt][3])};
+  }
+}
+
+template <int DT>
+__device__ __forceinline__ void clear(f32x4 (&v)[DT]) {
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) v[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+template <int D>
+__device__ __forceinline__ float plain_score(const AttnTrain &a, int64_t t, int64_t j, int h, int hk) {
+#pragma clang fp contract(off)
+  return plain_dot<D>(a.q + t * a.ldq + h * D, a.k + j * a.ldk + hk * D) * a.scale;
+}
+
+// Softmax over keys start .. t: the maximum m, the sum l and the sums of V.
+template <int D, int DT>
+__device__ __forceinline__ void plain_forward(const AttnTrain &a, int64_t t, int64_t start, int h, int hk, int lg,
+                                              float &m, float &l, f32x4 (&acc)[DT]) {
+  m = -1e30f;
+#pragma unroll 1
+  for (int64_t j = start; j <= t; ++j) m = fmaxf(m, plain_score<D>(a, t, j, h, hk));
+  l = 0.f;
+  clear(acc);
+#pragma unroll 1
+  for (int64_t j = start; j <= t; ++j) {
+    const float p = exp_natural(plain_score<D>(a, t, j, h, hk) - m);
+    l += p;
+    plain_add<D>(acc, p, a.v + j * a.ldv + hk * D, lg);
+  }
+}
+
+// P and dS of one (query, key) pair.
+template <int D>
+__device__ __forceinline__ void plain_pair(const AttnTrain &a, int64_t t, int64_t j, int h, int hk, float dsum, float &p,
+                                           float &ds) {
+  const int64_t row = t * a.H + h;
+  p = exp_natural(plain_score<D>(a, t, j, h, hk) - a.lse[row]);
+  ds = p * (plain_dot<D>(a.dout + row * D, a.v + j * a.ldv + hk * D) - dsum);
+}
+
 // Forward: online softmax over K / V tiles staged KT keys at a time.  S^T = K Q^T (keys on
 // the rows, the lane's query li on the column), row statistics per query across the four
 // lanes li + 16 lg, O^T += V^T P^T.
 template <int D, int PARTS>
-__global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_fwd_kernel(const AttnTrain a) {
+__global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 3) void attn_fwd_kernel(const AttnTrain a) {
   using S = AttnDims<D, PARTS>;
   __shared__ __align__(16) char lds[S::ROWS + S::COLS];
   char *const kr = lds, *const vc = lds + S::ROWS;
   const int hk = blockIdx.y, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-  const QueryStrip w = query_strip(a);
+  const QueryStrip w = query_strip(a, threadIdx.x);
   const int64_t t = w.t0 + li, w_last = min<int64_t>(a.n - 1, w.t0 + 15);
   const bool live = w.active && t < a.n;
   const int64_t start = live ? a.seq_start[a.seq_of[t]] : 0;
@@ -1102,6 +1183,12 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_
   f32x4 acc[S::DT];
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt) acc[dt] = sum[dt].total();
+  if (!(split_finite(l) && all_finite(acc))) {
+    const int tid = fresh_thread();
+    const QueryStrip z = query_strip(a, tid);
+    const int64_t tz = z.t0 + (tid & 15);
+    plain_forward<D>(a, tz, a.seq_start[a.seq_of[tz]], z.h, blockIdx.y, (tid & 63) >> 4, m, l, acc);
+  }
   float *orow = a.out + (t * a.H + w.h) * D;
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
@@ -1117,7 +1204,7 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_
   __shared__ __align__(16) char lds[2 * S::ROWS + S::COLS];
   char *const kr = lds, *const vr = lds + S::ROWS, *const kc = lds + 2 * S::ROWS;
   const int hk = blockIdx.y, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-  const QueryStrip w = query_strip(a);
+  const QueryStrip w = query_strip(a, threadIdx.x);
   const int64_t t = w.t0 + li, w_last = min<int64_t>(a.n - 1, w.t0 + 15);
   const bool live = w.active && t < a.n;
   const int64_t row = t * a.H + w.h;
@@ -1192,6 +1279,18 @@ __global__ __launch_bounds__(256, D <= 32 ? (PARTS == 1 ? 5 : 4) : 2) void attn_
   f32x4 acc[S::DT];
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt) acc[dt] = sum[dt].total();
+  if (!all_finite(acc)) {
+    const int tid = fresh_thread();
+    const QueryStrip z = query_strip(a, tid);
+    const int64_t tz = z.t0 + (tid & 15);
+    clear(acc);
+#pragma unroll 1
+    for (int64_t j = a.seq_start[a.seq_of[tz]]; j <= tz; ++j) {
+      float p, ds;
+      plain_pair<D>(a, tz, j, z.h, blockIdx.y, dsum, p, ds);
+      plain_add<D>(acc, ds, a.k + j * a.ldk + blockIdx.y * D, (tid & 63) >> 4);
+    }
+  }
   float *dqrow = a.dq + t * a.ldq + w.h * D;
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
@@ -1299,7 +1398,23 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const AttnTrain a) {
     dk[dt] = dk_sum[dt].total();
     dv[dt] = dv_sum[dt].total();
   }
-  const float dk_scale = PARTS == 3 ? 1.0f : a.scale;  // (of the staged queries)
+  float dk_scale = PARTS == 3 ? 1.0f : a.scale;  // (of the staged queries)
+  if (!(all_finite(dk) && all_finite(dv))) {
+    const int tid = fresh_thread(), lz = tid & 63;
+    const int64_t jz = j0 + 16 * (tid >> 6) + (lz & 15), stop = a.seq_start[a.seq_of[jz] + 1];
+    clear(dk);
+    clear(dv);
+    dk_scale = a.scale;
+#pragma unroll 1
+    for (int h = h0; h < h0 + G; ++h)
+#pragma unroll 1
+      for (int64_t t = jz; t < stop; ++t) {
+        float p, ds;
+        plain_pair<D>(a, t, jz, h, hk, a.dsum[t * a.H + h], p, ds);
+        plain_add<D>(dk, ds, a.q + t * a.ldq + h * D, lz >> 4);
+        plain_add<D>(dv, p, a.dout + (t * a.H + h) * D, lz >> 4);
+      }
+  }
   if (a.parts) {
     float *row = a.parts + (int64_t(blockIdx.z) * a.n + j) * 2 * a.KVH * D + hk * D;
 #pragma unroll

@@ -255,6 +255,63 @@ def test_attention_errors_cancel_in_sums(device):
         off = (a.double() - b).mean().abs() / b.abs().mean()
         assert off <= 2.0**-24 / 12, (name, off.item())
 
+def visible_attention(q, k, v, do, lengths, G):
+    """Causal GQA attention and its gradients in float64 with every query on its visible keys alone, so
+    that a row it does not see cannot reach it: (o, dq, dk, dv)."""
+
+    n, H, D = q.shape
+    o, dq, dk, dv = torch.zeros_like(q), torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v)
+    starts = np.repeat(np.concatenate([[0], np.cumsum(lengths)[:-1]]), lengths)
+    for t in range(n):
+        s = int(starts[t])
+        for h in range(H):
+            ks, vs = k[s : t + 1, h // G], v[s : t + 1, h // G]
+            p = ((ks * q[t, h]).sum(-1) / math.sqrt(D)).softmax(0)
+            o[t, h] = (p[:, None] * vs).sum(0)
+            ds = p * ((vs * do[t, h]).sum(-1) - (do[t, h] * o[t, h]).sum()) / math.sqrt(D)
+            dq[t, h] = (ds[:, None] * ks).sum(0)
+            dk[s : t + 1, h // G] += ds[:, None] * q[t, h]
+            dv[s : t + 1, h // G] += p[:, None] * do[t, h]
+    return o, dq, dk, dv
+
+
+@pytest.mark.parametrize("D,H,KVH", [(32, 8, 2), (64, 2, 2), (8, 4, 1)])
+@pytest.mark.parametrize("where, value", [("v", float("inf")), ("v", 3.4e38), ("v", float("nan")),
+                                          ("k", -float("inf")), ("q", 3.4e38), ("do", float("inf"))])
+def test_attention_with_non_finite_rows(device, D, H, KVH, where, value):
+    """An infinity, NaN or a value past bf16's largest number reaches the tokens that see it, as in
+    fp32, and nobody else's: no neighbour in a tile, no other sequence."""
+
+    lengths = [20, 70, 9, 40]
+    n, G, ld = sum(lengths), H // KVH, (H + 2 * KVH) * D
+    g = torch.Generator().manual_seed(D)
+    # (small enough that no product of the one large value overflows)
+    qkv, do = torch.randn(n, ld, generator=g).double() / 4, torch.randn(n, H, D, generator=g).double() * 1e-3
+    q, k, v = (t.reshape(n, -1, D) for t in qkv.split([H * D, KVH * D, KVH * D], 1))
+    {"q": q, "k": k, "v": v, "do": do}[where][60, 0, 2] = value
+    want = visible_attention(*(t.clone() for t in (q, k, v, do)), lengths, G)
+    rows = torch.cat([t.reshape(n, -1) for t in (q, k, v)], 1).float().to(device)
+    seq_start = torch.tensor(np.concatenate([[0], np.cumsum(lengths)]), dtype=torch.int64, device=device)
+    seq_of = torch.arange(len(lengths), device=device, dtype=torch.int32).repeat_interleave(torch.tensor(lengths, device=device))
+    stream = torch.cuda.current_stream().cuda_stream
+    o, lse, dsum = (torch.empty(n, c, device=device) for c in (H * D, H, H))
+    grads = torch.empty_like(rows)
+    at = nat.AttnTrain(n, H, KVH, D, 1.0 / math.sqrt(D), seq_start.data_ptr(), seq_of.data_ptr(),
+                       *(T._ptr(rows, c) for c in (0, H * D, (H + KVH) * D)), ld, ld, ld, o.data_ptr(), lse.data_ptr())
+    dod = do.float().reshape(n, -1).to(device)
+    nat.call("cg_attn_train_fwd", ctypes.byref(at), stream)
+    nat.call("cg_attn_train_bwd", ctypes.byref(at), dod.data_ptr(), dsum.data_ptr(),
+             *(T._ptr(grads, c) for c in (0, H * D, (H + KVH) * D)), stream)
+    got = (o, *grads.split([H * D, KVH * D, KVH * D], 1))
+    for name, x, y in zip(("o", "dq", "dk", "dv"), got, want):
+        x, y = x.double().cpu().reshape(y.shape), y.float().double()  # (past fp32's range: infinite)
+        assert torch.equal(x.isnan(), y.isnan()), name
+        assert torch.equal(x[y.isinf()], y[y.isinf()]), name
+        if where == "q" and name == "dk":
+            continue  # (the rounding of dS times 3.4e38)
+        scale = torch.where(y.isfinite(), y.abs(), 0).amax(-1, keepdim=True).clamp(min=1e-3)  # of the row
+        assert ((x - y).abs() <= 1e-4 * scale)[y.isfinite()].all(), name
+
 
 CONFIGS = [
     dict(d_model=64, n_layers=2, n_heads=4, n_kv_heads=2, d_ff=128, per_layer_dim=16, value_embeddings="alternating"),
