@@ -62,7 +62,8 @@ __device__ __forceinline__ float pairwise_tree(int n, int &index, const float (&
   return __shfl(v, 8 * (index++ & 7), 64);
 }
 
-template <int LEVEL, int ROUNDS>
+// STEPS: the most entries of a leaf that one running sum takes (8 for rows of at most 64 entries).
+template <int LEVEL, int ROUNDS, int STEPS = 16>
 __device__ __forceinline__ float pairwise_sum(const float *w, int n, int lane) {
   int at[ROUNDS], len[ROUNDS], count = 0;
 #pragma unroll
@@ -83,12 +84,12 @@ __device__ __forceinline__ float pairwise_sum(const float *w, int n, int lane) {
     const float *a = w + at[r];
     const int body = len[r] - len[r] % 8, j = lane & 7;
     if (body > 0) {
-      float v[16];
+      float v[STEPS];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = a[min(8 * i, body - 8) + j];
+      for (int i = 0; i < STEPS; ++i) v[i] = a[min(8 * i, body - 8) + j];
       float s = v[0];
 #pragma unroll
-      for (int i = 1; i < 16; ++i) s = 8 * i < body ? s + v[i] : s;
+      for (int i = 1; i < STEPS; ++i) s = 8 * i < body ? s + v[i] : s;
       s += __shfl_xor(s, 1, 64);
       s += __shfl_xor(s, 2, 64);
       s += __shfl_xor(s, 4, 64);
@@ -100,9 +101,9 @@ __device__ __forceinline__ float pairwise_sum(const float *w, int n, int lane) {
   return pairwise_tree<LEVEL>(n, index, leaf);
 }
 
-// NARROW: rows of up to 1024 entries, held in registers from the one pass over them (16 entries
-// per lane; four consecutive ones with VEC: 16-byte aligned rows, 4-byte aligned masks).
-template <bool NARROW, bool VEC>
+// E > 0: rows of up to 64 E entries, held in registers from the one pass over them, E per lane
+// (four consecutive ones with VEC: 16-byte aligned rows, 4-byte aligned masks).  E 0: any width.
+template <int E, bool VEC>
 __global__ __launch_bounds__(64 * ROWS_PER_BLOCK) void masked_probabilities_kernel(
     const float *__restrict__ logits, int64_t ld_logits, const uint8_t *__restrict__ mask, int64_t ld_mask,
     int32_t rows, int32_t width, float *__restrict__ probs, int64_t ld_probs) {
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(64 * ROWS_PER_BLOCK) void masked_probabilities_kern
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  if constexpr (!NARROW) {
+  if constexpr (E == 0) {
     for (int i = lane; i < width; i += 64) see(legal[i] ? x[i] : -INFINITY);
     settle();
     for (int i = lane; i < width; i += 64) w[i] = legal[i] ? expf(x[i] - m) : 0.f;
@@ -138,13 +139,13 @@ __global__ __launch_bounds__(64 * ROWS_PER_BLOCK) void masked_probabilities_kern
     const float total = pairwise_sum<6, 8>(w, width, lane);
     for (int i = lane; i < width; i += 64) p[i] = w[i] / total;
   } else {
-    float v[16];
-    bool on[16];
+    float v[E];
+    bool on[E];
     // Entry of v[e]: with VEC 256 (e / 4) + 4 lane + e % 4, else 64 e + lane.
     auto index = [&](int e) { return VEC ? 256 * (e >> 2) + 4 * lane + (e & 3) : 64 * e + lane; };
     if constexpr (VEC) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < E / 4; ++q) {
         const int i = 256 * q + 4 * lane, at = i < width ? i : 0;
         const float4 f = *reinterpret_cast<const float4 *>(x + at);
         const uchar4 l = *reinterpret_cast<const uchar4 *>(legal + at);
@@ -154,32 +155,36 @@ __global__ __launch_bounds__(64 * ROWS_PER_BLOCK) void masked_probabilities_kern
       }
     } else {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
+      for (int e = 0; e < E; ++e) {
         const int i = index(e), at = i < width ? i : 0;
         v[e] = x[at];
         on[e] = i < width && legal[at];
       }
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e) see(on[e] ? v[e] : -INFINITY);
+    for (int e = 0; e < E; ++e) see(on[e] ? v[e] : -INFINITY);
     settle();
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
+    for (int e = 0; e < E; ++e) {
       v[e] = on[e] ? expf(v[e] - m) : 0.f;
       if (index(e) < width) w[index(e)] = v[e];
     }
     visible();
-    const float total = pairwise_sum<4, 2>(w, width, lane);
+    // Leaves of at most 128: one up to 128 entries, four (two halvings) up to 256.
+    const float total = E == 1   ? pairwise_sum<0, 1, 8>(w, width, lane)
+                        : E == 4 ? pairwise_sum<2, 1>(w, width, lane)
+                       : E == 2 ? pairwise_sum<0, 1>(w, width, lane)
+                                 : pairwise_sum<4, 2>(w, width, lane);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] /= total;
+    for (int e = 0; e < E; ++e) v[e] /= total;
     if constexpr (VEC) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < E / 4; ++q)
         if (256 * q + 4 * lane < width)
           *reinterpret_cast<float4 *>(p + 256 * q + 4 * lane) = float4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
     } else {
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
+      for (int e = 0; e < E; ++e)
         if (index(e) < width) p[index(e)] = v[e];
     }
   }
@@ -200,12 +205,14 @@ __global__ __launch_bounds__(256) void sample_rows_kernel(
   const float *p[PER_WAVE];
   const uint8_t *legal[PER_WAVE];
   int last[PER_WAVE];
+  double u[PER_WAVE];
 #pragma unroll
   for (int r = 0; r < PER_WAVE; ++r) {  // rows past the end are read (not written) as the last one
     const int64_t row = min(mine + r, rows - 1);
     p[r] = probs + row * ld_probs;
     legal[r] = mask + row * ld_mask;
     last[r] = -1;
+    u[r] = uniforms[row];  // (in flight while the running sums form)
   }
 #pragma unroll 4
   for (int i = lane; i < width; i += 64) {
@@ -248,9 +255,8 @@ __global__ __launch_bounds__(256) void sample_rows_kernel(
     const int row = mine + r;
     if (row >= rows) break;  // whole wave
     // float c < double u  <=>  c < t, t the least float >= u (NaN and +-inf included).
-    const double u = uniforms[row];
-    float t = float(u);
-    if (double(t) < u) t = nextafterf(t, INFINITY);
+    float t = float(u[r]);
+    if (double(t) < u[r]) t = nextafterf(t, INFINITY);
     const float *pr = prow + (wave * PER_WAVE + r) * pitch;
     int below = 0, top = last[r];
     for (int i = lane; i < width; i += 64) below += pr[i] < t;
@@ -287,9 +293,13 @@ int cg_masked_probabilities(const float *logits, int64_t ld_logits, const uint8_
     const uintptr_t at = reinterpret_cast<uintptr_t>(logits) | reinterpret_cast<uintptr_t>(probs);
     const bool vec = width % 4 == 0 && (at & 15) == 0 && (reinterpret_cast<uintptr_t>(mask) & 3) == 0 &&
                      ((ld_logits | ld_mask | ld_probs) & 3) == 0;
-    const auto kernel = width > 1024 ? masked_probabilities_kernel<false, false>
-                        : vec        ? masked_probabilities_kernel<true, true>
-                                     : masked_probabilities_kernel<true, false>;
+    // Entries per lane by width: a lane of 16 does the exponentials and divisions of 1024 entries
+    // whatever the width (65536 rows of 8, 64 and 128 entries: 55 us; 16, 17 and 25 so).
+    const auto kernel = width > 1024  ? masked_probabilities_kernel<0, false>
+                        : width > 256 ? (vec ? masked_probabilities_kernel<16, true> : masked_probabilities_kernel<16, false>)
+                        : width > 128 ? (vec ? masked_probabilities_kernel<4, true> : masked_probabilities_kernel<4, false>)
+                        : width > 64  ? masked_probabilities_kernel<2, false>
+                                      : masked_probabilities_kernel<1, false>;
     kernel<<<grid, 64 * ROWS_PER_BLOCK, lds, as_stream(stream)>>>(logits, ld_logits, mask, ld_mask, rows, width, probs,
                                                                   ld_probs);
     CG_LAUNCHED();
@@ -305,9 +315,16 @@ int cg_sample_rows(const float *probs, int64_t ld_probs, const uint8_t *mask, in
     CG_REQUIRE(probs && mask && uniforms && sampled, CG_ERR_INVALID, "probs, mask, uniforms and sampled are required");
     CG_REQUIRE(ld_probs >= width && ld_mask >= width, CG_ERR_INVALID, "row strides must be at least the width");
     CG_REQUIRE(width <= MAX_WIDTH, CG_ERR_UNSUPPORTED, "sample_rows: rows wider than 4096");
-    // As many rows per block as fit in 64 KB of LDS: 16, 8 or 4 (one of 4096 entries takes 16 KB).
+    // Rows per block: 4 while that leaves few wavefronts to a CU or the rows are short (us for 4, 8 and 16
+    // rows: 64 x 8 2.6, 3.1, 4.4; 4096 x 64 3.5, 3.9, 4.9; 8192 x 256 7.7, 6.8, 7.7), 16 for many entries
+    // of rows that leave a CU four blocks of LDS (16384 x 256 14.6, 9.7, 8.9; 65536 x 512 84, 56, 52; but
+    // 65536 x 600 100, 67, 76), 8 between.  A row of 4096 entries takes 16 KB of 64.
     const int pitch = width > 4032 ? (width + 15) / 16 * 16 : (width + 63) / 64 * 64 + 4;
-    const int per_wave = 64 * pitch <= 65536 ? 4 : 32 * pitch <= 65536 ? 2 : 1;
+    const int64_t entries = int64_t(rows) * width;
+    const int per_wave = rows <= 1024 || entries <= (rows <= 4096 ? 1 << 20 : 1 << 19)        ? 1
+                         : rows >= 16384 && entries >= 1 << 21 && 64 * pitch <= 40960 ? 4
+                         : 32 * pitch <= 65536                                        ? 2
+                                                                                      : 1;
     const auto kernel = per_wave == 4 ? sample_rows_kernel<4> : per_wave == 2 ? sample_rows_kernel<2> : sample_rows_kernel<1>;
     kernel<<<unsigned((int64_t(rows) + 4 * per_wave - 1) / (4 * per_wave)), 256, size_t(4 * per_wave) * pitch * 4,
              as_stream(stream)>>>(probs, ld_probs, mask, ld_mask, uniforms, rows, width, pitch, sampled);

@@ -81,8 +81,7 @@ def test_rows_without_a_legal_entry_follow_numpy(device):
                         torch.from_numpy(uniforms).to(device)).cpu().numpy() == ref.sample_rows(want, mask, uniforms)).all()
 
 
-# Register-held rows (vector and scalar loads), wide rows, and 16 / 8 / 4 rows per sampling block,
-# with row counts that leave a block partly empty.
+# Register-held rows (vector and scalar loads) and wide rows, with row counts that leave a block partly empty.
 @pytest.mark.parametrize("rows, width", [(1, 3), (17, 16), (5, 127), (66, 260), (33, 1020), (3, 1023), (9, 1025),
                                          (7, 2047), (5, 4033), (6, 4096)])
 def test_every_row_shape_matches_the_oracle(device, rows, width):
@@ -111,3 +110,23 @@ def test_pairwise_sum_order_is_numpys(device):
         weights = torch.exp(torch.from_numpy(logits - logits.max(1, keepdims=True)).to(device)).cpu().numpy()
         # torch's device exp is the same function, so only the order of the sum could differ
         np.testing.assert_array_equal(got, weights / weights.sum(1, keepdims=True))
+
+
+# 1, 2, 4 and 16 entries per lane, at the edges of each, and 4, 8 and 16 rows per sampling block with a
+# block partly empty: the normaliser in numpy's order (the device's exp divided by its sum, bit for bit)
+# and the picks of the oracle.
+@pytest.mark.parametrize("rows, width", [(5, 1), (5, 7), (6, 63), (7, 64), (5, 65), (6, 127), (7, 128), (5, 129), (6, 132),
+                                         (7, 255), (6, 256), (5, 257), (1025, 8), (4101, 300), (16385, 130),
+                                         (16389, 512), (20001, 64), (2051, 1030)])
+def test_rows_of_each_width(device, rows, width):
+    logits, mask, rng = case(rows, width, rows + 3 * width)
+    x, m = torch.from_numpy(logits).to(device), torch.from_numpy(mask).to(device)
+    top = torch.where(m, x, -torch.inf).amax(1, keepdim=True)
+    weights = torch.where(m, torch.exp(x - top), 0).cpu().numpy()
+    got = masked_probabilities(x, m)
+    np.testing.assert_array_equal(got.cpu().numpy(), weights / weights.sum(1, keepdims=True))
+    probs = got.cpu().numpy()
+    cdf = np.cumsum(probs, axis=1).astype(np.float64)
+    for uniforms in (rng.random(rows), cdf[np.arange(rows), rng.integers(0, width, rows)]):
+        picked = sample_rows(got, m, torch.from_numpy(uniforms).to(device)).cpu().numpy()
+        assert (picked == ref.sample_rows(probs, mask, uniforms)).all()
