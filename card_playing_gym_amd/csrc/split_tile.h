@@ -132,12 +132,25 @@ __device__ __forceinline__ void tile_load_tail(TileRegs<MODE, ROWS, NK> &t, cons
 // The largest row stride (MODE 1) or k stride (MODE 2) whose offsets inside a tile fit 32 bits.
 constexpr int64_t TILE_MAX_STRIDE = int64_t(1) << 22;
 
+// A long sum with the rounding errors of its additions carried beside it (Knuth's two-sum): a bias
+// gradient adds tens of thousands of rows, hundreds of them in one thread.
+struct CarriedSum {
+  float sum = 0.f, lost = 0.f;
+  __device__ __forceinline__ void add(float x) {
+#pragma clang fp contract(off) reassociate(off)
+    const float s = sum + x, b = s - sum;
+    lost += (sum - (s - b)) + (x - b);
+    sum = s;
+  }
+  __device__ __forceinline__ float value() const { return split_finite(lost) ? sum + lost : sum; }  // (infinities)
+};
+
 // Converts the stage's values and writes them to `lds`: part p of k step s at byte
 // (s PLANES + p) plane.  TAIL: k >= k_left is zeroed (the last stage of a ragged k).
 // `sums` (one per row of the thread, or NULL) receives the values as multiplied.
 template <int MODE, int ROWS, int NK, int PLANES, bool TAIL>
 __device__ __forceinline__ void tile_store(char *lds, int plane, const TileRegs<MODE, ROWS, NK> &t, int k_left, int tid,
-                                           float *sums = nullptr) {
+                                           CarriedSum *sums = nullptr) {
 #pragma unroll
   for (int s = 0; s < NK; ++s)
 #pragma unroll
@@ -164,14 +177,14 @@ __device__ __forceinline__ void tile_store(char *lds, int plane, const TileRegs<
         *reinterpret_cast<split_u32x4 *>(o) = p.hi;
         *reinterpret_cast<split_u32x4 *>(o + plane) = p.mid;
         *reinterpret_cast<split_u32x4 *>(o + 2 * plane) = p.lo;
-        if (sums) sums[e] += ((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]));
+        if (sums) sums[e].add(((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3])));
       } else {
         const split_u32x4 p = {split_pack(x[0], x[1]), split_pack(x[2], x[3]), split_pack(y[0], y[1]),
                                split_pack(y[2], y[3])};
         *reinterpret_cast<split_u32x4 *>(o) = p;
         if (sums) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sums[e] += __uint_as_float(p[i] << 16) + __uint_as_float(p[i] & 0xffff0000u);
+          auto two = [&](int i) { return __uint_as_float(p[i] << 16) + __uint_as_float(p[i] & 0xffff0000u); };
+          sums[e].add((two(0) + two(1)) + (two(2) + two(3)));
         }
       }
     }
@@ -209,7 +222,7 @@ __device__ __forceinline__ void tile_product(const float *__restrict__ a, int64_
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = cor[i][j] = split_f32x4{0.f, 0.f, 0.f, 0.f};
   if (kbeg >= kend) return;  // (never with SUMS: slices are not empty)
-  float sums[TM / 64] = {};
+  CarriedSum sums[TM / 64];
   TileRegs<AM, TM, NK> ra;
   TileRegs<BM, ST_N, NK> rb;
   const int last = kbeg + (kend - kbeg - 1) / KS * KS;  // first k of the last stage
@@ -303,13 +316,14 @@ __device__ __forceinline__ void tile_product(const float *__restrict__ a, int64_
         __syncthreads();
         float *meet = reinterpret_cast<float *>(lds);  // [4][TM]
 #pragma unroll
-        for (int e = 0; e < TM / 64; ++e) meet[wave * TM + (TM / 64) * lane + e] = sums[e];
+        for (int e = 0; e < TM / 64; ++e) meet[wave * TM + (TM / 64) * lane + e] = sums[e].value();
         __syncthreads();
         if (tid < TM && tid < ma) row_sums[tid] = (meet[tid] + meet[TM + tid]) + (meet[2 * TM + tid] + meet[3 * TM + tid]);
       } else {
 #pragma unroll
         for (int e = 0; e < TM / 64; ++e) {
-          float v = sums[e] + __shfl_xor(sums[e], 1);
+          float v = sums[e].value();
+          v += __shfl_xor(v, 1);
           v += __shfl_xor(v, 2);
           const int row = (tid + e * 256) >> 2;
           if ((tid & 3) == 0 && row < ma) row_sums[row] = v;

@@ -243,8 +243,16 @@ __device__ __forceinline__ void rows_frag(const float *__restrict__ p, int64_t s
   }
 }
 
-constexpr int ROWS_K = 1024;  // longest reduction and most tiles of the kernel below
-constexpr int64_t ROWS_TILES = 512;
+// Up to 512 tiles (two blocks a CU) and k of 1024: us here and through staged tiles, x w^T fp32 2040 x 256 x
+// 256 6.6, 12.7, at k 1024 19.7, 24.4; 64 x 256 x 1024 10.3, 11.5, bf16 there 9.4, 8.7, all in one launch.
+// Weight gradients in bf16 read both operands a value at a time here (2040 x 256 over 1024 26.0, 22.7; 792 x
+// 512 16.2, 20.4), so the longest of them with the most tiles stay staged.
+constexpr int ROWS_K = 1024;
+constexpr int64_t ROWS_TILES = 512, ROWS_GRAD_WORK = 448 * 1024;
+bool few_rows(int32_t m, int32_t n, int32_t k, bool bf16_gradient) {
+  const int64_t tiles = int64_t((m + 31) / 32) * ((n + 31) / 32);
+  return k > 0 && k <= ROWS_K && tiles <= ROWS_TILES && (!bf16_gradient || tiles * k <= ROWS_GRAD_WORK);
+}
 
 template <int AM, int BM, bool BF, bool SUMS>
 __global__ __launch_bounds__(512) void gemm_rows_kernel(int32_t M, int32_t N, int32_t K, float alpha,
@@ -355,63 +363,81 @@ __global__ __launch_bounds__(512) void gemm_rows_kernel(int32_t M, int32_t N, in
   }
 }
 
-// C[m, n] = epilogue(alpha * sum_z part[z][m, n]).  A thread takes four consecutive entries
-// (float4 loads when N is a multiple of 4) and keeps four slices in flight.
-__global__ void gemm_reduce_kernel(int32_t M, int32_t N, int32_t slices, float alpha, const float *__restrict__ part,
-                                   float beta, float *__restrict__ C, int64_t ldc, const Epi epi) {
-  const int64_t total = int64_t(M) * N, quads = (total + 3) / 4;
-  const bool vec = (N & 3) == 0;
+// C[m, n] = epilogue(alpha * sum_z part[z][m, n]).  A block takes 64 times four consecutive entries
+// (float4 loads when N is a multiple of 4); its wave w sums the slices z = w mod 4, four at a time, and the
+// waves' sums meet in LDS, so that few entries of many slices still fill the chip with loads in flight.
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(int32_t M, int32_t N, int32_t slices, float alpha,
+                                                          const float *__restrict__ part, float beta,
+                                                          float *__restrict__ C, int64_t ldc, const Epi epi) {
+  __shared__ __align__(16) float red[4][256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t total = int64_t(M) * N, first = 256 * int64_t(blockIdx.x), i0 = first + 4 * lane;
+  f32x4 s[4] = {};
+  if ((N & 3) == 0) {
+    if (i0 < total) {
+      int z = wave;
+      for (; z + 12 < slices; z += 16)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s[u] += *reinterpret_cast<const f32x4 *>(part + int64_t(z + 4 * u) * total + i0);
+      for (; z < slices; z += 4) s[0] += *reinterpret_cast<const f32x4 *>(part + int64_t(z) * total + i0);
+    }
+  } else {
+    for (int z = wave; z < slices; z += 4)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i0 + e < total) s[0][e] += part[int64_t(z) * total + i0 + e];
+  }
+  *reinterpret_cast<f32x4 *>(&red[wave][4 * lane]) = (s[0] + s[1]) + (s[2] + s[3]);
+  __syncthreads();
+  const int64_t i = first + tid;
+  if (i < total) {
+    const float v = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
+    epilogue(epi, alpha * v, beta, C, ldc, i / N, i % N);
+  }
   if (epi.row_sum) {
     const float *sums = part + int64_t(slices) * total;
-    for (int m = blockIdx.x * blockDim.x + threadIdx.x; m < M; m += gridDim.x * blockDim.x) {
-      float v = 0.f;
-      for (int z = 0; z < slices; ++z) v += sums[int64_t(z) * M + m];
-      epi.row_sum[m] = epi.round ? round_bf16(v) : v;
+    for (int64_t m0 = 64 * int64_t(blockIdx.x); m0 < M; m0 += 64 * int64_t(gridDim.x)) {
+      float t[4] = {};
+      const int64_t m = min<int64_t>(m0 + lane, M - 1);
+      int z = wave;
+      for (; z + 12 < slices; z += 16)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[u] += sums[int64_t(z + 4 * u) * M + m];
+      for (; z < slices; z += 4) t[0] += sums[int64_t(z) * M + m];
+      __syncthreads();
+      red[wave][lane] = (t[0] + t[1]) + (t[2] + t[3]);
+      __syncthreads();
+      if (wave == 0 && m0 + lane < M) {
+        const float v = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+        epi.row_sum[m0 + lane] = epi.round ? round_bf16(v) : v;
+      }
     }
-  }
-  for (int64_t q = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; q < quads; q += int64_t(gridDim.x) * blockDim.x) {
-    const int64_t i0 = 4 * q;
-    f32x4 s[4] = {};
-    if (vec) {
-      int z = 0;
-      for (; z + 3 < slices; z += 4)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) s[u] += *reinterpret_cast<const f32x4 *>(part + int64_t(z + u) * total + i0);
-      for (; z < slices; ++z) s[0] += *reinterpret_cast<const f32x4 *>(part + int64_t(z) * total + i0);
-    } else {
-      for (int z = 0; z < slices; ++z)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (i0 + e < total) s[0][e] += part[int64_t(z) * total + i0 + e];
-    }
-    const f32x4 t = (s[0] + s[1]) + (s[2] + s[3]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (i0 + e < total) epilogue(epi, alpha * t[e], beta, C, ldc, (i0 + e) / N, (i0 + e) % N);
   }
 }
 
-// Launch plan: row tile TM and split K.  A short reduction over few 128-row tiles takes
-// 64-row tiles (twice the blocks, no second pass); a reduction whose tiles leave most of the chip
-// idle is split over k into enough (tile, slice) blocks to fill it, and a second pass sums the
+// Launch plan: row tile TM and split K.  Products of few 128-row tiles take 64-row tiles (twice the
+// blocks): up to eight of them, or with a short reduction.  A reduction whose tiles leave most of the
+// chip idle is split over k into enough (tile, slice) blocks to fill it, and a second pass sums the
 // slices.
 struct GemmPlan {
   int tm, slices, kc;
 };
-GemmPlan gemm_plan(int32_t m, int32_t n, int32_t k, bool generic) {
+GemmPlan gemm_plan(int32_t m, int32_t n, int32_t k, bool generic, bool bf16) {
   const int64_t nt = (n + GT_N - 1) / GT_N, tiles128 = int64_t((m + GT_M - 1) / GT_M) * nt;
   int tm = GT_M;
-  if (!generic && m > 64 && tiles128 < 512 && !(k >= 1024 && tiles128 < 128)) tm = 64;
+  if (!generic && (m <= 64 || tiles128 <= 8 || (tiles128 < 512 && !(k >= 1024 && tiles128 < 128)))) tm = 64;
   const int64_t tiles = int64_t((m + tm - 1) / tm) * nt;
   // Split K toward the 512 blocks that the chip holds at once (256 CUs x 2), never past them: 408
   // tiles split in two would run as a full wave plus a tail, slower than unsplit (13041-token
   // packed batches hit this).  A slice keeps four 32-k stages, two where the unsplit tiles would
-  // leave three CUs in four idle (256 x 256 over 792 tokens: 37 us unsplit).
+  // leave three CUs in four idle.  At most 64 slices in three parts, 32 in one, whose slices are
+  // shorter against the second pass (dY^T X 256 x 256 over 16384 tokens, us at 32 and 64: fp32 32.0,
+  // 27.2, bf16 23.3, 24.6; 128-row tiles 40.3 and 23.2 at 32).
   const int stages = tiles <= 64 ? 2 : 4;
   int slices = 1;
   if (tiles <= 256 && k >= 2 * stages * GT_K) {
     slices = int(std::min<int64_t>(512 / tiles, k / (stages * GT_K)));
-    slices = std::max(1, std::min(slices, 32));
+    slices = std::max(1, std::min(slices, bf16 ? 32 : 64));
   }
   const int kc = std::max((k + slices - 1) / slices + GT_K - 1, GT_K) / GT_K * GT_K;  // (k 0: one empty slice)
   slices = std::max((k + kc - 1) / kc, 1);
@@ -1546,11 +1572,11 @@ int operand_mode(const float *p, int64_t sr, int64_t sk, int32_t rows, int32_t k
 size_t slice_bytes(const GemmPlan &pl, int32_t m, int32_t n) { return size_t(pl.slices) * size_t(m) * (size_t(n) + 1) * 4; }
 
 GemmPlan plan_of(int32_t m, int32_t n, int32_t k, const float *a, int64_t sam, int64_t sak, const float *b,
-                 int64_t sbk, int64_t sbn, int *am, int *bm) {
+                 int64_t sbk, int64_t sbn, bool bf16, int *am, int *bm) {
   *am = operand_mode(a, sam, sak, m, k);
   *bm = operand_mode(b, sbn, sbk, n, k);
   if (*am == 0 || *bm == 0) *am = *bm = 0;
-  return gemm_plan(m, n, k, *am == 0);
+  return gemm_plan(m, n, k, *am == 0, bf16);
 }
 
 void rows_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, int64_t sam, int64_t sak, const float *b,
@@ -1587,8 +1613,9 @@ void gemm_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, i
   CG_REQUIRE((epi.mode != EPI_GELU || epi.aux_out) && (epi.mode != EPI_GELU_GRAD || epi.aux_in), CG_ERR_INVALID,
              "GEMM epilogue: GELU needs its second output, GELU' its pre-activation");
   int am, bm;
-  const GemmPlan pl = plan_of(m, n, k, a, sam, sak, b, sbk, sbn, &am, &bm);
-  if (k > 0 && k <= ROWS_K && int64_t((m + 31) / 32) * ((n + 31) / 32) <= ROWS_TILES) {
+  const bool bf = epi.round != 0, sums = epi.row_sum != nullptr;
+  const GemmPlan pl = plan_of(m, n, k, a, sam, sak, b, sbk, sbn, bf, &am, &bm);
+  if (few_rows(m, n, k, bf && am == 2 && bm == 2)) {
     rows_launch(m, n, k, alpha, a, sam, sak, b, sbk, sbn, beta, c, ldc, epi, am, bm, as_stream(stream));
     return;
   }
@@ -1601,7 +1628,6 @@ void gemm_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, i
   hipStream_t s = as_stream(stream);
   float *part = pl.slices > 1 ? static_cast<float *>(workspace) : nullptr;
   const int32_t kc = pl.kc;
-  const bool bf = epi.round != 0, sums = epi.row_sum != nullptr;
   CG_REQUIRE(!sums || (am == 2 && bm == 2) || (am == 0 && bm == 0), CG_ERR_UNSUPPORTED, "GEMM: row sums of this layout");
 #define CG_GEMM_RUN(A_, B_, T_, BF_, S_)                                                                        \
   gemm_strided_kernel<A_, B_, T_, BF_, S_><<<grid, 256, 0, s>>>(m, n, k, kc, alpha, a, sam, sak, b, sbk, sbn, beta, c, \
@@ -1633,21 +1659,20 @@ void gemm_launch(int32_t m, int32_t n, int32_t k, float alpha, const float *a, i
 #undef CG_GEMM_CASE
   CG_LAUNCHED();
   if (part) {
-    gemm_reduce_kernel<<<grid_1d((int64_t(m) * n + 3) / 4), 256, 0, s>>>(m, n, pl.slices, alpha, part, beta, c, ldc,
-                                                                        epi);
+    gemm_reduce_kernel<<<blocks_of(int64_t(m) * n, 256), 256, 0, s>>>(m, n, pl.slices, alpha, part, beta, c, ldc, epi);
     CG_LAUNCHED();
   }
 }
 
-// Split-K partials of a GEMM (an upper bound over the operand layouts: the generic layout
-// never splits more than the others).
+// Split-K partials of a GEMM (the most over the operand layouts and precisions).
 size_t gemm_workspace_bytes(int32_t m, int32_t n, int32_t k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
   size_t most = 0;
-  for (bool generic : {false, true}) {
-    const GemmPlan pl = gemm_plan(m, n, k, generic);
-    if (pl.slices > 1) most = std::max(most, slice_bytes(pl, m, n));
-  }
+  for (bool generic : {false, true})
+    for (bool bf16 : {false, true}) {
+      const GemmPlan pl = gemm_plan(m, n, k, generic, bf16);
+      if (pl.slices > 1) most = std::max(most, slice_bytes(pl, m, n));
+    }
   return most;
 }
 
