@@ -452,15 +452,17 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void split_rows_kernel(GemmArgs 
     v[e] = red[0][r * PITCH + c];
 #pragma unroll
     for (int w = 1; w < WK; ++w) v[e] += red[w][r * PITCH + c];
-    if (ok[e] && !split_finite(v[e])) {  // see split.h
+    if (ok[e] && !split_holds(v[e])) {  // see split.h
       const float *ar = static_cast<const float *>(g.A) + int64_t(m) * g.lda;
       const float *wr = static_cast<const float *>(g.W) + int64_t(n) * g.K;
-      v[e] = 0.f;
+      CarriedSum sum;
+#pragma unroll 1
       for (int k = 0; k < g.K; ++k) {
         float x = ar[k];
         if constexpr (LN) x = fmaf((x - norm[0][r]) * norm[1][r], g.a_ln_w[k], g.a_ln_b[k]);
-        v[e] = fmaf(x, wr[k], v[e]);
+        sum.add(x * wr[k]);
       }
+      v[e] = sum.value();
     }
   }
   if (g.bias) {

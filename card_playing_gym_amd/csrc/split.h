@@ -2,7 +2,7 @@
 //
 // Rounding to nearest even leaves |x - hi| <= 2^-9 |x| and |x - hi - mid| <= 2^-17 |x|, both
 // differences exact in fp32 and the last one exact in bf16, so the three parts hold all 24
-// significand bits.  Of the nine products of two such numbers the six of at least 2^-18 are
+// significand bits of a number of at least 2^-110 (bf16 ends at 2^-133).  Of the nine products of two such numbers the six of at least 2^-18 are
 // kept; the dropped ones are below 2^-25 of the product, unsigned bias included, against the
 // 2^-24 of one fp32 rounding.  hi hi goes to one accumulator and the five corrections to
 // another, so the small terms are not rounded away against a large sum.  Six
@@ -11,7 +11,8 @@
 //
 // Infinities, NaN and magnitudes that round past bf16's largest number give a non-finite part
 // and so a non-finite sum, also where the fp32 product is finite (inf * 0 of a zero part).
-// Callers recompute every non-finite result in plain fp32.
+// Callers form every non-finite result again in plain fp32; products also those so small that
+// numbers below 2^-110 may have made them (split_holds).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -75,5 +76,27 @@ __device__ __forceinline__ void split_mma(const Split8 &a, const Split8 &b, spli
 }
 
 __device__ __forceinline__ bool split_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
+
+// Whether a product's result stands: zero, or finite and at least 2^-80 (numbers below 2^-110 take a
+// factor of 2^30 to reach that, and then an error of at most 2^-104).
+constexpr unsigned SPLIT_LEAST = 0x17800000u, SPLIT_INF = 0x7f800000u;  // 2^-80, infinity
+__device__ __forceinline__ bool split_holds(float v) {
+  const unsigned u = __float_as_uint(v) & 0x7fffffffu;
+  return __builtin_expect(u - SPLIT_LEAST < SPLIT_INF - SPLIT_LEAST, 1) || u == 0;
+}
+
+// A long sum with the rounding errors of its additions carried beside it (Knuth's two-sum): a bias
+// gradient adds tens of thousands of rows, hundreds of them in one thread, and a result that is formed
+// again (below) has one thread add all of k.
+struct CarriedSum {
+  float sum = 0.f, lost = 0.f;
+  __device__ __forceinline__ void add(float x) {
+#pragma clang fp contract(off) reassociate(off)
+    const float s = sum + x, b = s - sum;
+    lost += (sum - (s - b)) + (x - b);
+    sum = s;
+  }
+  __device__ __forceinline__ float value() const { return split_finite(lost) ? sum + lost : sum; }  // (infinities)
+};
 
 }  // namespace cg

@@ -132,19 +132,6 @@ __device__ __forceinline__ void tile_load_tail(TileRegs<MODE, ROWS, NK> &t, cons
 // The largest row stride (MODE 1) or k stride (MODE 2) whose offsets inside a tile fit 32 bits.
 constexpr int64_t TILE_MAX_STRIDE = int64_t(1) << 22;
 
-// A long sum with the rounding errors of its additions carried beside it (Knuth's two-sum): a bias
-// gradient adds tens of thousands of rows, hundreds of them in one thread.
-struct CarriedSum {
-  float sum = 0.f, lost = 0.f;
-  __device__ __forceinline__ void add(float x) {
-#pragma clang fp contract(off) reassociate(off)
-    const float s = sum + x, b = s - sum;
-    lost += (sum - (s - b)) + (x - b);
-    sum = s;
-  }
-  __device__ __forceinline__ float value() const { return split_finite(lost) ? sum + lost : sum; }  // (infinities)
-};
-
 // Converts the stage's values and writes them to `lds`: part p of k step s at byte
 // (s PLANES + p) plane.  TAIL: k >= k_left is zeroed (the last stage of a ragged k).
 // `sums` (one per row of the thread, or NULL) receives the values as multiplied.
@@ -339,20 +326,24 @@ __device__ __forceinline__ void tile_product(const float *__restrict__ a, int64_
   }
 }
 
-// Recomputes the tile's results that are not finite as plain fp32 sums (split.h).  m0 / n0: the
+// Recomputes the tile's results that do not hold (split.h) as plain fp32 sums.  m0 / n0: the
 // first row and column of the wave's part; a and b point at element k = 0 of the sum.
 template <int FM>
 __device__ __forceinline__ void tile_repair(split_f32x4 (&acc)[FM][4], const float *__restrict__ a, int64_t sam,
                                             int64_t sak, const float *__restrict__ b, int64_t sbk, int64_t sbn, int m0,
                                             int n0, int M, int N, int k) {
-  bool bad = false;
+  unsigned least = SPLIT_LEAST, most = 0;  // (two instructions a result; zeros take the test below)
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bad = bad || !split_finite(acc[i][j][r]);
-  if (!__any(bad)) return;
+      for (int r = 0; r < 4; ++r) {
+        const unsigned u = __float_as_uint(acc[i][j][r]) & 0x7fffffffu;
+        least = min(least, u);
+        most = max(most, u);
+      }
+  if (!__any(least < SPLIT_LEAST || most >= SPLIT_INF)) return;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -361,12 +352,12 @@ __device__ __forceinline__ void tile_repair(split_f32x4 (&acc)[FM][4], const flo
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + i * 16 + 4 * lg + r, n = n0 + j * 16 + li;
-        if (split_finite(acc[i][j][r]) || m >= M || n >= N) continue;
+        if (split_holds(acc[i][j][r]) || m >= M || n >= N) continue;
         const float *ar = a + int64_t(m) * sam, *bc = b + int64_t(n) * sbn;
-        float v = 0.f;
+        CarriedSum v;
 #pragma unroll 1
-        for (int e = 0; e < k; ++e) v = fmaf(ar[int64_t(e) * sak], bc[int64_t(e) * sbk], v);
-        acc[i][j][r] = v;
+        for (int e = 0; e < k; ++e) v.add(ar[int64_t(e) * sak] * bc[int64_t(e) * sbk]);
+        acc[i][j][r] = v.value();
       }
 }
 

@@ -347,9 +347,11 @@ __global__ __launch_bounds__(512) void gemm_rows_kernel(int32_t M, int32_t N, in
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) v += red[w][r * PITCH + c];
     if (m >= M || n >= N) continue;
-    if (!BF && !split_finite(v)) {  // see split.h
-      v = 0.f;
-      for (int k = 0; k < K; ++k) v = fmaf(A[m * sam + k * sak], B[k * sbk + n * sbn], v);
+    if (!BF && !split_holds(v)) {  // see split.h
+      CarriedSum sum;
+#pragma unroll 1
+      for (int k = 0; k < K; ++k) sum.add(A[m * sam + k * sak] * B[k * sbk + n * sbn]);
+      v = sum.value();
     }
     epilogue(epi, alpha * v, beta, C, ldc, m, n);
   }
