@@ -1371,11 +1371,12 @@ void launch_mfma(const AttnArgs &a, int queries, hipStream_t s) {
   } else {
     const int64_t units = int64_t(a.n_seqs) * a.kv_heads;
     // fp32 pools.  One-token rows of up to four heads per KV head: a block splits each unit's keys
-    // over its waves, four while the chip is not full of units (256 games of up to 256 keys: 9.1 us,
-    // two waves 10.4, the one-wave matrix-core kernel 20.2), two from 1024 units on (1024 games:
-    // 18.0 against 20.5 and 27.3).
-    if (D == 32 && queries <= QB && !a.seq_start) {
-      if (units < 1024) return launch_d<TKV, D, 4>(a, s);
+    // over its waves, four while the chip is not full of units, two beyond.  us with four waves, two, and
+    // the one-wave matrix-core kernel, 8 / 2 heads, up to 256 keys: head_dim 32, 512 units 6.7, 8.0, 17.0,
+    // 1024 11.5, 9.4, 19.5, 8192 64, 48, 71; head_dim 64, 128 units 8.3, 9.6, 26.2, 512 16.5, 12.0, 27.6,
+    // 2048 61, 41, 48, 4096 (4 / 4 heads) 124, 76, 86, 8192 260, 163, 151.
+    if (queries <= QB && !a.seq_start && (D == 32 || units <= 4096)) {
+      if (units < (D == 32 ? 1024 : 512)) return launch_d<TKV, D, 4>(a, s);
       return launch_d<TKV, D, 2>(a, s);
     }
     // More queries: one wave per 16 of a unit while that gives at most four waves per CU (64 rows x

@@ -280,26 +280,25 @@ __device__ __forceinline__ float scale_add(const GemmArgs &g, float c, float add
 // that a LayerNorm in the producer's epilogue needs.
 constexpr int SPLIT_LN_K = 256;  // widest A row that a block normalises by itself
 
-template <int BM, int BN, int WM, int WN, int WK, int EPI, bool LN>
-__global__ __launch_bounds__(64 * WM * WN * WK) void split_rows_kernel(GemmArgs g) {
-  constexpr int THREADS = 64 * WM * WN * WK;
-  constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
+template <int BM, int BN, int WK, int EPI, bool LN>
+__global__ __launch_bounds__(64 * WK) void split_rows_kernel(GemmArgs g) {
+  constexpr int THREADS = 64 * WK;
+  constexpr int FM = BM / 16, FN = BN / 16;
   constexpr int PITCH = BN + 4;  // the four row groups of a wave's stores start 16 banks apart
   constexpr int LN_STEPS = LN ? SPLIT_LN_K / 32 / WK : 1;
   __shared__ float red[WK][BM * PITCH];
   __shared__ float stat[LN ? 2 : 1][LN ? WK : 1][LN ? BM : 1];
   __shared__ float norm[LN ? 2 : 1][LN ? BM : 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
+  const int tid = threadIdx.x, lane = tid & 63, wk = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const float *arow[FM], *wrow[FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
-    arow[i] = static_cast<const float *>(g.A) + int64_t(min(m0 + wm * FM * 16 + i * 16 + li, g.M - 1)) * g.lda + 8 * lg;
+    arow[i] = static_cast<const float *>(g.A) + int64_t(min(m0 + i * 16 + li, g.M - 1)) * g.lda + 8 * lg;
 #pragma unroll
   for (int j = 0; j < FN; ++j)
-    wrow[j] = static_cast<const float *>(g.W) + int64_t(min(n0 + wn * FN * 16 + j * 16 + li, g.N - 1)) * g.K + 8 * lg;
+    wrow[j] = static_cast<const float *>(g.W) + int64_t(min(n0 + j * 16 + li, g.N - 1)) * g.K + 8 * lg;
   const split_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   // One lane's eight values of step s (K is a multiple of 8: all of them or none are inside).
   auto load = [&](const float *row, int s, split_f32x4 (&v)[2]) {
@@ -368,15 +367,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void split_rows_kernel(GemmArgs 
       }
       q += __shfl_xor(q, 16);
       q += __shfl_xor(q, 32);
-      if (wn == 0 && lg == 0) {
-        stat[0][wk][wm * FM * 16 + i * 16 + li] = mean;
-        stat[1][wk][wm * FM * 16 + i * 16 + li] = q;
+      if (lg == 0) {
+        stat[0][wk][i * 16 + li] = mean;
+        stat[1][wk][i * 16 + li] = q;
       }
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int r = wm * FM * 16 + i * 16 + li;
+      const int r = i * 16 + li;
       float mean = 0.f, q = 0.f;
 #pragma unroll
       for (int w = 0; w < WK; ++w) mean += stat[0][w][r] * float(held(w));
@@ -387,7 +386,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void split_rows_kernel(GemmArgs 
         q += stat[1][w][r] + off * off * float(held(w));
       }
       const float rstd = rsqrtf(q / float(g.K) + g.a_eps);
-      if (wk == 0 && wn == 0 && lg == 0) {
+      if (wk == 0 && lg == 0) {
         norm[0][r] = mean;
         norm[1][r] = rstd;
       }
@@ -434,7 +433,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void split_rows_kernel(GemmArgs 
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        red[wk][(wm * FM * 16 + i * 16 + 4 * lg + r) * PITCH + wn * FN * 16 + j * 16 + li] = acc[i][j][r] + cor[i][j][r];
+        red[wk][(i * 16 + 4 * lg + r) * PITCH + j * 16 + li] = acc[i][j][r] + cor[i][j][r];
   __syncthreads();
   // A thread's results, then everything their epilogue reads at once, then the epilogue: read
   // element by element, each load waited for the store before it (a 1024-row fp32 decode step of
@@ -705,11 +704,11 @@ void launch_split_tile(const GemmArgs &g, hipStream_t s) {
   const dim3 grid((g.N + tn - 1) / tn, (g.M + tm - 1) / tm);
   CG_REQUIRE(grid.y <= 65535u, CG_ERR_UNSUPPORTED, "too many rows for one launch");
   if (tile == SPLIT_16) {
-    split_rows_kernel<16, 16, 1, 1, 8, EPI, LN><<<grid, 512, 0, s>>>(g);
+    split_rows_kernel<16, 16, 8, EPI, LN><<<grid, 512, 0, s>>>(g);
   } else if (tile == SPLIT_32) {
-    split_rows_kernel<32, 32, 1, 1, 8, EPI, LN><<<grid, 512, 0, s>>>(g);
+    split_rows_kernel<32, 32, 8, EPI, LN><<<grid, 512, 0, s>>>(g);
   } else if (tile == SPLIT_32x64) {
-    split_rows_kernel<32, 64, 1, 1, 4, EPI, LN><<<grid, 256, 0, s>>>(g);
+    split_rows_kernel<32, 64, 4, EPI, LN><<<grid, 256, 0, s>>>(g);
   } else {
     CG_REQUIRE(!LN, CG_ERR_UNSUPPORTED, "the staged product takes rows that are already normalised");
     if (tile == SPLIT_TILE_64) split_tile_kernel<64, EPI><<<grid, 256, 0, s>>>(g);

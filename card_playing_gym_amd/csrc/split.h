@@ -2,9 +2,9 @@
 //
 // Rounding to nearest even leaves |x - hi| <= 2^-9 |x| and |x - hi - mid| <= 2^-17 |x|, both
 // differences exact in fp32 and the last one exact in bf16, so the three parts hold all 24
-// significand bits of a number of at least 2^-110 (bf16 ends at 2^-133).  Of the nine products of two such numbers the six of at least 2^-18 are
-// kept; the dropped ones are below 2^-25 of the product, unsigned bias included, against the
-// 2^-24 of one fp32 rounding.  hi hi goes to one accumulator and the five corrections to
+// significand bits of a number of at least 2^-110 (bf16 ends at 2^-133).  Of the nine products of
+// two such numbers the six of at least 2^-18 are kept; the dropped ones are below 2^-25 of the
+// product, unsigned bias included, against the 2^-24 of one fp32 rounding.  hi hi goes to one accumulator and the five corrections to
 // another, so the small terms are not rounded away against a large sum.  Six
 // v_mfma_f32_16x16x32_bf16 take 96 cycles where the eight v_mfma_f32_16x16x4_f32 they replace
 // take 256.
@@ -12,7 +12,8 @@
 // Infinities, NaN and magnitudes that round past bf16's largest number give a non-finite part
 // and so a non-finite sum, also where the fp32 product is finite (inf * 0 of a zero part).
 // Callers form every non-finite result again in plain fp32; products also those so small that
-// numbers below 2^-110 may have made them (split_holds).
+// numbers below 2^-110 may have made them (split_holds).  Attention does not: its weights are at
+// most 1, and one below 2^-110 is uncertain by 76 x 2^-24 already through the score in its exponent.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -259,3 +259,19 @@ def test_fp32_pool_launch_rules(device, games, steps, longest):
     hidden = torch.arange(max_len, device=device)[None, None, None] >= seen[:, None, :, None]
     want = torch.matmul(scores.masked_fill(hidden, float("-inf")).softmax(-1), values)
     assert (got.double() - want).abs().max() <= 1e-5  # the fp32-pool bar of this file
+
+
+# Blocks of four and two waves per unit (2 KV heads), and one wave from 4097 units on.
+@pytest.mark.parametrize("games, longest", [(1, 1), (3, 64), (130, 130), (255, 65), (257, 200), (2048, 20), (2049, 20)])
+def test_fp32_pool_of_head_dim_64(device, games, longest):
+    gen = torch.Generator(device=device).manual_seed(games)
+    randn = lambda *s: torch.randn(s, generator=gen, device=device)  # noqa: E731
+    k, v, q = randn(games, 2, longest + 2, 64), randn(games, 2, longest + 2, 64), randn(games, 8, 1, 64)
+    rows = torch.randperm(games, generator=gen, device=device)
+    lengths = torch.randint(0, longest + 1, (games,), generator=gen, device=device) + 1
+    got = decode_attention(q, k, v, rows, lengths, longest + 2, 0.125)
+    keys, values = (t[rows].double().repeat_interleave(4, 1) for t in (k, v))
+    scores = torch.matmul(q.double(), keys.transpose(-1, -2).contiguous()) * 0.125
+    hidden = torch.arange(longest + 2, device=device)[None, None, None] >= lengths[:, None, None, None]
+    want = torch.matmul(scores.masked_fill(hidden, float("-inf")).softmax(-1), values)
+    assert (got.double() - want).abs().max() <= 1e-5  # the fp32-pool bar of this file
