@@ -347,7 +347,7 @@ __global__ __launch_bounds__(512) void gemm_rows_kernel(int32_t M, int32_t N, in
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) v += red[w][r * PITCH + c];
     if (m >= M || n >= N) continue;
-    if (!BF && !split_holds(v)) {  // see split.h
+    if (!BF && __builtin_expect(!split_holds(v), 0)) {  // see split.h
       CarriedSum sum;
 #pragma unroll 1
       for (int k = 0; k < K; ++k) sum.add(A[m * sam + k * sak] * B[k * sbk + n * sbn]);

@@ -317,8 +317,8 @@ CONFIGS = [
     dict(d_model=64, n_layers=2, n_heads=4, n_kv_heads=2, d_ff=128, per_layer_dim=16, value_embeddings="alternating"),
     dict(d_model=96, n_layers=1, n_heads=3, n_kv_heads=1, d_ff=160, per_layer_dim=0, value_embeddings="all"),
     dict(d_model=64, n_layers=2, n_heads=2, n_kv_heads=2, d_ff=64, per_layer_dim=64, value_embeddings="off"),
-    # long reductions (d_model, d_ff >= 1024): split-K GEMMs whose second pass applies the
-    # residual / bias / GELU' epilogues
+    # wide rows (d_model, d_ff 1024): with this few rows every product is one launch of 32 x 32 tiles
+    # (test_gradients_of_large_updates takes the staged and the split ones)
     dict(d_model=1024, n_layers=1, n_heads=16, n_kv_heads=4, d_ff=1024, per_layer_dim=0, value_embeddings="off"),
 ]
 
@@ -565,3 +565,148 @@ def test_attention_at_tile_edges(device, lengths, precision):
         grads.append(torch.autograd.grad(hidden.square().sum(), [x, trunk.blocks[0].qkv_proj.weight]))
     for exact, got in zip(*grads):
         assert (got - exact).norm() <= 2e-2 * exact.norm()
+
+
+# ---- updates past the few-rows products -------------------------------------------------------
+
+
+def ragged_lengths(total: int, longest: int, seed: int) -> list[int]:
+    rng, lengths = np.random.default_rng(seed), []
+    while sum(lengths) < total:
+        lengths.append(int(min(rng.integers(1, longest + 1), total - sum(lengths))))
+    return lengths
+
+
+def packed_bounds(lengths):
+    starts = np.concatenate([[0], np.cumsum(lengths)])
+    return torch.from_numpy(np.repeat(np.stack([starts[:-1], starts[1:]], 1), lengths, axis=0))
+
+
+class RefTrunk64(RefTrunk):
+    """The oracle in float64 throughout (its LayerNorm widens bf16 rows to float32)."""
+
+    def layer_norm(self, x, name):
+        return F.layer_norm(x, (x.shape[-1],), self.s[f"{name}.weight"], self.s[f"{name}.bias"], self.c.eps)
+
+
+def oracle_gradients(state, config, precision, x, weight, lengths, dtype=torch.float32):
+    """The oracle's hidden rows, their gradient to x and to every parameter: sequences padded, packed back."""
+
+    keep = torch.cat([torch.arange(n) + b * max(lengths) for b, n in enumerate(lengths)])
+    ref_state = {k: v.to(dtype, copy=True).requires_grad_() for k, v in state.items()}
+    rows = x.to(dtype, copy=True).requires_grad_()
+    padded = torch.zeros(len(lengths) * max(lengths), x.shape[1], dtype=dtype).index_copy(0, keep, rows)
+    ref = (RefTrunk64 if dtype == torch.float64 else RefTrunk)(ref_state, ref_config_of(config), precision)
+    hidden = ref.forward_full(padded.view(len(lengths), max(lengths), -1)).reshape(padded.shape)[keep]
+    (hidden * weight.to(dtype)).sum().backward()
+    return hidden.detach(), rows.grad, {k: v.grad for k, v in ref_state.items() if v.grad is not None}
+
+
+def trunk_gradients(device, state, config, precision, x, weight, lengths):
+    trunk = Trunk(config)
+    trunk.load_state_dict({k[len("trunk."):]: v for k, v in state.items()})
+    trunk, rows = trunk.to(device).train(), x.to(device, copy=True).requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=precision == "bf16"):
+        hidden = trunk(rows, None, None, packed_bounds(lengths))
+    (hidden * weight.to(device)).sum().backward()
+    return hidden.detach(), rows.grad, {"trunk." + k: p.grad for k, p in trunk.named_parameters() if p.grad is not None}
+
+
+def relative(got, want):
+    got, want = got.double().cpu(), want.double().cpu()
+    return ((got - want).norm() / want.norm()).item()
+
+
+# 1100 and 2100 tokens: staged products with the residual, bias, GELU and GELU' epilogues in whole and
+# overhanging tiles, weight gradients split over k with their row sums beside the slices, dK / dV heads
+# split four ways; 2100: 128-row tiles at k = 1024; 8300: 128-row tiles at k = 256; d_ff 1023: operands of
+# neither contiguous layout.
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("tokens, d_ff", [(1100, 1024), (2100, 1024), (8300, 1024), (1100, 1023)])
+def test_gradients_of_large_updates(device, tokens, d_ff, precision):
+    config = TrunkConfig(d_model=256, n_layers=1, n_heads=8, n_kv_heads=2, d_ff=d_ff)
+    state = random_trunk(config, seed=51)
+    lengths = ragged_lengths(tokens, 96, seed=tokens)
+    g = torch.Generator().manual_seed(tokens)
+    x, weight = (torch.randn(tokens, 256, generator=g) for _ in range(2))
+    weight += 0.5  # bias gradients that do not average out
+    hidden, dx, grads = trunk_gradients(device, state, config, precision, x, weight, lengths)
+    if precision == "fp32":
+        # (measured: 4e-7 at most; the oracle in float64)
+        want, want_dx, want_grads = oracle_gradients(state, config, "fp32", x, weight, lengths, torch.float64)
+        bar, token_bar = 1.5e-6, 5e-6
+    else:
+        # bf16 noise (test_trunk_gradients_bf16_autocast), and no token far beyond it.
+        want, want_dx, want_grads = oracle_gradients(state, config, "bf16", x, weight, lengths)
+        bar, token_bar = 1.5e-2, 5e-2
+    assert grads.keys() == want_grads.keys()
+    for name in grads:
+        assert relative(grads[name], want_grads[name]) <= bar, (name, relative(grads[name], want_grads[name]))
+    for got, ref in ((hidden, want), (dx, want_dx)):
+        off = (got.double().cpu() - ref.double()).norm(dim=1) / ref.double().norm(dim=1)
+        assert off.max() <= token_bar, (off.argmax().item(), off.max().item())
+
+
+@pytest.mark.parametrize("heads, kv_heads", [(8, 2), (4, 2), (4, 4)], ids=["split-4", "split-2", "whole"])
+@pytest.mark.parametrize("lengths", [[16, 17, 31, 32, 33], [63, 64, 65, 1], [127, 2, 129, 200], [15, 1, 1, 1, 48, 96]])
+def test_bf16_attention_token_by_token(device, lengths, heads, kv_heads):
+    """The one-part kernels and the merge of split head groups against the oracle, at sequence ends around
+    the 16-token strips, 32-row contractions and 64-row tiles: a wrong token is off by its whole size."""
+
+    config = TrunkConfig(d_model=32 * heads, n_layers=1, n_heads=heads, n_kv_heads=kv_heads, d_ff=128)
+    state = random_trunk(config, seed=61, scale=0.08)
+    n = sum(lengths)
+    g = torch.Generator().manual_seed(n)
+    x, weight = (torch.randn(n, config.d_model, generator=g) for _ in range(2))
+    hidden, dx, grads = trunk_gradients(device, state, config, "bf16", x, weight, lengths)
+    want, want_dx, want_grads = oracle_gradients(state, config, "bf16", x, weight, lengths)
+    for got, ref in ((hidden, want), (dx, want_dx)):
+        off = (got.double().cpu() - ref.double()).norm(dim=1) / ref.double().norm(dim=1)
+        assert off.max() <= 5e-2, (off.argmax().item(), off.max().item())
+    name = "trunk.blocks.0.qkv_proj.weight"
+    width = 32 * kv_heads
+    for part in (slice(0, 32 * heads), slice(32 * heads, 32 * heads + width), slice(32 * heads + width, None)):
+        assert relative(grads[name][part], want_grads[name][part]) <= 2e-2
+
+
+@pytest.mark.parametrize("n", [1100, 13824, 16384])
+def test_bias_gradients_are_sums_of_their_rows(device, n):
+    """Blocks that add nothing to the residual stream: the down projection's bias gradient is the column
+    sum of the final norm's input gradient, for columns of any mean, within one rounding of a float32
+    (root mean square over the columns)."""
+
+    torch.manual_seed(n)
+    trunk = Trunk(TrunkConfig(d_model=256, n_layers=1, n_heads=8, n_kv_heads=2, d_ff=256)).to(device).train()
+    block = trunk.blocks[0]
+    with torch.no_grad():
+        for p in (block.out_proj.weight, *block.mlp[2].parameters(), *block.mlp[0].parameters()):
+            p.zero_()
+    x = torch.randn(n, 256, device=device)
+    dy = torch.randn(n, 256, device=device) + torch.linspace(-1, 1, 256, device=device)
+    hidden = trunk(x, None, None, packed_bounds(ragged_lengths(n, 64, seed=n)))
+    got = torch.autograd.grad(hidden, block.mlp[2].bias, dy)[0].double()
+    norm = trunk.final_norm
+    _, mean, rstd = T.layernorm_fwd(x, norm.weight, norm.bias, norm.eps)
+    rows = T.norm_bwd(x, dy, norm.weight, mean, rstd, torch.empty_like(norm.weight), torch.empty_like(norm.bias))
+    want = rows.double().sum(0)
+    assert ((got - want) / want).square().mean().sqrt() <= 2.0**-24
+
+
+def test_layers_that_share_a_value_slot(device):
+    """Two layers reading one slot: its gradient is the sum of both, and a slot nobody reads has none."""
+
+    config = TrunkConfig(d_model=64, n_layers=2, n_heads=4, n_kv_heads=2, d_ff=64, value_embeddings="all")
+    trunk = Trunk(config).to(device).train()
+    g = torch.Generator().manual_seed(5)
+    x, weight = (torch.randn(2, 9, 64, generator=g).to(device) for _ in range(2))
+    slots = torch.randn(2, 9, 2, config.kv_width, generator=g).to(device)
+
+    def grad(index, values):
+        trunk._value_index = index
+        values = values.clone().requires_grad_()
+        return torch.autograd.grad((trunk(x, None, values) * weight).sum(), values)[0]
+
+    shared = grad({0: 1, 1: 1}, slots)
+    apart = grad({0: 0, 1: 1}, slots[:, :, 1:].expand(-1, -1, 2, -1))
+    assert torch.equal(shared[:, :, 0], torch.zeros_like(shared[:, :, 0]))
+    close(shared[:, :, 1], apart.sum(2), tol=1e-6)
