@@ -399,18 +399,18 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(int32_t M, int32_t N, 
   if (epi.row_sum) {
     const float *sums = part + int64_t(slices) * total;
     for (int64_t m0 = 64 * int64_t(blockIdx.x); m0 < M; m0 += 64 * int64_t(gridDim.x)) {
-      float t[4] = {};
+      CarriedSum t;
       const int64_t m = min<int64_t>(m0 + lane, M - 1);
-      int z = wave;
-      for (; z + 12 < slices; z += 16)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) t[u] += sums[int64_t(z + 4 * u) * M + m];
-      for (; z < slices; z += 4) t[0] += sums[int64_t(z) * M + m];
+#pragma unroll 4
+      for (int z = wave; z < slices; z += 4) t.add(sums[int64_t(z) * M + m]);
       __syncthreads();
-      red[wave][lane] = (t[0] + t[1]) + (t[2] + t[3]);
+      red[wave][lane] = t.sum;
+      red[wave][64 + lane] = t.lost;
       __syncthreads();
       if (wave == 0 && m0 + lane < M) {
-        const float v = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+        for (int w = 1; w < 4; ++w) t.add(red[w][lane]);
+        t.lost += (red[1][64 + lane] + red[2][64 + lane]) + red[3][64 + lane];
+        const float v = t.value();
         epi.row_sum[m0 + lane] = epi.round ? round_bf16(v) : v;
       }
     }
