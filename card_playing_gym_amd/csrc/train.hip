@@ -418,24 +418,27 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(int32_t M, int32_t N, 
 }
 
 // Launch plan: row tile TM and split K.  Products of few 128-row tiles take 64-row tiles (twice the
-// blocks): up to eight of them, or with a short reduction.  A reduction whose tiles leave most of the
-// chip idle is split over k into enough (tile, slice) blocks to fill it, and a second pass sums the
-// slices.
+// blocks): with a short reduction, or up to sixteen of them, three parts over 8192 and more up to eight
+// (dY^T X 1024 x 256, us in 64-row and 128-row tiles: bf16 over 16384 tokens 39.8, 45.4, fp32 over 4096
+// 25.6, 28.6, over 8192 40.4, 39.8, over 16384 66.8, 62.4; 256 x 256 over 16384 fp32 27.4, 28.2).  A
+// reduction whose tiles leave most of the chip idle is split over k into enough (tile, slice) blocks to
+// fill it, and a second pass sums the slices.
 struct GemmPlan {
   int tm, slices, kc;
 };
 GemmPlan gemm_plan(int32_t m, int32_t n, int32_t k, bool generic, bool bf16) {
   const int64_t nt = (n + GT_N - 1) / GT_N, tiles128 = int64_t((m + GT_M - 1) / GT_M) * nt;
   int tm = GT_M;
-  if (!generic && (m <= 64 || tiles128 <= 8 || (tiles128 < 512 && !(k >= 1024 && tiles128 < 128)))) tm = 64;
+  if (!generic && (m <= 64 || tiles128 <= (bf16 || k < 8192 ? 16 : 8) || (tiles128 < 512 && !(k >= 1024 && tiles128 < 128)))) tm = 64;
   const int64_t tiles = int64_t((m + tm - 1) / tm) * nt;
   // Split K toward the 512 blocks that the chip holds at once (256 CUs x 2), never past them: 408
   // tiles split in two would run as a full wave plus a tail, slower than unsplit (13041-token
-  // packed batches hit this).  A slice keeps four 32-k stages, two where the unsplit tiles would
-  // leave three CUs in four idle.  At most 64 slices in three parts, 32 in one, whose slices are
-  // shorter against the second pass (dY^T X 256 x 256 over 16384 tokens, us at 32 and 64: fp32 32.0,
-  // 27.2, bf16 23.3, 24.6; 128-row tiles 40.3 and 23.2 at 32).
-  const int stages = tiles <= 64 ? 2 : 4;
+  // packed batches hit this).  A slice keeps four 32-k stages, two where four would leave most of the
+  // chip idle (us at two and four, fp32: 256 x 256 over 1100 11.4, 13.4, 512 x 256 12.6, 13.9, 64 x 64
+  // over 2048 8.8, 10.8, but 384 x 256 16.9, 14.1).  At most 64 slices in three parts, 32 in one, whose
+  // slices are shorter against the second pass (256 x 256 over 16384, at 32 and 64: fp32 32.0, 27.4,
+  // bf16 23.4, 24.6).
+  const int stages = tiles <= 8 || k < 2048 ? 2 : 4;
   int slices = 1;
   if (tiles <= 256 && k >= 2 * stages * GT_K) {
     slices = int(std::min<int64_t>(512 / tiles, k / (stages * GT_K)));

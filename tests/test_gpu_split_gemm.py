@@ -82,7 +82,7 @@ def test_non_finite_operands_behave_as_in_fp32(device, m, n, k):
 
 # Operand layouts of the training products: k contiguous, rows contiguous, and neither (odd sizes).
 @pytest.mark.parametrize("m, n, k", [(4, 4, 4), (128, 64, 32), (132, 260, 36), (129, 67, 33), (1000, 256, 1028),
-                                     (13041, 256, 64), (40000, 256, 32)])
+                                     (13041, 256, 64), (40000, 256, 32), (2048, 40, 256), (9000, 384, 520)])
 def test_training_products_are_fp32_in_every_layout(device, m, n, k):
     gen = torch.Generator(device=device).manual_seed(m * n + k)
     randn = lambda *s: torch.randn(s, generator=gen, device=device)  # noqa: E731

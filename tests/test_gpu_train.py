@@ -384,7 +384,8 @@ def _bf(t):
     return t.bfloat16().double()
 
 
-@pytest.mark.parametrize("size", [(200, 136, 1040), (70, 45, 133)], ids=["split-k", "generic"])
+@pytest.mark.parametrize("size", [(200, 136, 1040), (70, 45, 133), (2048, 40, 256), (2100, 1024, 256)],
+                         ids=["split-k", "generic", "under-64-rows", "64-row-split"])
 def test_gemm_bf16(device, size):
     """CG_BF16: products of bf16-rounded operands with fp32 accumulation, returned rounded to
     bf16 (what F.linear / @ give under autocast): within half a bf16 ulp of the exact product
