@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256, 2) void gemm_strided_kernel(int32_t M, int32_t
 
 // ---- products of few rows --------------------------------------------------------------
 // A microbatch of hundreds of rows is bound by launches and by the latency of each: a staged product
-// split over k takes a second launch for its slices (792 x 256 x 512: 9.6 + 4 us).  Here one launch
+// split over k takes a second launch for its slices (792 x 256 x 512: 11.4 us, 7.1 here).  Here one launch
 // spreads k over the eight waves of a 32 x 32 tile's block, each reading its operand fragments straight
 // from global memory (lane (li, lg): row li, k 8 lg .. 8 lg + 7 of a 32-k step) and the partial tiles
 // meeting in LDS.
@@ -1767,7 +1767,7 @@ void attn_bwd_launch(const cg_attn_train *p, const float *dout, float *dsum, flo
   CG_REQUIRE(aligned16(dout), CG_ERR_INVALID, "attention dO: 16-byte aligned");
   // Heads split while the blocks stay within eight per CU (13.8 k ragged tokens fp32: 432 blocks 77 us,
   // 1728 blocks 52 and the merge 9), with one-part operands, whose walk is shorter, within two (64 x 256
-  // tokens: 512 blocks 45 us, 2048 blocks 37 and the merge 10).
+  // tokens: 512 blocks 39.5 us, 2048 blocks 32.9 and the merge 9.7).
   const int64_t blocks = int64_t(blocks_of(p->n, 64)) * p->KVH, width = int64_t(p->KVH) * p->head_dim;
   for (int z = 4; z > 1 && parts; z /= 2)
     if (p->H / p->KVH % z == 0 && blocks * z <= (bf16_operands ? 512 : 2048) && z * 2 * width * p->n <= part_floats) {

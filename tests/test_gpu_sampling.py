@@ -125,8 +125,15 @@ def test_rows_of_each_width(device, rows, width):
     weights = torch.where(m, torch.exp(x - top), 0).cpu().numpy()
     got = masked_probabilities(x, m)
     np.testing.assert_array_equal(got.cpu().numpy(), weights / weights.sum(1, keepdims=True))
+    # Rows of a wider matrix, starting off a 16-byte boundary: the same numbers.
+    wide, marks = torch.zeros(rows, width + 6, device=device), torch.zeros(rows, width + 6, dtype=torch.bool, device=device)
+    wide[:, 1 : 1 + width], marks[:, 3 : 3 + width] = x, m
+    assert torch.equal(masked_probabilities(wide[:, 1 : 1 + width], marks[:, 3 : 3 + width]).nan_to_num(2), got.nan_to_num(2))
     probs = got.cpu().numpy()
     cdf = np.cumsum(probs, axis=1).astype(np.float64)
     for uniforms in (rng.random(rows), cdf[np.arange(rows), rng.integers(0, width, rows)]):
         picked = sample_rows(got, m, torch.from_numpy(uniforms).to(device)).cpu().numpy()
         assert (picked == ref.sample_rows(probs, mask, uniforms)).all()
+    wide[:, 1 : 1 + width] = got
+    again = sample_rows(wide[:, 1 : 1 + width], marks[:, 3 : 3 + width], torch.from_numpy(uniforms).to(device))
+    assert (again.cpu().numpy() == picked).all()
