@@ -451,7 +451,7 @@ __global__ __launch_bounds__(64 * WK) void split_rows_kernel(GemmArgs g) {
     v[e] = red[0][r * PITCH + c];
 #pragma unroll
     for (int w = 1; w < WK; ++w) v[e] += red[w][r * PITCH + c];
-    if (__builtin_expect(ok[e] && !split_holds(v[e]), 0)) {  // see split.h
+    if (__builtin_expect(ok[e] & !split_holds(v[e]), 0)) {  // see split.h
       const float *ar = static_cast<const float *>(g.A) + int64_t(m) * g.lda;
       const float *wr = static_cast<const float *>(g.W) + int64_t(n) * g.K;
       CarriedSum sum;

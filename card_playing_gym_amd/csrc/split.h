@@ -83,7 +83,7 @@ __device__ __forceinline__ bool split_finite(float v) { return fabsf(v) <= 3.402
 constexpr unsigned SPLIT_LEAST = 0x17800000u, SPLIT_INF = 0x7f800000u;  // 2^-80, infinity
 __device__ __forceinline__ bool split_holds(float v) {
   const unsigned u = __float_as_uint(v) & 0x7fffffffu;
-  return __builtin_expect(u - SPLIT_LEAST < SPLIT_INF - SPLIT_LEAST, 1) || u == 0;
+  return (u - SPLIT_LEAST < SPLIT_INF - SPLIT_LEAST) | (u == 0);  // (no branch)
 }
 
 // A long sum with the rounding errors of its additions carried beside it (Knuth's two-sum): a bias
